@@ -73,8 +73,8 @@ struct fdtd_batch {
     std::vector<fdtd::StripGeom> sgeom;
     int2* d_swork = nullptr;
     int snwork = 0;
-    int snblocks = 0;
     size_t slds = 0;
+    int sdepth = 0;  // input planes the strip tiles stage in LDS (0: direct)
     void* d_sgrids = nullptr;
     size_t sgrid_desc_bytes = 0;
     std::vector<unsigned char> h_sgrids;
@@ -94,7 +94,7 @@ void drop_graph(fdtd_batch* b) {
 // The values a graph captured for nsteps steps depends on (see graph_key).
 std::vector<long long> graph_key_of(const fdtd_batch* b, int nsteps) {
     auto addr = [](const void* p) { return static_cast<long long>(reinterpret_cast<uintptr_t>(p)); };
-    return {nsteps, b->total_src, b->sL, b->sV, b->sR, b->sW, b->snwork, b->snblocks,
+    return {nsteps, b->total_src, b->sL, b->sV, b->sR, b->sW, b->sdepth, b->snwork,
             b->nwork, b->nblocks, b->shape.V, b->shape.NT,
             addr(b->d_src), addr(b->d_vals), addr(b->d_kstart), addr(b->d_grids),
             addr(b->d_sgrids), addr(b->d_work), addr(b->d_swork), addr(b->d_counters),
@@ -262,12 +262,14 @@ constexpr bool batch_strip_built(int csize, int V, int R) {
 }
 
 template <typename S, int V, int R, int L, bool FINAL>
-const void* batch_strip_kernel() {
+const void* batch_strip_kernel(bool stage) {
     using C = typename fdtd::ComputeOf<S>::type;
     if constexpr (!batch_strip_built(sizeof(C), V, R)) {
         return nullptr;
     } else {
-        return reinterpret_cast<const void*>(fdtd::batch_strip_sweep<S, C, V, R, L, FINAL>);
+        if constexpr (fdtd::strip_stage_built(V, R, L))
+            if (stage) return reinterpret_cast<const void*>(fdtd::batch_strip_sweep<S, C, V, R, L, FINAL, true>);
+        return reinterpret_cast<const void*>(fdtd::batch_strip_sweep<S, C, V, R, L, FINAL, false>);
     }
 }
 
@@ -285,9 +287,10 @@ int launch_batch_strip_v(fdtd_batch* b, int parity, const double* vals) {
         a.vals = vals;
         a.vstride = b->total_src;
         a.pad = 0;
-        a.counters = b->d_counters;
-        hipLaunchKernelGGL((fdtd::batch_strip_sweep<S, C, V, R, L, FINAL>), dim3(b->snblocks),
-                           dim3(64 * b->sW), b->slds, b->stream, a);
+        auto kern = fdtd::batch_strip_sweep<S, C, V, R, L, FINAL, false>;
+        if constexpr (fdtd::strip_stage_built(V, R, L))
+            if (b->sdepth > 0) kern = fdtd::batch_strip_sweep<S, C, V, R, L, FINAL, true>;
+        hipLaunchKernelGGL(kern, dim3(b->snwork), dim3(64 * b->sW), b->slds, b->stream, a);
         HIP_TRY(hipGetLastError());
         return FDTD_OK;
     }
@@ -327,28 +330,28 @@ int launch_batch_strip(fdtd_batch* b, bool final, int parity, const double* vals
 }
 
 template <typename S, int V, int R>
-const void* strip_kernel_l(int L, bool final) {
+const void* strip_kernel_l(int L, bool final, bool stage) {
     switch (L) {
-        case 1: return final ? batch_strip_kernel<S, V, R, 1, true>() : batch_strip_kernel<S, V, R, 1, false>();
-        case 2: return final ? batch_strip_kernel<S, V, R, 2, true>() : batch_strip_kernel<S, V, R, 2, false>();
-        case 3: return final ? batch_strip_kernel<S, V, R, 3, true>() : batch_strip_kernel<S, V, R, 3, false>();
-        default: return final ? batch_strip_kernel<S, V, R, 4, true>() : batch_strip_kernel<S, V, R, 4, false>();
+        case 1: return final ? batch_strip_kernel<S, V, R, 1, true>(stage) : batch_strip_kernel<S, V, R, 1, false>(stage);
+        case 2: return final ? batch_strip_kernel<S, V, R, 2, true>(stage) : batch_strip_kernel<S, V, R, 2, false>(stage);
+        case 3: return final ? batch_strip_kernel<S, V, R, 3, true>(stage) : batch_strip_kernel<S, V, R, 3, false>(stage);
+        default: return final ? batch_strip_kernel<S, V, R, 4, true>(stage) : batch_strip_kernel<S, V, R, 4, false>(stage);
     }
 }
 
 template <typename S>
-const void* strip_kernel_s(int V, int R, int L, bool final) {
-    if (V == 1 && R == 2) return strip_kernel_l<S, 1, 2>(L, final);
-    if (V == 1 && R == 4) return strip_kernel_l<S, 1, 4>(L, final);
-    if (V == 2 && R == 2) return strip_kernel_l<S, 2, 2>(L, final);
+const void* strip_kernel_s(int V, int R, int L, bool final, bool stage) {
+    if (V == 1 && R == 2) return strip_kernel_l<S, 1, 2>(L, final, stage);
+    if (V == 1 && R == 4) return strip_kernel_l<S, 1, 4>(L, final, stage);
+    if (V == 2 && R == 2) return strip_kernel_l<S, 2, 2>(L, final, stage);
     return nullptr;
 }
 
-const void* strip_kernel(int precision, int V, int R, int L, bool final) {
+const void* strip_kernel(int precision, int V, int R, int L, bool final, bool stage) {
     switch (precision) {
-        case FDTD_FP64: return strip_kernel_s<double>(V, R, L, final);
-        case FDTD_FP32: return strip_kernel_s<float>(V, R, L, final);
-        default: return strip_kernel_s<_Float16>(V, R, L, final);
+        case FDTD_FP64: return strip_kernel_s<double>(V, R, L, final, stage);
+        case FDTD_FP32: return strip_kernel_s<float>(V, R, L, final, stage);
+        default: return strip_kernel_s<_Float16>(V, R, L, final, stage);
     }
 }
 
@@ -367,21 +370,23 @@ int apply_strips(fdtd_batch* b, int L, int V, int R, int W) {
         64 * W > fdtd::strip_max_threads(V, R, L, cs))
         return fail(FDTD_ERR_INVALID_ARGUMENT, "strip blocking L=%d V=%d R=%d W=%d not available",
                     L, V, R, W);
-    int Gx = 0, TX = 0;
-    strip_x_geometry(L, V, storage_size(b->precision), &Gx, &TX, false);
-    const int TY = W * R - 2 * L;
-    if (TX < 1 || TY < 1)
+    if (W * R - 2 * L < 1)
         return fail(FDTD_ERR_INVALID_ARGUMENT, "strip tiles of W=%d R=%d leave no stored rows", W, R);
     for (size_t q = 0; q < b->grids.size(); ++q) {
         const fdtd_grid* g = b->grids[q];
         if (g->Ni % V || (unsigned long long)g->Ni * g->Nj * g->esize >= (1ull << 31))
             return fail(FDTD_ERR_INVALID_ARGUMENT, "grid %zu cannot take strips with V=%d", q, V);
     }
-    const size_t lds = fdtd::strip_lds_bytes(L, W, V, cs);
+    // planes staged in LDS when every grid's rows allow it
+    int depth = 2;
+    for (const fdtd_grid* g : b->grids)
+        depth = std::min(depth, strip_stage_depth(L, V, R, W, g->Ni, b->precision));
+    const int TY = fdtd::strip_tile_rows(W, R, cs) - 2 * L;
+    const size_t lds = fdtd::strip_lds_bytes(L, W, V, R, cs, (int)storage_size(b->precision), depth);
     if (lds > kLdsLimit) return fail(FDTD_ERR_INVALID_ARGUMENT, "strip tiles need too much LDS");
     int per_cu = 0;
     for (bool final : {false, true}) {
-        const void* kern = strip_kernel(b->precision, V, R, L, final);
+        const void* kern = strip_kernel(b->precision, V, R, L, final, depth > 0);
         if (!kern) return fail(FDTD_ERR_UNSUPPORTED, "strip variant not built");
         if (int rc = allow_dynamic_lds(kern, lds)) return rc;
         if (!final) HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 64 * W, lds));
@@ -408,16 +413,23 @@ int apply_strips(fdtd_batch* b, int L, int V, int R, int W) {
             G.Nj = g->Nj;
             G.Nk = g->Nk;
             G.W = W;
-            G.Gx = Gx;
-            G.TX = TX;
+            // the granule-aligned width where it needs no more tiles
+            int Gx = 0, TX = 0;
+            strip_x_geometry(L, V, b->precision, depth > 0, &Gx, &TX, false);
+            strip_x_geometry(L, V, b->precision, depth > 0, &G.Gx, &G.TX, true);
+            if ((g->Ni + TX - 1) / TX < (g->Ni + G.TX - 1) / G.TX) {
+                G.Gx = Gx;
+                G.TX = TX;
+            }
             G.TY = TY;
             const int kc = std::min(kmax, g->Nk);
             const int nchunk = (g->Nk + kc - 1) / kc;
             G.kchunk = (g->Nk + nchunk - 1) / nchunk;
-            G.ntx = (g->Ni + TX - 1) / TX;
+            G.ntx = (g->Ni + G.TX - 1) / G.TX;
             G.nty = (g->Nj + TY - 1) / TY;
             G.ntiles = G.ntx * G.nty * nchunk;
             G.per_xcd = (G.ntiles + 7) / 8;
+            G.depth = depth;
             for (int t = 0; t < G.ntiles; ++t) {
                 const int chunk = t / (G.ntx * G.nty);
                 const int kcount = std::min(G.kchunk, g->Nk - chunk * G.kchunk) + 2 * (L - 1);
@@ -459,8 +471,8 @@ int apply_strips(fdtd_batch* b, int L, int V, int R, int W) {
                       hipMemcpyHostToDevice));
     b->sgeom = geom;
     b->snwork = (int)sorted.size();
-    b->snblocks = std::max(1, std::min(b->snwork, per_cu * cus));
     b->slds = lds;
+    b->sdepth = depth;
     b->sL = L;
     b->sV = V;
     b->sR = R;

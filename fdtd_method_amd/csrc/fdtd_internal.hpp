@@ -61,32 +61,48 @@ inline size_t storage_size(int precision) {
     return precision == FDTD_FP64 ? 8 : (precision == FDTD_FP32 ? 4 : 2);
 }
 
-// x geometry of a strip tile: a window of 64*V columns with Gx ghost columns
-// on each side (at least L, a multiple of V) and TX stored columns; tiles
-// start at multiples of TX.  With 4-byte storage, TX is a multiple of 16
-// columns, so every stored row is whole, aligned 64-byte granules: stores of
-// 56-column (224-byte) rows that begin mid-granule ran at about half the
-// bandwidth (measured at 512^3: the pass took 2.16 ms with 56 stored columns
-// and 1.90 ms with 48, bit-identical, although the narrower tiles compute
-// 10% more cells).  FP64 rows of 56 doubles are whole granules already; FP16
-// keeps 56 columns (a granule-aligned FP16 tile would store 32).  Batches of
-// small grids take the unaligned width (align false): most of their rows
-// hold one to three tiles, whose first tile is aligned anyway, and the 11%
-// more tiles of the aligned width cost more than the aligned stores save
-// (256-grid batch, same box: 236.0 Gcell/s with 56 stored columns, 221.5
-// with 48).
-inline void strip_x_geometry(int L, int V, size_t esize, int* Gx, int* TX, bool align = true) {
-    *Gx = (L + V - 1) / V * V;
-    *TX = 64 * V - 2 * *Gx;
-    if (align && esize == 4) {
+inline size_t compute_size(int precision) { return precision == FDTD_FP64 ? 8 : 4; }
+
+// Input planes a strip tile stages in LDS (0: the direct path, which takes
+// any row length).  Staged rows move as 16-byte packs, so Ni is a whole
+// number of them, and two wavefronts share loads; two planes where the LDS holds them (the next plane's
+// loads are then always in flight: 512^3 FP32 L = 4, 1.61 ms per pass
+// against 1.65 with one), else one.
+inline int strip_stage_depth(int L, int V, int R, int W, int Ni, int precision) {
+    const size_t es = storage_size(precision);
+    const int cs = (int)compute_size(precision);
+    if (!fdtd::strip_stage_built(V, R, L) || W % 2 != 0 || (Ni * es) % 16 != 0) return 0;
+    for (int depth = 2; depth >= 1; --depth)
+        if (fdtd::strip_lds_bytes(L, W, V, R, cs, (int)es, depth) <= kLdsLimit - 64) return depth;
+    return 0;
+}
+
+// x geometry of a strip tile: a window of 64*V columns (FP64: 32) with Gx
+// ghost columns on each side (at least L, a multiple of V) and TX stored
+// columns; tiles start at multiples of TX.  With 4-byte storage, TX is a
+// multiple of 16 columns, so every stored row is whole, aligned 64-byte
+// granules: rows that begin mid-granule are written as 32-byte requests
+// (512^3 FP32 L = 4, staged: 2.01 ms per pass with 56 stored columns, 1.61
+// with 48).  FP64 rows of 24 doubles are whole granules already; FP16 keeps
+// 56 columns (a granule-aligned FP16 tile would store 32).  Grids of a batch
+// take the unaligned width (align false) where it saves a tile in x: one to
+// four tiles hold their rows, and a tile more costs more than the aligned
+// stores save (256-grid batch, both widths for all grids: 236.0 Gcell/s with
+// 56 stored columns, 221.5 with 48).
+// Staged tiles start and end on 16-byte packs: four ghost columns for every L.
+inline void strip_x_geometry(int L, int V, int precision, bool stage, int* Gx, int* TX,
+                             bool align = true) {
+    const int RW = fdtd::strip_row_lanes((int)compute_size(precision)) * V;
+    *Gx = stage ? 4 : (L + V - 1) / V * V;
+    *TX = RW - 2 * *Gx;
+    if (align && storage_size(precision) == 4) {
         const int aligned = *TX / 16 * 16;
         if (aligned >= 16 && aligned % V == 0 && aligned < *TX) {
             *TX = aligned;
-            *Gx = (64 * V - aligned) / 2;
+            *Gx = (RW - aligned) / 2;
         }
     }
 }
-inline size_t compute_size(int precision) { return precision == FDTD_FP64 ? 8 : 4; }
 inline size_t current_size(int precision) { return precision == FDTD_FP64 ? 8 : 4; }
 
 

@@ -1878,27 +1878,35 @@ blocked_sweep(BlockedArgs<S, C> a) {
 // Wavefront-strip temporally blocked sweep: L fused steps per pass over HBM.
 //
 // A workgroup of W wavefronts covers a tile of 64*V columns by W*R rows of
-// every plane.  Lane l of wavefront w owns columns l*V .. l*V+V-1 of tile
+// every plane (FP64: 32 columns by 2*W*R rows, two row groups of 32 lanes per
+// wavefront).  Lane l of row group w owns columns l*V .. l*V+V-1 of tile
 // rows w*R .. w*R+R-1 and keeps them in registers, so of the x and y
 // neighbours a cell update reads:
 //   - x: the neighbouring lane's cell, moved by a DPP wavefront shift
 //     (wave_shr:1 / wave_shl:1) -- no LDS;
-//   - y: the lane's own next/previous row, except across a wavefront's
+//   - y: the lane's own next/previous row, except across a row group's
 //     first and last row, whose two needed components (Bx, Bz below; Ex, Ez
 //     above) go through a small LDS row exchange.
-// The outer Gx columns (L rounded up to a multiple of V) and L rows on each
-// side are ghost cells: computed on every level, never stored (overlapped
-// tiling), since after L levels only cells at least L from the tile edge
-// hold the values of L unblocked steps.  Along z the levels form the same
-// pipeline as blocked_sweep: at iteration kk level l computes E_l at plane
-// kk-l and B_l at plane kk-l-1, with the per-cell expressions of
-// fused_tile, so results are bit-identical to L single fused sweeps.
+// The outer Gx columns (at least L) and L rows on each side are ghost cells:
+// computed on every level, never stored (overlapped tiling), since after L
+// levels only cells at least L from the tile edge hold the values of L
+// unblocked steps.  Along z the levels form the same pipeline as
+// blocked_sweep: at iteration kk level l computes E_l at plane kk-l and B_l at
+// plane kk-l-1, with the per-cell expressions of fused_tile, so results are
+// bit-identical to L single fused sweeps.
 //
-// LDS (per level l): sB[l] holds each wavefront's last-row Bx, Bz input of
-// level l (published before level l runs); sE[l] holds each wavefront's
-// first-row Ex, Ez of E_l one plane below (published one phase after the
-// reads of the previous value).  One barrier per level and plane (two for
-// L = 1).
+// LDS rows of level l: sB holds each row group's last-row Bx, Bz input of
+// level l, sE its first-row Ex, Ez of E_l one plane below; both are published
+// before the barrier in front of level l.  One barrier per level and plane
+// (two for L = 1).
+//
+// What bounds it (512^3 FP32, L = 4, one MI355X, staged path): 1.53 ms per
+// pass = 5.3 TB/s of real traffic (4.8 GB read: the minimum times 1.49, since
+// neighbouring tiles drift apart by more planes than an L2 holds; 3.3 GB
+// written), with the VALU busy about three quarters of the time; the
+// arithmetic alone, without loads and stores, takes 1.1 ms.  Before planes
+// went through LDS: 1.83 ms.  FP64 (64 x 16 tiles, direct): 4.62 ms, now 3.38;
+// FP16 1.74 -> 1.62 ms.
 
 // p advanced by a 32-bit unsigned byte offset (zero-extended): lets the
 // compiler address memory as a scalar base plus a 32-bit lane offset.
@@ -1939,17 +1947,56 @@ __device__ __forceinline__ T* generic(gptr<T> p) {
 
 struct StripGeom {
     int Ni, Nj, Nk;
-    int W;            // wavefronts per tile (R rows each)
-    int Gx;           // ghost columns per side: L rounded up to a multiple of V
-    int TX, TY;       // stored columns and rows per tile: 64V - 2Gx, W*R - 2L
+    int W;            // wavefronts per tile
+    int Gx;           // ghost columns per side
+    int TX, TY;       // stored columns and rows per tile
     int kchunk;
     int ntx, nty;
     int ntiles;
     int per_xcd;
+    int depth;        // staged path: input planes in LDS (1 or 2)
 };
 
-__host__ __device__ inline size_t strip_lds_bytes(int L, int W, int V, int csize) {
-    return static_cast<size_t>(4) * L * W * 64 * V * csize;
+// Lanes of a tile row.  Float compute: a wavefront is one row group of 64
+// lanes.  Double compute holds twice the register bytes per cell, so a
+// workgroup covers half as many cells; a 64 x 16 tile would store 56 x 8 of
+// them at L = 4 (2.29 cells computed per cell stored), a 32 x 32 tile
+// stores 24 x 24 (1.78): there a wavefront is two row groups of 32 lanes.
+__host__ __device__ constexpr int strip_row_lanes(int csize) { return csize == 8 ? 32 : 64; }
+
+// Tile rows of W wavefronts with R rows per lane.
+__host__ __device__ constexpr int strip_tile_rows(int W, int R, int csize) {
+    return W * R * (64 / strip_row_lanes(csize));
+}
+
+// LDS of a tile: the row exchange (per buffer two B and two E rows of every
+// row group; levels take the buffers in turn, and a buffer is written again
+// only after a barrier behind its last reads) and, on the staged path,
+// `depth` input planes and the stored rows of one output plane, all six
+// components.
+__host__ __device__ constexpr int strip_exchange_bufs(int L) { return L % 2 == 0 ? 2 : (L < 3 ? L : 3); }
+__host__ __device__ inline size_t strip_exchange_bytes(int L, int W, int V, int csize) {
+    return static_cast<size_t>(4) * strip_exchange_bufs(L) * W * 64 * V * csize;
+}
+__host__ __device__ constexpr int strip_out_row_bytes(int csize, int ssize) {
+    return (strip_row_lanes(csize) - 8) * ssize;
+}
+__host__ __device__ inline size_t strip_lds_bytes(int L, int W, int V, int R, int csize, int ssize,
+                                                  int depth) {
+    const size_t plane = static_cast<size_t>(6) * W * 64 * V * R * ssize;
+    const int stored = strip_tile_rows(W, R, csize) - 2 * L;
+    return strip_exchange_bytes(L, W, V, csize) + depth * plane +
+           (depth > 0 ? static_cast<size_t>(6) * stored * strip_out_row_bytes(csize, ssize) : 0);
+}
+
+// Point source lists up to this length are searched once per tile for
+// sources in its columns and rows.
+constexpr int kTileSrcScan = 64;
+
+// The staged path is built for V = 1, R = 2, L >= 2 and takes an even number
+// of wavefronts (two share their rows' loads).
+__host__ __device__ constexpr bool strip_stage_built(int V, int R, int L) {
+    return V == 1 && R == 2 && L >= 2;
 }
 
 // Workgroup size bound of a strip variant: lanes holding more state get
@@ -2004,13 +2051,39 @@ __device__ __forceinline__ double lane_next(double x) {
     return __builtin_bit_cast(double, h);
 }
 
+// Global memory straight to LDS: lane i's BYTES bytes at base + off go to
+// LDS offset lds + i*BYTES (base and lds are uniform; lanes switched off
+// write nothing).  No register is written: the data is there once the
+// wavefront has waited for vmcnt.  In assembly, because the compiler makes
+// every later LDS read wait for the builtin's transfer.
+template <int BYTES, typename T>
+__device__ __forceinline__ void load_to_lds(gptr<T> base, unsigned off, unsigned lds) {
+    static_assert(BYTES == 4 || BYTES == 16, "4 or 16 bytes per lane");
+    if constexpr (BYTES == 16)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off),
+                     "s"(base), "s"(lds) : "memory");
+    else
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off),
+                     "s"(base), "s"(lds) : "memory");
+}
+
 // One tile (index < a.g.ntiles) of a strip pass; every thread of the
-// workgroup calls it with the same tile.  RESCALE (FP16 storage only): the
-// pass after an in-run rescaling decision, which scales what it reads.
-template <typename S, typename C, int V, int R, int L, bool FINAL, bool RESCALE = false,
-          bool PROBE = false>
+// workgroup calls it with the same tile.
+// STAGE: planes come in and go out through LDS.  Each wavefront moves its
+// own rows, 16 bytes per lane (4 for FP16, whose rows start at multiples of
+// 8 bytes), straight from memory to LDS one plane ahead, and writes its
+// results to LDS and from there to memory 16 bytes per lane: 3 loads and 3
+// stores per wavefront and plane instead of 12 and 12 (FP32).  Issued in
+// bursts between the levels' barriers, the 12 + 12 accesses kept the
+// wavefronts waiting for the memory pipe's queue.  Needs rows that are
+// whole 16-byte packs (Ni, TX) at pack-aligned window starts.
+// RESCALE (FP16 storage only): the pass after an in-run rescaling decision,
+// which scales what it reads.
+template <typename S, typename C, int V, int R, int L, bool FINAL, bool STAGE,
+          bool RESCALE = false, bool PROBE = false>
 __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int tile,
                                            C* __restrict__ lds) {
+    static_assert(!STAGE || strip_stage_built(V, R, L), "staged shape");
     const StripGeom& G = a.g;
     const int txy = G.ntx * G.nty;
     const int chunk = tile / txy;
@@ -2018,11 +2091,13 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
     const int ty = rem / G.ntx;
     const int tx = rem - ty * G.ntx;
 
-    constexpr int RW = 64 * V;
-    const int Ni = G.Ni, Nj = G.Nj, Nk = G.Nk, W = G.W;
-    const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
-    const int cx0 = lane * V;                          // tile column of the lane's first cell
+    constexpr int LN = strip_row_lanes(sizeof(C));
+    constexpr int GPW = 64 / LN;                       // row groups per wavefront
+    constexpr int RW = LN * V;                         // tile columns
+    const int Ni = G.Ni, Nj = G.Nj, Nk = G.Nk;
+    const int ngroups = G.W * GPW;
+    const int w = threadIdx.x / LN;                    // row group
+    const int cx0 = (threadIdx.x & (LN - 1)) * V;      // tile column of the lane's first cell
     const int px0 = tx * G.TX;                         // global column of the first stored column
     const int gi0 = wrap_mod(px0 - G.Gx + cx0, Ni);    // V | Gx, V | TX: packs never straddle the wrap
     const int py0 = ty * G.TY;
@@ -2048,14 +2123,14 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
     const int k0 = chunk * G.kchunk;
     const int k1 = min(k0 + G.kchunk, Nk);
     const int plane = Ni * Nj;
-    // Memory path.  FP64 and FP16 storage prefetch and store through plane
-    // buffer resources, issued on every path, so that waiting for the
-    // prefetch does not wait for the stores issued after it (measured:
-    // FP64 passes about 11%, FP16 passes 12-16% faster than with global
-    // accesses).
-    // FP32 keeps global accesses under branches, whose waits do include the
-    // previous plane's stores: its buffer form measured 4-5% slower.
-    constexpr bool kBuf = sizeof(S) != 4;
+    const size_t pbytes64 = static_cast<size_t>(plane) * sizeof(S);
+    // Memory path without STAGE.  FP64 and FP16 storage prefetch and store
+    // through plane buffer resources, issued on every path, so that waiting
+    // for the prefetch does not wait for the stores issued after it.  FP32
+    // uses global accesses, its loads two components per level (512^3, L = 4:
+    // 1.68 ms per pass against 1.83 with all twelve loads in one burst).
+    constexpr bool kBuf = !STAGE && sizeof(S) != 4;
+    constexpr bool kGlob = !STAGE && sizeof(S) == 4;
     const unsigned pbytes = static_cast<unsigned>(plane) * static_cast<unsigned>(sizeof(S));
     // store offsets: kBufSkip outside the stored rows and columns
     unsigned st_off[R][V];
@@ -2065,21 +2140,182 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
         for (int v = 0; v < V; ++v)
             st_off[r][v] = kBuf && row_out[r] && col_out[v]
                                ? row_off[r] + static_cast<unsigned>(v * sizeof(S)) : kBufSkip;
-    // wavefront whose last row lies below / first row above this one's
-    // (the end wavefronts read their own: those rows are ghost rows)
-    const int wm = w > 0 ? w - 1 : w, wp = w + 1 < W ? w + 1 : w;
-    // LDS rows grouped by wavefront, so that the level and component parts
+    // row group whose last row lies below / first row above this one's
+    // (the end groups read their own: those rows are ghost rows)
+    const int wm = w > 0 ? w - 1 : w, wp = w + 1 < ngroups ? w + 1 : w;
+    // LDS rows grouped by row group, so that the buffer and component parts
     // of an address are compile-time offsets from one of three bases (this,
-    // the previous and the next wavefront's block)
+    // the previous and the next group's block).  Level l's rows are published
+    // before the barrier in front of it; the staged path reads level 0's B
+    // rows from the staged plane.
     using lds_c = __attribute__((address_space(3))) C*;
+    using lds_b = __attribute__((address_space(3))) char*;
+    constexpr int NXB = strip_exchange_bufs(L);
+    constexpr int XB = 4 * NXB * RW;
     auto sB = [&](int l, int c, int ww) {
-        return (lds_c)lds + ww * (4 * L * RW) + (l * 2 + c) * RW + cx0;
+        return (lds_c)lds + ww * XB + ((l % NXB) * 4 + c) * RW + cx0;
     };
     auto sE = [&](int l, int c, int ww) {
-        return (lds_c)lds + ww * (4 * L * RW) + ((L + l) * 2 + c) * RW + cx0;
+        return (lds_c)lds + ww * XB + ((l % NXB) * 4 + 2 + c) * RW + cx0;
     };
     const Coefs<C> c = a.c;
     const cptr<int> kst = as_const(a.kstart);
+    const int kfirst = k0 - L + 1, klast = k1 + L - 1;
+
+    // ---- staged planes: input per RL rows [component][row][RW] (components
+    // Ex Ey Ez Bx By Bz), output [stored row][component][RW - 8]
+    constexpr int RPW = R * GPW;                       // tile rows per wavefront
+    constexpr int RB = RW * static_cast<int>(sizeof(S));
+    constexpr int CB = RPW * RB;                       // one component's rows
+    constexpr int OB = strip_out_row_bytes(sizeof(C), sizeof(S));
+    constexpr int LB = sizeof(S) == 2 ? 4 : 16;        // bytes a lane loads at once
+    constexpr int RL = 64 * LB / RB > 0 ? 64 * LB / RB : 1;  // rows of one load (one component)
+    constexpr int WL = RL / RPW > 0 ? RL / RPW : 1;    // wavefronts sharing their rows' loads
+    constexpr int NQ = 6 / WL;                         // loads per wavefront and plane
+    static_assert(!STAGE || (RL == WL * RPW && RL * RB == 64 * LB), "whole rows per load");
+    constexpr int WM = strip_max_threads(V, R, L, sizeof(C)) / 64;
+    constexpr int NST = STAGE ? ((WM * RPW - 2 * L) * 6 * (OB / 16) + 64 * WM - 1) / (64 * WM) : 1;
+    constexpr int NSA = STAGE ? (3 * RPW * (OB / 16) + 63) / 64 : 1;
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4), may_alias));
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane64 = threadIdx.x & 63;
+    const int depth = G.depth;
+    const int stage_bytes = G.W * (6 * CB);
+    const lds_b stage0 = (lds_b)lds + ngroups * XB * static_cast<int>(sizeof(C));
+    const lds_b out0 = stage0 + depth * stage_bytes;
+    auto stage_row = [&](int ww) {  // row 0, component 0 of row group ww, this lane's column
+        return stage0 + (ww / (WL * GPW)) * (6 * WL * CB) + (ww % (WL * GPW)) * (R * RB) +
+               cx0 * static_cast<int>(sizeof(S));
+    };
+    using lds_s = const __attribute__((address_space(3))) S*;
+    const lds_b in_own = stage_row(w), in_prev = stage_row(wm);
+    const lds_b out_own = out0 + (w * R - L) * (6 * OB) + (cx0 - G.Gx) * static_cast<int>(sizeof(S));
+    const S* ldp[NQ];          // component of each load (uniform)
+    unsigned ld_off = 0;       // this lane's byte offset in a plane
+    bool ld_ok = false;        // its columns are within L of the stored ones
+    char* stp[NST];            // this lane's target of each store, plane 0 (B: plane -1)
+    int st_lag[NST];           // 0 (E), 1 (B: one plane behind) or out of range
+    unsigned st_lds[NST];      // its offset in out0
+    char* sap[NSA];            // the same for the carried half step (this wavefront's rows), plane 0
+    unsigned sa_lds[NSA];
+    if constexpr (STAGE) {
+        const int row = lane64 * LB / RB, col = lane64 * LB % RB / static_cast<int>(sizeof(S));
+        ld_off = static_cast<unsigned>(wrap_mod(py0 - L + wave / WL * RL + row, Nj) * Ni +
+                                       wrap_mod(px0 - G.Gx + col, Ni)) * static_cast<unsigned>(sizeof(S));
+        ld_ok = col + LB / static_cast<int>(sizeof(S)) > G.Gx - L && col < G.Gx + G.TX + L;
+        static_assert(WL <= 2, "E by even, B by odd wavefronts");
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+            ldp[q] = WL == 2 ? (wave & 1 ? a.in.b[q % 3] : a.in.e[q % 3])
+                             : (q < 3 ? a.in.e[q % 3] : a.in.b[q % 3]);
+        // 16-byte pack p of the stored rows [row0, row0 + rows) (in tile rows
+        // from L), components [0, ncomp): its place in memory and in out0
+        constexpr int PK = 16 / static_cast<int>(sizeof(S));
+        const int txc = G.TX / PK;
+        auto target = [&](int p, int row0, int rows, int ncomp, int* cc, size_t* off, unsigned* lo) {
+            const int rc = p / txc, col0 = (p - rc * txc) * PK;
+            const int rr = row0 + rc / ncomp;
+            *cc = rc - (rc / ncomp) * ncomp;
+            const bool ok = rc < rows * ncomp && rr >= 0 && rr < G.TY && py0 + rr < Nj && px0 + col0 < Ni;
+            *off = ok ? static_cast<size_t>((py0 + rr) * Ni + px0 + col0) * sizeof(S) : 0;
+            *lo = ok ? (rr * 6 + *cc) * OB + col0 * static_cast<int>(sizeof(S)) : 0;
+            return ok;
+        };
+#pragma unroll
+        for (int i = 0; i < NST; ++i) {
+            int cc;
+            size_t off;
+            const bool ok = target(i * 64 * G.W + threadIdx.x, 0, G.TY, 6, &cc, &off, &st_lds[i]);
+            S* p = a.out.e[0];
+            if (cc == 1) p = a.out.e[1];
+            if (cc == 2) p = a.out.e[2];
+            if (cc == 3) p = a.out.b[0];
+            if (cc == 4) p = a.out.b[1];
+            if (cc == 5) p = a.out.b[2];
+            st_lag[i] = ok ? (cc >= 3 ? 1 : 0) : (1 << 30);
+            stp[i] = reinterpret_cast<char*>(p) + off - (cc >= 3 ? pbytes64 : 0);
+        }
+        if constexpr (FINAL) {
+#pragma unroll
+            for (int i = 0; i < NSA; ++i) {
+                int cc;
+                size_t off;
+                const bool ok = target(i * 64 + lane64, wave * RPW - L, RPW, 3, &cc, &off, &sa_lds[i]) &&
+                                a.ahead[0] != nullptr;
+                S* p = a.ahead[0];
+                if (cc == 1) p = a.ahead[1];
+                if (cc == 2) p = a.ahead[2];
+                sap[i] = ok ? reinterpret_cast<char*>(p) + off : nullptr;
+            }
+        }
+    }
+    // Whether a point source lies in this tile's columns and rows (ghosts
+    // included): other tiles look at no source table while they march.  Long
+    // lists are not searched.
+    bool tile_src = a.nsrc > kTileSrcScan;
+    if (a.nsrc > 0 && !tile_src) {
+        const cptr<PointSource> src = as_const(a.src);
+        for (int q = 0; q < a.nsrc; ++q) {
+            const int di = wrap_mod(src[q].i - px0 + G.Gx, Ni), dj = wrap_mod(src[q].j - py0 + L, Nj);
+            tile_src = tile_src || (di < RW && dj < ngroups * R);
+        }
+    }
+    // Likewise for the probes and the cells this tile stores.
+    bool tile_probe = PROBE && a.probe.n > kTileSrcScan;
+    if (PROBE && !tile_probe) {
+        const cptr<Probe> pr = as_const(a.probe.p);
+        for (int q = 0; q < a.probe.n; ++q)
+            tile_probe = tile_probe || (pr[q].i >= px0 && pr[q].i < px0 + G.TX && pr[q].j >= py0 &&
+                                        pr[q].j < py0 + G.TY);
+    }
+    // Adds sources q0..q1-1 to the first curl terms, as add_point_sources
+    // does.  The lane's cell is worked out here, from an opaque copy of the
+    // thread index, so that the march does not keep it in registers.
+    auto add_sources = [&](C (&t)[R][3][V], int q0, int q1, const double* vals_g) {
+        int th = threadIdx.x;
+        asm volatile("" : "+v"(th));
+        const cptr<PointSource> src = as_const(a.src);
+        const cptr<double> vals = as_const(vals_g);
+        const int si0 = wrap_mod(px0 - G.Gx + (th & (LN - 1)) * V, Ni);
+        for (int q = q0; q < q1; ++q) {
+            const int comp = src[q].comp, di = src[q].i - si0;
+            const C x = (comp == 0 ? c.jx : (comp == 1 ? c.jy : c.jz)) * C(vals[q]);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const bool row = wrap_mod(py0 - L + (th / LN) * R + r, Nj) == src[q].j;
+#pragma unroll
+                for (int v = 0; v < V; ++v) {
+                    const bool hit = row && di == v;
+#pragma unroll
+                    for (int d = 0; d < 3; ++d)
+                        if (comp == d) t[r][d][v] = hit ? x + t[r][d][v] : t[r][d][v];
+                }
+            }
+        }
+    };
+    // plane kk of the input on its way to this wavefront's part of the stage
+    auto stage_at = [&](int kk) { return depth == 2 ? ((kk - kfirst) & 1) * stage_bytes : 0; };
+    auto stage_load = [&](int kk) {
+        const size_t off = static_cast<size_t>(wrap_mod(kk, Nk)) * plane;
+        const lds_b d0 = stage0 + stage_at(kk) + wave / WL * (6 * WL * CB) + wave % WL * (NQ * RL * RB);
+        const unsigned dst = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(
+            reinterpret_cast<unsigned long long>(d0)));
+        if (ld_ok) {
+#pragma unroll
+            for (int q = 0; q < NQ; ++q)
+                load_to_lds<LB>(uniform_gptr<const S>(ldp[q] + off), ld_off, dst + q * 64 * LB);
+        }
+    };
+    // the tile's results (E at plane pe, B at pe-1) from LDS to memory
+    auto stage_store = [&](int pe) {
+        const long long off = static_cast<long long>(pe) * static_cast<long long>(pbytes64);
+#pragma unroll
+        for (int i = 0; i < NST; ++i)
+            if (static_cast<unsigned>(pe - st_lag[i] - k0) < static_cast<unsigned>(k1 - k0)) {
+                const u32x4 x = *(const __attribute__((address_space(3))) u32x4*)(out0 + st_lds[i]);
+                __builtin_nontemporal_store(x, reinterpret_cast<u32x4*>(stp[i] + off));
+            }
+    };
 
     C bP[L][3][R][V];  // level l: B input one plane below its E plane
     C eP[L][3][R][V];  // level l: E output of the previous iteration
@@ -2095,11 +2331,27 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
                     eP[l][d][r][v] = C(0);
                 }
 
-    const int kfirst = k0 - L + 1, klast = k1 + L - 1;
     C en[3][R][V], bn[3][R][V];
+    auto rescale_plane = [&]() {
+        if constexpr (RESCALE) {
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+#pragma unroll
+                    for (int v = 0; v < V; ++v) {
+                        bn[d][r][v] = as_stored<S>(bn[d][r][v] * a.iscale[3 + d]);
+                        en[d][r][v] = as_stored<S>(en[d][r][v] * a.iscale[d]);
+                    }
+        }
+    };
     {
         const size_t offm = static_cast<size_t>(wrap_mod(kfirst - 1, Nk)) * plane;
         const size_t off = static_cast<size_t>(wrap_mod(kfirst, Nk)) * plane;
+        if constexpr (STAGE) {
+            stage_load(kfirst);
+            if (depth == 2 && kfirst < klast) stage_load(kfirst + 1);
+        }
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
             const gptr<const S> bm = uniform_gptr<const S>(a.in.b[d] + offm);
@@ -2108,8 +2360,10 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 load_pack<S, C, V>(generic(at(bm, row_off[r])), bP[0][d][r]);
-                load_pack<S, C, V>(generic(at(b0, row_off[r])), bn[d][r]);
-                load_pack<S, C, V>(generic(at(e0, row_off[r])), en[d][r]);
+                if constexpr (!STAGE) {
+                    load_pack<S, C, V>(generic(at(b0, row_off[r])), bn[d][r]);
+                    load_pack<S, C, V>(generic(at(e0, row_off[r])), en[d][r]);
+                }
             }
         }
     }
@@ -2119,20 +2373,16 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
 #pragma unroll
             for (int r = 0; r < R; ++r)
 #pragma unroll
-                for (int v = 0; v < V; ++v) {
+                for (int v = 0; v < V; ++v)
                     bP[0][d][r][v] = as_stored<S>(bP[0][d][r][v] * a.iscale[3 + d]);
-                    bn[d][r][v] = as_stored<S>(bn[d][r][v] * a.iscale[3 + d]);
-                    en[d][r][v] = as_stored<S>(en[d][r][v] * a.iscale[d]);
-                }
+        if constexpr (!STAGE) rescale_plane();
     }
-    // E rows are read (for ghost-plane results only) before their first write
+    // level 0's E rows (read for ghost-plane results only)
 #pragma unroll
-    for (int l = 0; l < L; ++l)
+    for (int q = 0; q < 2; ++q)
 #pragma unroll
-        for (int q = 0; q < 2; ++q)
-#pragma unroll
-            for (int v = 0; v < V; ++v) sE(l, q, w)[v] = C(0);
-    // level 0's B input row for the wavefront below: the buffer path
+        for (int v = 0; v < V; ++v) sE(0, q, w)[v] = C(0);
+    // level 0's B input row for the row group below: the buffer path
     // publishes it at the end of the previous iteration (after the barriers
     // that follow its last reads), once the prefetch has been waited for
     if constexpr (kBuf) {
@@ -2146,26 +2396,23 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
     // for its own prefetches (and, in the global path, not for its stores)
     wait_vmem_all();
 
-    // One plane iteration: level l reads its state of the previous
-    // iteration from (ePi, bPi) and leaves the new one in (ePo, bPo) -- the
-    // same arrays here: each element is read before it is overwritten.
-    // (Alternating two state sets over an unrolled pair of iterations
-    // removes the register copies of the pipeline rotation, but measured
-    // slower: FP32 L=4 spills at 128 VGPRs, FP16 -5%, FP64 +3%.)
-    auto plane_step = [&](const int kk, const C (&ePi)[L][3][R][V], const C (&bPi)[L][3][R][V],
-                          C (&ePo)[L][3][R][V], C (&bPo)[L][3][R][V])
-                          __attribute__((always_inline)) {
+    // One plane iteration.  Two are unrolled on the staged path: the pipeline
+    // state then alternates between two register sets instead of being copied
+    // to its place after every plane (45 of the FP32 loop's 335 VALU
+    // instructions; 512^3 L = 4: 1.58 -> 1.53 ms per pass, FP64 3.45 -> 3.38,
+    // FP16 1.71 -> 1.62).
+    auto plane_step = [&](const int kk) __attribute__((always_inline)) {
         // lane offsets of this iteration's global accesses, redefined each
         // iteration (an empty asm) so that the compiler forms every address
         // as a scalar plane base plus a 32-bit lane offset instead of
         // hoisting 64-bit per-lane sums out of the loop
         unsigned lo[R];
+        if constexpr (kGlob) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            lo[r] = row_off[r];
-            asm volatile("" : "+v"(lo[r]));
-        }
-        if constexpr (!kBuf) {
+            for (int r = 0; r < R; ++r) {
+                lo[r] = row_off[r];
+                asm volatile("" : "+v"(lo[r]));
+            }
 #pragma unroll
             for (int v = 0; v < V; ++v) {
                 sB(0, 0, w)[v] = bn[0][R - 1][v];
@@ -2173,24 +2420,10 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
             }
         }
         // prefetch of plane kk+1 (buffer path: a size-0 resource after the
-        // last plane)
+        // last plane; global path: the last plane again)
         RawPack<S, V> rawE[3][R], rawB[3][R];
         const bool more = kk < klast;
-        if constexpr (!kBuf) {
-            if (more) {
-                const size_t off = static_cast<size_t>(wrap_mod(kk + 1, Nk)) * plane;
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    const gptr<const S> bb = uniform_gptr<const S>(a.in.b[d] + off);
-                    const gptr<const S> eb = uniform_gptr<const S>(a.in.e[d] + off);
-#pragma unroll
-                    for (int r = 0; r < R; ++r) {
-                        rawB[d][r] = load_raw<S, V>(generic(at(bb, lo[r])));
-                        rawE[d][r] = load_raw<S, V>(generic(at(eb, lo[r])));
-                    }
-                }
-            }
-        } else {
+        if constexpr (kBuf) {
             const unsigned nb = more ? pbytes : 0u;
             const size_t off = static_cast<size_t>(wrap_mod(kk + 1, Nk)) * plane;
 #pragma unroll
@@ -2204,7 +2437,35 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
                 }
             }
         }
+        // the staged plane kk (each wavefront's own loads) has arrived; with
+        // two planes staged, the NQ loads of plane kk+1 may be in flight
+        if constexpr (STAGE) {
+            if (depth == 2 && more)
+                __builtin_amdgcn_s_waitcnt(0x0F70 | NQ);
+            else
+                wait_vmem_all();
+        }
         __syncthreads();
+
+        C b_prev[2][V];  // level 0: Bx, Bz of the row below the group
+        if constexpr (STAGE) {
+            const int sat = stage_at(kk);
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    en[d][r][0] = static_cast<C>(*(lds_s)(in_own + sat + d * (WL * CB) + r * RB));
+                    bn[d][r][0] = static_cast<C>(*(lds_s)(in_own + sat + (3 + d) * (WL * CB) + r * RB));
+                }
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                b_prev[q][0] = static_cast<C>(*(lds_s)(in_prev + sat + (3 + 2 * q) * (WL * CB) + (R - 1) * RB));
+                if constexpr (RESCALE)
+                    b_prev[q][0] = as_stored<S>(b_prev[q][0] * a.iscale[3 + 2 * q]);
+            }
+            rescale_plane();
+            stage_store(kk - L);  // the previous iteration's results
+        }
 
         C bin[3][R][V];  // B input of the current level at its E plane
         C ein[3][R][V];  // E input of the current level
@@ -2212,7 +2473,7 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
         // (B + d) + d of the last level's B plane kk-L, as it is computed
         const bool carry_plane = FINAL && a.ahead[0] != nullptr && kk - L >= k0 && kk - L < k1;
         const size_t carry_off = static_cast<size_t>(carry_plane ? kk - L : k0) * plane;
-        C cy[3][R][V];  // global path, FINAL: the carried half step of the last level
+        C cy[3][R][V];  // FINAL, but for the buffer path: the carried half step of the last level
 #pragma unroll
         for (int d = 0; d < 3; ++d)
 #pragma unroll
@@ -2224,49 +2485,68 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
                 }
 #pragma unroll
         for (int l = 0; l < L; ++l) {
-            // this level's E plane is kk - l (pkl wrapped); its B plane is kk - l - 1
-            if (L > 1) {
-                // publish the first-row Ex, Ez of the level whose readers
-                // have all passed the last barrier
-                const int lp = l == 0 ? L - 1 : l - 1;
-                const C (&prevE)[3][R][V] = l == 0 ? ePi[L - 1] : ePo[(l + L - 1) % L];
+            // this level's E plane is kk - l; its B plane is kk - l - 1
+            if (kGlob && l < 3) {
+                // prefetch of plane kk+1, component l
+                const size_t off = static_cast<size_t>(wrap_mod(more ? kk + 1 : kk, Nk)) * plane;
+                const gptr<const S> bb = uniform_gptr<const S>(a.in.b[l] + off);
+                const gptr<const S> eb = uniform_gptr<const S>(a.in.e[l] + off);
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    rawB[l][r] = load_raw<S, V>(generic(at(bb, lo[r])));
+                    rawE[l][r] = load_raw<S, V>(generic(at(eb, lo[r])));
+                }
+#pragma unroll
+                for (int d = L; d < 3; ++d)  // passes of fewer than three levels: the rest here
+                    if (l == L - 1) {
+                        const gptr<const S> bd = uniform_gptr<const S>(a.in.b[d] + off);
+                        const gptr<const S> ed = uniform_gptr<const S>(a.in.e[d] + off);
+#pragma unroll
+                        for (int r = 0; r < R; ++r) {
+                            rawB[d][r] = load_raw<S, V>(generic(at(bd, lo[r])));
+                            rawE[d][r] = load_raw<S, V>(generic(at(ed, lo[r])));
+                        }
+                    }
+            }
+            C t[R][3][V];
+            C bx_jm[R][V], bz_im[R][V];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
 #pragma unroll
                 for (int v = 0; v < V; ++v) {
-                    sE(lp, 0, w)[v] = prevE[0][0][v];
-                    sE(lp, 1, w)[v] = prevE[2][0][v];
+                    C bz_jm;
+                    if (r > 0) {
+                        bx_jm[r][v] = bin[0][r - 1][v];
+                        bz_jm = bin[2][r - 1][v];
+                    } else if (STAGE && l == 0) {
+                        bx_jm[r][v] = b_prev[0][v];
+                        bz_jm = b_prev[1][v];
+                    } else {
+                        bx_jm[r][v] = sB(l, 0, wm)[v];
+                        bz_jm = sB(l, 1, wm)[v];
+                    }
+                    const C by_im = v > 0 ? bin[1][r][v - 1] : lane_prev(bin[1][r][V - 1]);
+                    bz_im[r][v] = v > 0 ? bin[2][r][v - 1] : lane_prev(bin[2][r][V - 1]);
+                    t[r][0][v] = c.ex_bz * (bin[2][r][v] - bz_jm);
+                    t[r][1][v] = c.ey_bx * (bin[0][r][v] - bP[l][0][r][v]);
+                    t[r][2][v] = c.ez_by * (bin[1][r][v] - by_im);
                 }
             }
-            // point sources of plane pkl: [kstart[pkl], kstart[pkl + 1])
-            const int pkl = wrap_mod(kk - l, Nk);
-            int q0 = 0, q1 = 0;
-            if (a.nsrc > 0) {
-                q0 = kst[pkl];
-                q1 = kst[pkl + 1];
+            if (tile_src) {
+                // point sources of plane pkl: [kstart[pkl], kstart[pkl + 1])
+                const int pkl = wrap_mod(kk - l, Nk);
+                const int q0 = kst[pkl], q1 = kst[pkl + 1];
+                if (q1 > q0) add_sources(t, q0, q1, a.vals + l * a.vstride);
             }
             C enew[3][R][V];
 #pragma unroll
-            for (int r = 0; r < R; ++r) {
-                C t[3][V];
+            for (int r = 0; r < R; ++r)
 #pragma unroll
                 for (int v = 0; v < V; ++v) {
-                    const C bz_jm = r > 0 ? bin[2][r - 1][v] : sB(l, 1, wm)[v];
-                    const C by_im = v > 0 ? bin[1][r][v - 1] : lane_prev(bin[1][r][V - 1]);
-                    t[0][v] = c.ex_bz * (bin[2][r][v] - bz_jm);
-                    t[1][v] = c.ey_bx * (bin[0][r][v] - bPi[l][0][r][v]);
-                    t[2][v] = c.ez_by * (bin[1][r][v] - by_im);
+                    enew[0][r][v] = ein[0][r][v] + sub_mul(t[r][0][v], c.ex_by, bin[1][r][v] - bP[l][1][r][v]);
+                    enew[1][r][v] = ein[1][r][v] + sub_mul(t[r][1][v], c.ey_bz, bin[2][r][v] - bz_im[r][v]);
+                    enew[2][r][v] = ein[2][r][v] + sub_mul(t[r][2][v], c.ez_bx, bin[0][r][v] - bx_jm[r][v]);
                 }
-                if (q1 > q0)
-                    add_point_sources<C, V>(t, c, a.src, a.vals + l * a.vstride, q0, q1, gi0, gj[r],
-                                            pkl);
-#pragma unroll
-                for (int v = 0; v < V; ++v) {
-                    const C bx_jm = r > 0 ? bin[0][r - 1][v] : sB(l, 0, wm)[v];
-                    const C bz_im = v > 0 ? bin[2][r][v - 1] : lane_prev(bin[2][r][V - 1]);
-                    enew[0][r][v] = ein[0][r][v] + sub_mul(t[0][v], c.ex_by, bin[1][r][v] - bPi[l][1][r][v]);
-                    enew[1][r][v] = ein[1][r][v] + sub_mul(t[1][v], c.ey_bz, bin[2][r][v] - bz_im);
-                    enew[2][r][v] = ein[2][r][v] + sub_mul(t[2][v], c.ez_bx, bin[0][r][v] - bx_jm);
-                }
-            }
             // B_l at plane pe-1 from E_l(pe-1) (eP) and E_l(pe) (enew)
             C bnew[3][R][V];
             C bh[3][R][V];  // B after step l of the pass (the first half step's sum)
@@ -2274,16 +2554,16 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
             for (int r = 0; r < R; ++r)
 #pragma unroll
                 for (int v = 0; v < V; ++v) {
-                    const C ey_ip = v < V - 1 ? ePi[l][1][r][v + 1] : lane_next(ePi[l][1][r][0]);
-                    const C ez_ip = v < V - 1 ? ePi[l][2][r][v + 1] : lane_next(ePi[l][2][r][0]);
-                    const C ex_jp = r < R - 1 ? ePi[l][0][r + 1][v] : sE(l, 0, wp)[v];
-                    const C ez_jp = r < R - 1 ? ePi[l][2][r + 1][v] : sE(l, 1, wp)[v];
-                    const C dbx = sub_mul(c.bx_ey * (enew[1][r][v] - ePi[l][1][r][v]), c.bx_ez, ez_jp - ePi[l][2][r][v]);
-                    const C dby = sub_mul(c.by_ez * (ez_ip - ePi[l][2][r][v]), c.by_ex, enew[0][r][v] - ePi[l][0][r][v]);
-                    const C dbz = sub_mul(c.bz_ex * (ex_jp - ePi[l][0][r][v]), c.bz_ey, ey_ip - ePi[l][1][r][v]);
-                    bnew[0][r][v] = bPi[l][0][r][v] + dbx;
-                    bnew[1][r][v] = bPi[l][1][r][v] + dby;
-                    bnew[2][r][v] = bPi[l][2][r][v] + dbz;
+                    const C ey_ip = v < V - 1 ? eP[l][1][r][v + 1] : lane_next(eP[l][1][r][0]);
+                    const C ez_ip = v < V - 1 ? eP[l][2][r][v + 1] : lane_next(eP[l][2][r][0]);
+                    const C ex_jp = r < R - 1 ? eP[l][0][r + 1][v] : sE(l, 0, wp)[v];
+                    const C ez_jp = r < R - 1 ? eP[l][2][r + 1][v] : sE(l, 1, wp)[v];
+                    const C dbx = sub_mul(c.bx_ey * (enew[1][r][v] - eP[l][1][r][v]), c.bx_ez, ez_jp - eP[l][2][r][v]);
+                    const C dby = sub_mul(c.by_ez * (ez_ip - eP[l][2][r][v]), c.by_ex, enew[0][r][v] - eP[l][0][r][v]);
+                    const C dbz = sub_mul(c.bz_ex * (ex_jp - eP[l][0][r][v]), c.bz_ey, ey_ip - eP[l][1][r][v]);
+                    bnew[0][r][v] = bP[l][0][r][v] + dbx;
+                    bnew[1][r][v] = bP[l][1][r][v] + dby;
+                    bnew[2][r][v] = bP[l][2][r][v] + dbz;
                     bh[0][r][v] = bnew[0][r][v];
                     bh[1][r][v] = bnew[1][r][v];
                     bh[2][r][v] = bnew[2][r][v];
@@ -2297,8 +2577,7 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
                         buf_store_nt(static_cast<S>(bnew[1][r][v] + dby), plane_rsrc(a.ahead[1] + carry_off, nb), st_off[r][v]);
                         buf_store_nt(static_cast<S>(bnew[2][r][v] + dbz), plane_rsrc(a.ahead[2] + carry_off, nb), st_off[r][v]);
                     } else if (!kBuf) {
-                        // stored with the level's B plane below, after the
-                        // wait for the prefetch
+                        // stored with the level's B plane below
                         cy[0][r][v] = bnew[0][r][v] + dbx;
                         cy[1][r][v] = bnew[1][r][v] + dby;
                         cy[2][r][v] = bnew[2][r][v] + dbz;
@@ -2306,10 +2585,10 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
 #pragma unroll
                     for (int d = 0; d < 3; ++d) bnew[d][r][v] = as_stored<S>(bnew[d][r][v]);
                 }
-            if constexpr (PROBE) {
+            if (PROBE && tile_probe) {
                 // probes of step l: E of plane pkl, B of plane pkl-1, cells
                 // this tile stores
-                const int pe = kk - l;
+                const int pe = kk - l, pkl = wrap_mod(pe, Nk);
                 const bool e_ok = pe >= k0 && pe < k1, b_ok = pe - 1 >= k0 && pe - 1 < k1;
                 double* const pout = a.probe.out + static_cast<size_t>(l) * a.probe.stride;
 #pragma unroll
@@ -2335,9 +2614,9 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
                 for (int r = 0; r < R; ++r)
 #pragma unroll
                     for (int v = 0; v < V; ++v) {
-                        ein[d][r][v] = as_stored<S>(ePi[l][d][r][v]);
-                        ePo[l][d][r][v] = enew[d][r][v];
-                        bPo[l][d][r][v] = bin[d][r][v];
+                        ein[d][r][v] = as_stored<S>(eP[l][d][r][v]);
+                        eP[l][d][r][v] = enew[d][r][v];
+                        bP[l][d][r][v] = bin[d][r][v];
                         bin[d][r][v] = bnew[d][r][v];
                     }
             if (l < L - 1) {
@@ -2345,13 +2624,51 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
                 for (int v = 0; v < V; ++v) {
                     sB(l + 1, 0, w)[v] = bin[0][R - 1][v];
                     sB(l + 1, 1, w)[v] = bin[2][R - 1][v];
+                    sE(l + 1, 0, w)[v] = eP[l + 1][0][0][v];
+                    sE(l + 1, 1, w)[v] = eP[l + 1][2][0][v];
                 }
                 __syncthreads();
+                // every wavefront has read the staged plane kk: another may
+                // take its place
+                if (STAGE && l == 0 && kk + depth <= klast) stage_load(kk + depth);
             }
         }
         // stores of the last level: E_{L-1} at plane kk-L+1, B_{L-1} at kk-L
         // (buffer path: size-0 resources for planes outside the chunk)
-        if constexpr (!kBuf) {
+        if constexpr (STAGE) {
+            // the lanes that hold stored cells; memory gets the plane in the
+            // next iteration, the carried half step at once
+            if constexpr (FINAL) {
+                if (carry_plane) {
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        if (row_out[r] && col_out[0])
+#pragma unroll
+                            for (int d = 0; d < 3; ++d)
+                                *(__attribute__((address_space(3))) S*)(out_own + (r * 6 + d) * OB) =
+                                    static_cast<S>(cy[d][r][0]);
+                    asm volatile("" ::: "memory");
+#pragma unroll
+                    for (int i = 0; i < NSA; ++i)
+                        if (sap[i] != nullptr) {
+                            const u32x4 x = *(const __attribute__((address_space(3))) u32x4*)(out0 + sa_lds[i]);
+                            __builtin_nontemporal_store(
+                                x, reinterpret_cast<u32x4*>(sap[i] + static_cast<size_t>(kk - L) * pbytes64));
+                        }
+                    asm volatile("" ::: "memory");
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (row_out[r] && col_out[0])
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) {
+                        *(__attribute__((address_space(3))) S*)(out_own + (r * 6 + d) * OB) =
+                            static_cast<S>(eP[L - 1][d][r][0]);
+                        *(__attribute__((address_space(3))) S*)(out_own + (r * 6 + 3 + d) * OB) =
+                            static_cast<S>(bin[d][r][0]);
+                    }
+        } else if constexpr (kGlob) {
             // the prefetch of plane kk+1 has arrived before this plane's
             // stores are issued: the wait at the end of the iteration then
             // leaves the stores in flight (their count is not known to the
@@ -2371,7 +2688,7 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
 #pragma unroll
                             for (int v = 0; v < V; ++v)
                                 if (col_out[v])
-                                    __builtin_nontemporal_store(static_cast<S>(ePo[L - 1][d][r][v]), dst + v);
+                                    __builtin_nontemporal_store(static_cast<S>(eP[L - 1][d][r][v]), dst + v);
                         }
             }
             if (pe - 1 >= k0 && pe - 1 < k1) {
@@ -2410,20 +2727,20 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
                 for (int r = 0; r < R; ++r)
 #pragma unroll
                     for (int v = 0; v < V; ++v) {
-                        buf_store_nt(static_cast<S>(ePo[L - 1][d][r][v]), re, st_off[r][v]);
+                        buf_store_nt(static_cast<S>(eP[L - 1][d][r][v]), re, st_off[r][v]);
                         buf_store_nt(static_cast<S>(bin[d][r][v]), rb, st_off[r][v]);
                     }
             }
         }
-        if (L == 1) {
-            __syncthreads();
+        // level 0's E rows of the next iteration (with one level, its rows
+        // have to be read first)
+        if (L == 1) __syncthreads();
 #pragma unroll
-            for (int v = 0; v < V; ++v) {
-                sE(0, 0, w)[v] = ePo[0][0][0][v];
-                sE(0, 1, w)[v] = ePo[0][2][0][v];
-            }
+        for (int v = 0; v < V; ++v) {
+            sE(0, 0, w)[v] = eP[0][0][0][v];
+            sE(0, 1, w)[v] = eP[0][2][0][v];
         }
-        if (kBuf || more) {
+        if constexpr (!STAGE) {
 #pragma unroll
             for (int d = 0; d < 3; ++d)
 #pragma unroll
@@ -2431,17 +2748,7 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
                     widen<S, C, V>(rawB[d][r], bn[d][r]);
                     widen<S, C, V>(rawE[d][r], en[d][r]);
                 }
-            if constexpr (RESCALE) {
-#pragma unroll
-                for (int d = 0; d < 3; ++d)
-#pragma unroll
-                    for (int r = 0; r < R; ++r)
-#pragma unroll
-                        for (int v = 0; v < V; ++v) {
-                            bn[d][r][v] = as_stored<S>(bn[d][r][v] * a.iscale[3 + d]);
-                            en[d][r][v] = as_stored<S>(en[d][r][v] * a.iscale[d]);
-                        }
-            }
+            rescale_plane();
         }
         if constexpr (kBuf) {
 #pragma unroll
@@ -2451,33 +2758,49 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
             }
         }
     };
-    for (int kk = kfirst; kk <= klast; ++kk) plane_step(kk, eP, bP, eP, bP);
+    constexpr int UNR = STAGE && !PROBE ? 2 : 1;
+    for (int kk = kfirst;;) {
+        bool done = false;
+#pragma unroll
+        for (int u = 0; u < UNR; ++u) {
+            plane_step(kk);
+            if (++kk > klast) {
+                done = true;
+                break;
+            }
+        }
+        if (done) break;
+    }
+    if constexpr (STAGE) {
+        __syncthreads();
+        stage_store(klast - L + 1);
+    }
 }
 
 // PROBE: the variant that records StripArgs::probe after each level (the
 // level's B is held in registers until then: up to 35 more VGPRs, which the
 // plain variant does without).
-template <typename S, typename C, int V, int R, int L, bool FINAL, bool PROBE = false>
+template <typename S, typename C, int V, int R, int L, bool FINAL, bool STAGE, bool PROBE = false>
 __global__ void __launch_bounds__(strip_max_threads(V, R, L, sizeof(C)))
 strip_sweep(StripArgs<S, C> a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const int blk = blockIdx.x;
     const int tile = (blk & 7) * a.g.per_xcd + (blk >> 3);
     if (tile >= a.g.ntiles) return;  // whole workgroup
-    strip_tile<S, C, V, R, L, FINAL, false, PROBE>(a, tile, reinterpret_cast<C*>(lds_raw));
+    strip_tile<S, C, V, R, L, FINAL, STAGE, false, PROBE>(a, tile, reinterpret_cast<C*>(lds_raw));
 }
 
 // FP16 storage: the strip pass after an in-run rescaling decision, reading
 // the state scaled by StripArgs::iscale (a kernel of its own, so that the
 // other passes carry none of it).
-template <typename S, typename C, int V, int R, int L, bool FINAL, bool PROBE = false>
+template <typename S, typename C, int V, int R, int L, bool FINAL, bool STAGE, bool PROBE = false>
 __global__ void __launch_bounds__(strip_max_threads(V, R, L, sizeof(C)))
 strip_rescale_sweep(StripArgs<S, C> a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const int blk = blockIdx.x;
     const int tile = (blk & 7) * a.g.per_xcd + (blk >> 3);
     if (tile >= a.g.ntiles) return;  // whole workgroup
-    strip_tile<S, C, V, R, L, FINAL, true, PROBE>(a, tile, reinterpret_cast<C*>(lds_raw));
+    strip_tile<S, C, V, R, L, FINAL, STAGE, true, PROBE>(a, tile, reinterpret_cast<C*>(lds_raw));
 }
 
 // ---------------------------------------------------------------------------
@@ -2594,8 +2917,9 @@ batch_fused_sweep(BatchArgs<S, C> a) {
     }
 }
 
-// Batched temporal blocking: one persistent launch per pass of L steps
-// over the strip tiles of every grid (the same strip_tile as a single grid).
+// Batched temporal blocking: one launch per pass of L steps, a workgroup per
+// strip tile of every grid (the same strip_tile as a single grid), costliest
+// tiles first.
 template <typename S, typename C> struct BatchStripGrid {
     Fields<S> buf[2];        // buf[p]: the grid's buffer pair used at parity p
     const PointSource* src;  // this grid's sources, sorted by plane
@@ -2614,69 +2938,53 @@ template <typename S, typename C> struct BatchStripArgs {
     const double* vals;      // source values of the pass's first step (null: no sources)
     int vstride;             // value-table row length (all sources of the batch)
     int pad;
-    unsigned int* counters;  // [0] next work item, [1] finished workgroups
 };
 
+// Strip arguments of one grid of a batch at a given parity, read as scalars
+// through the constant address space (the descriptors do not change during
+// a launch).
 template <typename S, typename C>
-__device__ __forceinline__ StripArgs<S, C> load_batch_strip_grid(const BatchStripGrid<S, C>* p,
+__device__ __forceinline__ StripArgs<S, C> load_batch_strip_grid(cptr<BatchStripGrid<S, C>> p,
                                                                  int parity, const double* vals,
                                                                  int vstride) {
     StripArgs<S, C> a;
-    const Fields<S>* in = p->buf + parity;
-    const Fields<S>* out = p->buf + (1 - parity);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        a.in.e[d] = uni(in->e[d]);
-        a.in.b[d] = uni(in->b[d]);
-        a.out.e[d] = uni(out->e[d]);
-        a.out.b[d] = uni(out->b[d]);
+        a.in.e[d] = p->buf[parity].e[d];
+        a.in.b[d] = p->buf[parity].b[d];
+        a.out.e[d] = p->buf[1 - parity].e[d];
+        a.out.b[d] = p->buf[1 - parity].b[d];
         a.ahead[d] = nullptr;
     }
-    a.src = uni(p->src);
-    a.kstart = uni(p->kstart);
-    a.vals = vals ? vals + uni(p->src_off) : nullptr;
-    a.nsrc = uni(p->nsrc);
+    a.src = p->src;
+    a.kstart = p->kstart;
+    a.vals = vals ? vals + p->src_off : nullptr;
+    a.nsrc = p->nsrc;
     a.vstride = vstride;
 #pragma unroll
     for (int c6 = 0; c6 < 6; ++c6) a.iscale[c6] = 1.0f;
     a.probe = ProbeArgs{};  // batches record no probes
-    const Coefs<C>& c = p->c;
-    a.c.ex_bz = uni(c.ex_bz); a.c.ex_by = uni(c.ex_by); a.c.ey_bx = uni(c.ey_bx);
-    a.c.ey_bz = uni(c.ey_bz); a.c.ez_by = uni(c.ez_by); a.c.ez_bx = uni(c.ez_bx);
-    a.c.jx = uni(c.jx); a.c.jy = uni(c.jy); a.c.jz = uni(c.jz);
-    a.c.bx_ey = uni(c.bx_ey); a.c.bx_ez = uni(c.bx_ez); a.c.by_ez = uni(c.by_ez);
-    a.c.by_ex = uni(c.by_ex); a.c.bz_ex = uni(c.bz_ex); a.c.bz_ey = uni(c.bz_ey);
-    const StripGeom& q = p->g;
-    a.g.Ni = uni(q.Ni); a.g.Nj = uni(q.Nj); a.g.Nk = uni(q.Nk); a.g.W = uni(q.W);
-    a.g.Gx = uni(q.Gx); a.g.TX = uni(q.TX); a.g.TY = uni(q.TY); a.g.kchunk = uni(q.kchunk);
-    a.g.ntx = uni(q.ntx); a.g.nty = uni(q.nty); a.g.ntiles = uni(q.ntiles);
-    a.g.per_xcd = uni(q.per_xcd);
+    a.c.ex_bz = p->c.ex_bz; a.c.ex_by = p->c.ex_by; a.c.ey_bx = p->c.ey_bx;
+    a.c.ey_bz = p->c.ey_bz; a.c.ez_by = p->c.ez_by; a.c.ez_bx = p->c.ez_bx;
+    a.c.jx = p->c.jx; a.c.jy = p->c.jy; a.c.jz = p->c.jz;
+    a.c.bx_ey = p->c.bx_ey; a.c.bx_ez = p->c.bx_ez; a.c.by_ez = p->c.by_ez;
+    a.c.by_ex = p->c.by_ex; a.c.bz_ex = p->c.bz_ex; a.c.bz_ey = p->c.bz_ey;
+    a.g.Ni = p->g.Ni; a.g.Nj = p->g.Nj; a.g.Nk = p->g.Nk; a.g.W = p->g.W;
+    a.g.Gx = p->g.Gx; a.g.TX = p->g.TX; a.g.TY = p->g.TY; a.g.kchunk = p->g.kchunk;
+    a.g.ntx = p->g.ntx; a.g.nty = p->g.nty; a.g.ntiles = p->g.ntiles;
+    a.g.per_xcd = p->g.per_xcd; a.g.depth = p->g.depth;
     return a;
 }
 
-template <typename S, typename C, int V, int R, int L, bool FINAL>
+template <typename S, typename C, int V, int R, int L, bool FINAL, bool STAGE>
 __global__ void __launch_bounds__(strip_max_threads(V, R, L, sizeof(C)))
 batch_strip_sweep(BatchStripArgs<S, C> a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    __shared__ int item;
-    for (;;) {
-        if (threadIdx.x == 0) item = static_cast<int>(atomicAdd(&a.counters[0], 1u));
-        __syncthreads();
-        const int t = __builtin_amdgcn_readfirstlane(item);
-        __syncthreads();
-        if (t >= a.nwork) break;
-        const int2 wv = a.work[t];
-        const StripArgs<S, C> sa = load_batch_strip_grid(a.grids + uni(wv.x), a.parity, a.vals,
-                                                         a.vstride);
-        strip_tile<S, C, V, R, L, FINAL>(sa, uni(wv.y), reinterpret_cast<C*>(lds_raw));
-    }
-    if (threadIdx.x == 0) {
-        const unsigned done = atomicAdd(&a.counters[1], 1u);
-        if (done == gridDim.x - 1) {
-            atomicExch(&a.counters[0], 0u);
-            atomicExch(&a.counters[1], 0u);
-        }
-    }
+    const cptr<int> work = reinterpret_cast<cptr<int>>(as_const(a.work));  // (grid, tile) pairs
+    const int grid = work[2 * blockIdx.x], tile = work[2 * blockIdx.x + 1];
+    const StripArgs<S, C> sa = load_batch_strip_grid<S, C>(as_const(a.grids) + grid, a.parity,
+                                                           a.vals, a.vstride);
+    strip_tile<S, C, V, R, L, FINAL, STAGE>(sa, tile, reinterpret_cast<C*>(lds_raw));
 }
 
 // B half step of grid q of a batch, reading its current buffers (buf[0])

@@ -318,8 +318,9 @@ fdtd::StripGeom make_strip_geom(const fdtd_grid* g, const BlockTuning& t) {
     G.Nj = g->Nj;
     G.Nk = g->Nk;
     G.W = t.TYg / t.R;
-    strip_x_geometry(t.L, t.V, g->esize, &G.Gx, &G.TX);
-    G.TY = t.TYg - 2 * t.L;
+    G.depth = strip_stage_depth(t.L, t.V, t.R, G.W, g->Ni, g->precision);
+    strip_x_geometry(t.L, t.V, g->precision, G.depth > 0, &G.Gx, &G.TX);
+    G.TY = fdtd::strip_tile_rows(G.W, t.R, (int)compute_size(g->precision)) - 2 * t.L;
     G.kchunk = t.kchunk;
     G.ntx = (g->Ni + G.TX - 1) / G.TX;
     G.nty = (g->Nj + G.TY - 1) / G.TY;
@@ -342,10 +343,8 @@ bool strip_valid(const fdtd_grid* g, const BlockTuning& t) {
     if ((unsigned long long)g->Ni * g->Nj * g->esize >= (1ull << 31)) return false;  // 32-bit plane offsets, buffer range checks
     const int W = t.TYg / t.R;
     if (W < 1 || W > 16 || 64 * W > fdtd::strip_max_threads(t.V, t.R, t.L, cs)) return false;
-    int Gx = 0, TX = 0;
-    strip_x_geometry(t.L, t.V, g->esize, &Gx, &TX);
-    if (TX < 1 || t.TYg - 2 * t.L < 1) return false;
-    return fdtd::strip_lds_bytes(t.L, W, t.V, cs) <= kLdsLimit;
+    if (t.TYg - 2 * t.L < 1) return false;
+    return fdtd::strip_lds_bytes(t.L, W, t.V, t.R, cs, (int)g->esize, 0) <= kLdsLimit;
 }
 
 template <typename S>
@@ -824,21 +823,27 @@ int launch_blocked_v(fdtd_grid* g, int slot, int in, int out) {
     return FDTD_OK;
 }
 
+// The strip kernel of a launch (STAGE: planes through LDS).  FP16: the pass
+// after an in-run rescaling decision scales its reads; passes of a run with
+// probes record them.
+template <typename S, int V, int R, int L, bool FINAL, bool STAGE>
+auto strip_kernel(bool rescale, bool probe) {
+    using C = typename fdtd::ComputeOf<S>::type;
+    auto kern = probe ? fdtd::strip_sweep<S, C, V, R, L, FINAL, STAGE, true>
+                      : fdtd::strip_sweep<S, C, V, R, L, FINAL, STAGE, false>;
+    if constexpr (sizeof(S) == 2)
+        if (rescale)
+            kern = probe ? fdtd::strip_rescale_sweep<S, C, V, R, L, FINAL, STAGE, true>
+                         : fdtd::strip_rescale_sweep<S, C, V, R, L, FINAL, STAGE, false>;
+    return kern;
+}
+
 template <typename S, int V, int R, int L, bool FINAL>
 int launch_strip_v(fdtd_grid* g, int slot, int in, int out, void* const* in_b, void* const* ahead) {
     using C = typename fdtd::ComputeOf<S>::type;
     if constexpr (!strip_built(sizeof(C), V, R)) {
         return fail(FDTD_ERR_UNSUPPORTED, "strip variant V=%d R=%d not built", V, R);
     } else {
-        // FP16: the pass after an in-run rescaling decision scales its
-        // reads; passes of a run with probes record them
-        const bool probe = probing(g);
-        auto kern = probe ? fdtd::strip_sweep<S, C, V, R, L, FINAL, true>
-                          : fdtd::strip_sweep<S, C, V, R, L, FINAL, false>;
-        if constexpr (sizeof(S) == 2)
-            if (g->pass_rescale)
-                kern = probe ? fdtd::strip_rescale_sweep<S, C, V, R, L, FINAL, true>
-                             : fdtd::strip_rescale_sweep<S, C, V, R, L, FINAL, false>;
         const BlockTuning& t = g->btune;
         fdtd::StripArgs<S, C> a;
         a.in = fields_of<S>(g, in);
@@ -855,7 +860,10 @@ int launch_strip_v(fdtd_grid* g, int slot, int in, int out, void* const* in_b, v
         a.g = make_strip_geom(g, t);
         for (int c = 0; c < 6; ++c) a.iscale[c] = g->pass_iscale[c];
         a.probe = probe_args(g);
-        const size_t lds = fdtd::strip_lds_bytes(L, a.g.W, V, sizeof(C));
+        auto kern = strip_kernel<S, V, R, L, FINAL, false>(g->pass_rescale, probing(g));
+        if constexpr (fdtd::strip_stage_built(V, R, L))
+            if (a.g.depth > 0) kern = strip_kernel<S, V, R, L, FINAL, true>(g->pass_rescale, probing(g));
+        const size_t lds = fdtd::strip_lds_bytes(L, a.g.W, V, R, sizeof(C), sizeof(S), a.g.depth);
         if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
         hipLaunchKernelGGL(kern, dim3(8 * a.g.per_xcd), dim3(64 * a.g.W), lds, g->stream, a);
         HIP_TRY(hipGetLastError());
@@ -866,13 +874,15 @@ int launch_strip_v(fdtd_grid* g, int slot, int in, int out, void* const* in_b, v
 
 // Workgroups of a strip variant resident per CU (0 if it cannot launch).
 template <typename S, int V, int R, int L>
-int strip_occupancy_v(int W) {
+int strip_occupancy_v(int W, int depth) {
     using C = typename fdtd::ComputeOf<S>::type;
     if constexpr (!strip_built(sizeof(C), V, R)) {
         return 0;
     } else {
-        auto kern = fdtd::strip_sweep<S, C, V, R, L, false>;
-        const size_t lds = fdtd::strip_lds_bytes(L, W, V, sizeof(C));
+        auto kern = fdtd::strip_sweep<S, C, V, R, L, false, false>;
+        if constexpr (fdtd::strip_stage_built(V, R, L))
+            if (depth > 0) kern = fdtd::strip_sweep<S, C, V, R, L, false, true>;
+        const size_t lds = fdtd::strip_lds_bytes(L, W, V, R, sizeof(C), sizeof(S), depth);
         if (allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds) != FDTD_OK) return 0;
         int n = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, 64 * W, lds) != hipSuccess) {
@@ -884,29 +894,30 @@ int strip_occupancy_v(int W) {
 }
 
 template <typename S, int V, int R>
-int strip_occupancy_l(int L, int W) {
+int strip_occupancy_l(int L, int W, int depth) {
     switch (L) {
-        case 1: return strip_occupancy_v<S, V, R, 1>(W);
-        case 2: return strip_occupancy_v<S, V, R, 2>(W);
-        case 3: return strip_occupancy_v<S, V, R, 3>(W);
-        default: return strip_occupancy_v<S, V, R, 4>(W);
+        case 1: return strip_occupancy_v<S, V, R, 1>(W, depth);
+        case 2: return strip_occupancy_v<S, V, R, 2>(W, depth);
+        case 3: return strip_occupancy_v<S, V, R, 3>(W, depth);
+        default: return strip_occupancy_v<S, V, R, 4>(W, depth);
     }
 }
 
 template <typename S>
-int strip_occupancy_s(const BlockTuning& t) {
+int strip_occupancy_s(const BlockTuning& t, int depth) {
     const int W = t.TYg / t.R;
-    if (t.V == 1 && t.R == 2) return strip_occupancy_l<S, 1, 2>(t.L, W);
-    if (t.V == 1 && t.R == 4) return strip_occupancy_l<S, 1, 4>(t.L, W);
-    if (t.V == 2 && t.R == 2) return strip_occupancy_l<S, 2, 2>(t.L, W);
+    if (t.V == 1 && t.R == 2) return strip_occupancy_l<S, 1, 2>(t.L, W, depth);
+    if (t.V == 1 && t.R == 4) return strip_occupancy_l<S, 1, 4>(t.L, W, depth);
+    if (t.V == 2 && t.R == 2) return strip_occupancy_l<S, 2, 2>(t.L, W, depth);
     return 0;
 }
 
 int strip_occupancy(const fdtd_grid* g, const BlockTuning& t) {
+    const int depth = strip_stage_depth(t.L, t.V, t.R, t.TYg / t.R, g->Ni, g->precision);
     switch (g->precision) {
-        case FDTD_FP64: return strip_occupancy_s<double>(t);
-        case FDTD_FP32: return strip_occupancy_s<float>(t);
-        default: return strip_occupancy_s<_Float16>(t);
+        case FDTD_FP64: return strip_occupancy_s<double>(t, depth);
+        case FDTD_FP32: return strip_occupancy_s<float>(t, depth);
+        default: return strip_occupancy_s<_Float16>(t, depth);
     }
 }
 
