@@ -257,101 +257,41 @@ int launch_batch(fdtd_batch* b, bool steady, int parity, const double* vals_row)
 
 // ---- strip passes --------------------------------------------------------
 
-constexpr bool batch_strip_built(int csize, int V, int R) {
-    return (V == 1 || V == 2) && (R == 2 || R == 4) && V * R * csize <= 16;
-}
-
-template <typename S, int V, int R, int L, bool FINAL>
-const void* batch_strip_kernel(bool stage) {
-    using C = typename fdtd::ComputeOf<S>::type;
-    if constexpr (!batch_strip_built(sizeof(C), V, R)) {
-        return nullptr;
-    } else {
-        if constexpr (fdtd::strip_stage_built(V, R, L))
-            if (stage) return reinterpret_cast<const void*>(fdtd::batch_strip_sweep<S, C, V, R, L, FINAL, true>);
-        return reinterpret_cast<const void*>(fdtd::batch_strip_sweep<S, C, V, R, L, FINAL, false>);
-    }
-}
-
-template <typename S, int V, int R, int L, bool FINAL>
-int launch_batch_strip_v(fdtd_batch* b, int parity, const double* vals) {
-    using C = typename fdtd::ComputeOf<S>::type;
-    if constexpr (!batch_strip_built(sizeof(C), V, R)) {
-        return fail(FDTD_ERR_UNSUPPORTED, "strip variant V=%d R=%d not built", V, R);
-    } else {
-        fdtd::BatchStripArgs<S, C> a;
-        a.grids = static_cast<const fdtd::BatchStripGrid<S, C>*>(b->d_sgrids);
-        a.work = b->d_swork;
-        a.nwork = b->snwork;
-        a.parity = parity;
-        a.vals = vals;
-        a.vstride = b->total_src;
-        a.pad = 0;
-        auto kern = fdtd::batch_strip_sweep<S, C, V, R, L, FINAL, false>;
-        if constexpr (fdtd::strip_stage_built(V, R, L))
-            if (b->sdepth > 0) kern = fdtd::batch_strip_sweep<S, C, V, R, L, FINAL, true>;
-        hipLaunchKernelGGL(kern, dim3(b->snwork), dim3(64 * b->sW), b->slds, b->stream, a);
-        HIP_TRY(hipGetLastError());
-        return FDTD_OK;
-    }
-}
-
-template <typename S, int V, int R, bool FINAL>
-int launch_batch_strip_l(fdtd_batch* b, int parity, const double* vals) {
-    switch (b->sL) {
-        case 1: return launch_batch_strip_v<S, V, R, 1, FINAL>(b, parity, vals);
-        case 2: return launch_batch_strip_v<S, V, R, 2, FINAL>(b, parity, vals);
-        case 3: return launch_batch_strip_v<S, V, R, 3, FINAL>(b, parity, vals);
-        default: return launch_batch_strip_v<S, V, R, 4, FINAL>(b, parity, vals);
-    }
-}
-
-template <typename S, bool FINAL>
-int launch_batch_strip_s(fdtd_batch* b, int parity, const double* vals) {
-    if (b->sV == 1 && b->sR == 2) return launch_batch_strip_l<S, 1, 2, FINAL>(b, parity, vals);
-    if (b->sV == 1 && b->sR == 4) return launch_batch_strip_l<S, 1, 4, FINAL>(b, parity, vals);
-    return launch_batch_strip_l<S, 2, 2, FINAL>(b, parity, vals);
-}
-
-// One strip pass of sL steps over every grid; source values are the rows
-// starting at vals (null: no sources).
-int launch_batch_strip(fdtd_batch* b, bool final, int parity, const double* vals) {
-    switch (b->precision) {
-        case FDTD_FP64:
-            return final ? launch_batch_strip_s<double, true>(b, parity, vals)
-                         : launch_batch_strip_s<double, false>(b, parity, vals);
-        case FDTD_FP32:
-            return final ? launch_batch_strip_s<float, true>(b, parity, vals)
-                         : launch_batch_strip_s<float, false>(b, parity, vals);
-        default:
-            return final ? launch_batch_strip_s<_Float16, true>(b, parity, vals)
-                         : launch_batch_strip_s<_Float16, false>(b, parity, vals);
-    }
-}
-
-template <typename S, int V, int R>
-const void* strip_kernel_l(int L, bool final, bool stage) {
-    switch (L) {
-        case 1: return final ? batch_strip_kernel<S, V, R, 1, true>(stage) : batch_strip_kernel<S, V, R, 1, false>(stage);
-        case 2: return final ? batch_strip_kernel<S, V, R, 2, true>(stage) : batch_strip_kernel<S, V, R, 2, false>(stage);
-        case 3: return final ? batch_strip_kernel<S, V, R, 3, true>(stage) : batch_strip_kernel<S, V, R, 3, false>(stage);
-        default: return final ? batch_strip_kernel<S, V, R, 4, true>(stage) : batch_strip_kernel<S, V, R, 4, false>(stage);
+const void* strip_kernel(int precision, int V, int R, int L, bool final, bool stage, bool first) {
+    switch (precision) {
+        case FDTD_FP64: return batch_strip_kernel<double>(V, R, L, final, stage, first);
+        case FDTD_FP32: return batch_strip_kernel<float>(V, R, L, final, stage, first);
+        default: return batch_strip_kernel<_Float16>(V, R, L, final, stage, first);
     }
 }
 
 template <typename S>
-const void* strip_kernel_s(int V, int R, int L, bool final, bool stage) {
-    if (V == 1 && R == 2) return strip_kernel_l<S, 1, 2>(L, final, stage);
-    if (V == 1 && R == 4) return strip_kernel_l<S, 1, 4>(L, final, stage);
-    if (V == 2 && R == 2) return strip_kernel_l<S, 2, 2>(L, final, stage);
-    return nullptr;
+int launch_batch_strip_s(fdtd_batch* b, bool final, bool first, int parity, const double* vals) {
+    using C = typename fdtd::ComputeOf<S>::type;
+    fdtd::BatchStripArgs<S, C> a;
+    a.grids = static_cast<const fdtd::BatchStripGrid<S, C>*>(b->d_sgrids);
+    a.work = b->d_swork;
+    a.nwork = b->snwork;
+    a.parity = parity;
+    a.vals = vals;
+    a.vstride = b->total_src;
+    a.pad = 0;
+    const void* kern = batch_strip_kernel<S>(b->sV, b->sR, b->sL, final, b->sdepth > 0, first);
+    if (!kern) return fail(FDTD_ERR_UNSUPPORTED, "strip variant V=%d R=%d not built", b->sV, b->sR);
+    if (int rc = allow_dynamic_lds(kern, b->slds)) return rc;
+    void* args[] = {&a};
+    HIP_TRY(hipLaunchKernel(kern, dim3(b->snwork), dim3(64 * b->sW), args, b->slds, b->stream));
+    return FDTD_OK;
 }
 
-const void* strip_kernel(int precision, int V, int R, int L, bool final, bool stage) {
-    switch (precision) {
-        case FDTD_FP64: return strip_kernel_s<double>(V, R, L, final, stage);
-        case FDTD_FP32: return strip_kernel_s<float>(V, R, L, final, stage);
-        default: return strip_kernel_s<_Float16>(V, R, L, final, stage);
+// One strip pass of sL steps over every grid; source values are the rows
+// starting at vals (null: no sources).  first: with the run's first B half
+// step.
+int launch_batch_strip(fdtd_batch* b, bool final, bool first, int parity, const double* vals) {
+    switch (b->precision) {
+        case FDTD_FP64: return launch_batch_strip_s<double>(b, final, first, parity, vals);
+        case FDTD_FP32: return launch_batch_strip_s<float>(b, final, first, parity, vals);
+        default: return launch_batch_strip_s<_Float16>(b, final, first, parity, vals);
     }
 }
 
@@ -366,7 +306,7 @@ const void* strip_kernel(int precision, int V, int R, int L, bool final, bool st
 // also has costs outside the model (descriptor loads, the queue, ramp-up).
 int apply_strips(fdtd_batch* b, int L, int V, int R, int W) {
     const int cs = (int)compute_size(b->precision);
-    if (L < 1 || L > 4 || !batch_strip_built(cs, V, R) || W < 1 || W > 16 ||
+    if (L < 1 || L > 4 || !strip_built(cs, V, R) || W < 1 || W > 16 ||
         64 * W > fdtd::strip_max_threads(V, R, L, cs))
         return fail(FDTD_ERR_INVALID_ARGUMENT, "strip blocking L=%d V=%d R=%d W=%d not available",
                     L, V, R, W);
@@ -386,7 +326,7 @@ int apply_strips(fdtd_batch* b, int L, int V, int R, int W) {
     if (lds > kLdsLimit) return fail(FDTD_ERR_INVALID_ARGUMENT, "strip tiles need too much LDS");
     int per_cu = 0;
     for (bool final : {false, true}) {
-        const void* kern = strip_kernel(b->precision, V, R, L, final, depth > 0);
+        const void* kern = strip_kernel(b->precision, V, R, L, final, depth > 0, false);
         if (!kern) return fail(FDTD_ERR_UNSUPPORTED, "strip variant not built");
         if (int rc = allow_dynamic_lds(kern, lds)) return rc;
         if (!final) HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 64 * W, lds));
@@ -637,11 +577,15 @@ int prologue_B(fdtd_batch* b) {
 // step_dev is non-null, from the device counter, which is advanced at the
 // end (graph replays then continue in time).
 int enqueue_steps(fdtd_batch* b, int nsteps, long long step0, bool device_step, int* swaps) {
-    if (int rc = prologue_B(b)) return rc;
     // strip passes of sL steps first (when set and the run is long enough),
-    // then the remaining steps as single sweeps; every launch swaps buffers
+    // then the remaining steps as single sweeps; every launch swaps buffers.
+    // Passes that stage two planes in LDS take the first B half step
+    // themselves.
     const int L = b->sL;
     const int npass = L > 0 ? nsteps / L : 0;
+    const bool own_half = npass > 0 && b->sdepth == 2;
+    if (!own_half)
+        if (int rc = prologue_B(b)) return rc;
     const int rem = nsteps - npass * L;
     int parity = 0;
     int s = 0;
@@ -663,7 +607,7 @@ int enqueue_steps(fdtd_batch* b, int nsteps, long long step0, bool device_step, 
         }
         const double* vals = b->total_src > 0 ? b->d_vals + (size_t)(s % pchunk) * b->total_src
                                               : nullptr;
-        if (int rc = launch_batch_strip(b, rem == 0 && p + 1 == npass, parity, vals)) return rc;
+        if (int rc = launch_batch_strip(b, rem == 0 && p + 1 == npass, own_half && p == 0, parity, vals)) return rc;
         parity ^= 1;
     }
     for (int q = 0; q < rem; ++q, ++s) {

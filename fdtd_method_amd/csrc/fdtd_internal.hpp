@@ -295,4 +295,26 @@ int flush_sources(fdtd_grid* g);
 int plain_B(fdtd_grid* g, bool layer = true);
 int zero_fill(void* p, size_t bytes, hipStream_t s);
 
+// Strip variants built: cells per lane V*R with V*R*sizeof(C) <= 16 bytes
+// (FP32/FP16: V=1 R=2, V=1 R=4, V=2 R=2; FP64: V=1 R=2).
+constexpr bool strip_built(int csize, int V, int R) {
+    return (V == 1 || V == 2) && (R == 2 || R == 4) && V * R * csize <= 16;
+}
+
+fdtd::StripGeom make_strip_geom(const fdtd_grid* g, const BlockTuning& t);
+// Probes are recorded by the stepping entry points only.
+bool probing(const fdtd_grid* g);
+fdtd::ProbeArgs probe_args(const fdtd_grid* g);
+
+// One strip pass of btune.L steps on the grid's stream (fdtd_strips.hpp).
+template <typename S>
+int launch_strip(fdtd_grid* g, bool final, bool first, int slot, int in, int out, void* const* in_b,
+                 void* const* ahead);
+// Workgroups of a strip shape resident per CU (0 if it cannot launch).
+template <typename S>
+int strip_occupancy_s(const BlockTuning& t, int depth);
+// The batched strip kernel of a shape (null: not built).
+template <typename S>
+const void* batch_strip_kernel(int V, int R, int L, bool final, bool stage, bool first);
+
 }  // namespace fdtd::rt

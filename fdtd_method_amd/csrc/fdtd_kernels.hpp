@@ -2077,13 +2077,20 @@ __device__ __forceinline__ void load_to_lds(gptr<T> base, unsigned off, unsigned
 // bursts between the levels' barriers, the 12 + 12 accesses kept the
 // wavefronts waiting for the memory pipe's queue.  Needs rows that are
 // whole 16-byte packs (Ni, TX) at pack-aligned window starts.
+// FIRST (staged path, two planes in LDS): the pass that starts from (E_n,
+// B_n) and takes the run's first B half step, (B_n + d), on the planes it
+// reads, instead of a sweep over E and B in front of the pass (512^3 FP32:
+// 0.93 ms, 4.8 GB).  Plane kk then needs E of plane kk+1, which is staged,
+// and one E column and row past the tile's high edges, which the edge lanes
+// and the last row group read from memory themselves.
 // RESCALE (FP16 storage only): the pass after an in-run rescaling decision,
 // which scales what it reads.
-template <typename S, typename C, int V, int R, int L, bool FINAL, bool STAGE,
+template <typename S, typename C, int V, int R, int L, bool FINAL, bool STAGE, bool FIRST = false,
           bool RESCALE = false, bool PROBE = false>
 __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int tile,
                                            C* __restrict__ lds) {
     static_assert(!STAGE || strip_stage_built(V, R, L), "staged shape");
+    static_assert(!FIRST || (STAGE && !RESCALE), "first passes are staged and rescale nothing");
     const StripGeom& G = a.g;
     const int txy = G.ntx * G.nty;
     const int chunk = tile / txy;
@@ -2161,6 +2168,7 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
     const Coefs<C> c = a.c;
     const cptr<int> kst = as_const(a.kstart);
     const int kfirst = k0 - L + 1, klast = k1 + L - 1;
+    const int kload = FIRST ? klast + 1 : klast;  // the last plane read
 
     // ---- staged planes: input per RL rows [component][row][RW] (components
     // Ex Ey Ez Bx By Bz), output [stored row][component][RW - 8]
@@ -2188,7 +2196,7 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
                cx0 * static_cast<int>(sizeof(S));
     };
     using lds_s = const __attribute__((address_space(3))) S*;
-    const lds_b in_own = stage_row(w), in_prev = stage_row(wm);
+    const lds_b in_own = stage_row(w), in_prev = stage_row(wm), in_next = stage_row(wp);
     const lds_b out_own = out0 + (w * R - L) * (6 * OB) + (cx0 - G.Gx) * static_cast<int>(sizeof(S));
     const S* ldp[NQ];          // component of each load (uniform)
     unsigned ld_off = 0;       // this lane's byte offset in a plane
@@ -2202,7 +2210,8 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
         const int row = lane64 * LB / RB, col = lane64 * LB % RB / static_cast<int>(sizeof(S));
         ld_off = static_cast<unsigned>(wrap_mod(py0 - L + wave / WL * RL + row, Nj) * Ni +
                                        wrap_mod(px0 - G.Gx + col, Ni)) * static_cast<unsigned>(sizeof(S));
-        ld_ok = col + LB / static_cast<int>(sizeof(S)) > G.Gx - L && col < G.Gx + G.TX + L;
+        ld_ok = col + LB / static_cast<int>(sizeof(S)) > G.Gx - L &&
+                col < G.Gx + G.TX + L + (FIRST ? 1 : 0);
         static_assert(WL <= 2, "E by even, B by odd wavefronts");
 #pragma unroll
         for (int q = 0; q < NQ; ++q)
@@ -2332,6 +2341,17 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
                 }
 
     C en[3][R][V], bn[3][R][V];
+    // b + d of row r (V = 1), the update of plain_update_B: E of the cell and
+    // its neighbours k+1 (kp), j+1 (jp) and i+1 (ip)
+    auto half_step = [&](C (&b)[3][R][V], int r, const C (&e)[3], C ex_kp, C ey_kp, C ex_jp, C ez_jp,
+                         C ey_ip, C ez_ip) {
+        const C dbx = sub_mul(c.bx_ey * (ey_kp - e[1]), c.bx_ez, ez_jp - e[2]);
+        const C dby = sub_mul(c.by_ez * (ez_ip - e[2]), c.by_ex, ex_kp - e[0]);
+        const C dbz = sub_mul(c.bz_ex * (ex_jp - e[0]), c.bz_ey, ey_ip - e[1]);
+        b[0][r][0] = as_stored<S>(b[0][r][0] + dbx);
+        b[1][r][0] = as_stored<S>(b[1][r][0] + dby);
+        b[2][r][0] = as_stored<S>(b[2][r][0] + dbz);
+    };
     auto rescale_plane = [&]() {
         if constexpr (RESCALE) {
 #pragma unroll
@@ -2350,7 +2370,7 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
         const size_t off = static_cast<size_t>(wrap_mod(kfirst, Nk)) * plane;
         if constexpr (STAGE) {
             stage_load(kfirst);
-            if (depth == 2 && kfirst < klast) stage_load(kfirst + 1);
+            if (depth == 2 && kfirst < kload) stage_load(kfirst + 1);
         }
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
@@ -2376,6 +2396,20 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
                 for (int v = 0; v < V; ++v)
                     bP[0][d][r][v] = as_stored<S>(bP[0][d][r][v] * a.iscale[3 + d]);
         if constexpr (!STAGE) rescale_plane();
+    }
+    if constexpr (FIRST) {
+        // the half step of plane kfirst-1 (V = 1), from memory
+        const size_t off0 = static_cast<size_t>(wrap_mod(kfirst - 1, Nk)) * plane;
+        const size_t off1 = static_cast<size_t>(wrap_mod(kfirst, Nk)) * plane;
+        const int ip = wrap_mod(gi0 + 1, Ni);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const size_t at0 = off0 + gj[r] * Ni, at1 = off1 + gj[r] * Ni;
+            const size_t jp = off0 + wrap_mod(gj[r] + 1, Nj) * Ni + gi0;
+            const C e[3] = {C(a.in.e[0][at0 + gi0]), C(a.in.e[1][at0 + gi0]), C(a.in.e[2][at0 + gi0])};
+            half_step(bP[0], r, e, C(a.in.e[0][at1 + gi0]), C(a.in.e[1][at1 + gi0]), C(a.in.e[0][jp]),
+                      C(a.in.e[2][jp]), C(a.in.e[1][at0 + ip]), C(a.in.e[2][at0 + ip]));
+        }
     }
     // level 0's E rows (read for ghost-plane results only)
 #pragma unroll
@@ -2440,7 +2474,7 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
         // the staged plane kk (each wavefront's own loads) has arrived; with
         // two planes staged, the NQ loads of plane kk+1 may be in flight
         if constexpr (STAGE) {
-            if (depth == 2 && more)
+            if (depth == 2 && more && !FIRST)
                 __builtin_amdgcn_s_waitcnt(0x0F70 | NQ);
             else
                 wait_vmem_all();
@@ -2457,8 +2491,44 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
                     en[d][r][0] = static_cast<C>(*(lds_s)(in_own + sat + d * (WL * CB) + r * RB));
                     bn[d][r][0] = static_cast<C>(*(lds_s)(in_own + sat + (3 + d) * (WL * CB) + r * RB));
                 }
+            if constexpr (FIRST) {
+                // E of plane kk+1, of row j+1 (the next group's first row; past
+                // the tile for the last group) and of column i+1 (past the tile
+                // for the edge lane)
+                const int sat1 = stage_at(kk + 1);
+                const size_t off = static_cast<size_t>(wrap_mod(kk, Nk)) * plane;
+                C ex_jp, ez_jp;
+                if (w + 1 < ngroups) {
+                    ex_jp = static_cast<C>(*(lds_s)(in_next + sat));
+                    ez_jp = static_cast<C>(*(lds_s)(in_next + sat + 2 * (WL * CB)));
+                } else {
+                    const size_t jp = off + wrap_mod(gj[R - 1] + 1, Nj) * Ni + gi0;
+                    ex_jp = C(a.in.e[0][jp]);
+                    ez_jp = C(a.in.e[2][jp]);
+                }
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
+                for (int r = 0; r < R; ++r) {
+                    C ey_ip = lane_next(en[1][r][0]), ez_ip = lane_next(en[2][r][0]);
+                    if (cx0 == RW - 1) {
+                        const size_t ip = off + gj[r] * Ni + wrap_mod(gi0 + 1, Ni);
+                        ey_ip = C(a.in.e[1][ip]);
+                        ez_ip = C(a.in.e[2][ip]);
+                    }
+                    const C e[3] = {en[0][r][0], en[1][r][0], en[2][r][0]};
+                    half_step(bn, r, e, static_cast<C>(*(lds_s)(in_own + sat1 + r * RB)),
+                              static_cast<C>(*(lds_s)(in_own + sat1 + WL * CB + r * RB)),
+                              r + 1 < R ? en[0][r + 1 < R ? r + 1 : r][0] : ex_jp,
+                              r + 1 < R ? en[2][r + 1 < R ? r + 1 : r][0] : ez_jp, ey_ip, ez_ip);
+                }
+                // level 0's B rows through the exchange, behind a barrier
+                sB(0, 0, w)[0] = bn[0][R - 1][0];
+                sB(0, 1, w)[0] = bn[2][R - 1][0];
+                __syncthreads();
+                b_prev[0][0] = sB(0, 0, wm)[0];
+                b_prev[1][0] = sB(0, 1, wm)[0];
+            }
+#pragma unroll
+            for (int q = 0; q < (FIRST ? 0 : 2); ++q) {
                 b_prev[q][0] = static_cast<C>(*(lds_s)(in_prev + sat + (3 + 2 * q) * (WL * CB) + (R - 1) * RB));
                 if constexpr (RESCALE)
                     b_prev[q][0] = as_stored<S>(b_prev[q][0] * a.iscale[3 + 2 * q]);
@@ -2630,7 +2700,7 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
                 __syncthreads();
                 // every wavefront has read the staged plane kk: another may
                 // take its place
-                if (STAGE && l == 0 && kk + depth <= klast) stage_load(kk + depth);
+                if (STAGE && l == 0 && kk + depth <= kload) stage_load(kk + depth);
             }
         }
         // stores of the last level: E_{L-1} at plane kk-L+1, B_{L-1} at kk-L
@@ -2758,7 +2828,8 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
             }
         }
     };
-    constexpr int UNR = STAGE && !PROBE ? 2 : 1;
+    // (not in the variants whose second set would spill)
+    constexpr int UNR = STAGE && !PROBE && !FIRST ? 2 : 1;
     for (int kk = kfirst;;) {
         bool done = false;
 #pragma unroll
@@ -2780,14 +2851,15 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
 // PROBE: the variant that records StripArgs::probe after each level (the
 // level's B is held in registers until then: up to 35 more VGPRs, which the
 // plain variant does without).
-template <typename S, typename C, int V, int R, int L, bool FINAL, bool STAGE, bool PROBE = false>
+template <typename S, typename C, int V, int R, int L, bool FINAL, bool STAGE, bool FIRST,
+          bool PROBE = false>
 __global__ void __launch_bounds__(strip_max_threads(V, R, L, sizeof(C)))
 strip_sweep(StripArgs<S, C> a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const int blk = blockIdx.x;
     const int tile = (blk & 7) * a.g.per_xcd + (blk >> 3);
     if (tile >= a.g.ntiles) return;  // whole workgroup
-    strip_tile<S, C, V, R, L, FINAL, STAGE, false, PROBE>(a, tile, reinterpret_cast<C*>(lds_raw));
+    strip_tile<S, C, V, R, L, FINAL, STAGE, FIRST, false, PROBE>(a, tile, reinterpret_cast<C*>(lds_raw));
 }
 
 // FP16 storage: the strip pass after an in-run rescaling decision, reading
@@ -2800,7 +2872,7 @@ strip_rescale_sweep(StripArgs<S, C> a) {
     const int blk = blockIdx.x;
     const int tile = (blk & 7) * a.g.per_xcd + (blk >> 3);
     if (tile >= a.g.ntiles) return;  // whole workgroup
-    strip_tile<S, C, V, R, L, FINAL, STAGE, true, PROBE>(a, tile, reinterpret_cast<C*>(lds_raw));
+    strip_tile<S, C, V, R, L, FINAL, STAGE, false, true, PROBE>(a, tile, reinterpret_cast<C*>(lds_raw));
 }
 
 // ---------------------------------------------------------------------------
@@ -2976,7 +3048,7 @@ __device__ __forceinline__ StripArgs<S, C> load_batch_strip_grid(cptr<BatchStrip
     return a;
 }
 
-template <typename S, typename C, int V, int R, int L, bool FINAL, bool STAGE>
+template <typename S, typename C, int V, int R, int L, bool FINAL, bool STAGE, bool FIRST>
 __global__ void __launch_bounds__(strip_max_threads(V, R, L, sizeof(C)))
 batch_strip_sweep(BatchStripArgs<S, C> a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -2984,7 +3056,7 @@ batch_strip_sweep(BatchStripArgs<S, C> a) {
     const int grid = work[2 * blockIdx.x], tile = work[2 * blockIdx.x + 1];
     const StripArgs<S, C> sa = load_batch_strip_grid<S, C>(as_const(a.grids) + grid, a.parity,
                                                            a.vals, a.vstride);
-    strip_tile<S, C, V, R, L, FINAL, STAGE>(sa, tile, reinterpret_cast<C*>(lds_raw));
+    strip_tile<S, C, V, R, L, FINAL, STAGE, FIRST>(sa, tile, reinterpret_cast<C*>(lds_raw));
 }
 
 // B half step of grid q of a batch, reading its current buffers (buf[0])

@@ -330,12 +330,6 @@ fdtd::StripGeom make_strip_geom(const fdtd_grid* g, const BlockTuning& t) {
     return G;
 }
 
-// Strip variants built: cells per lane V*R with V*R*sizeof(C) <= 16 bytes
-// (FP32/FP16: V=1 R=2, V=1 R=4, V=2 R=2; FP64: V=1 R=2).
-constexpr bool strip_built(int csize, int V, int R) {
-    return (V == 1 || V == 2) && (R == 2 || R == 4) && V * R * csize <= 16;
-}
-
 bool strip_valid(const fdtd_grid* g, const BlockTuning& t) {
     const int cs = (int)compute_size(g->precision);
     if (t.L < 1 || t.L > 4 || !strip_built(cs, t.V, t.R)) return false;
@@ -823,95 +817,6 @@ int launch_blocked_v(fdtd_grid* g, int slot, int in, int out) {
     return FDTD_OK;
 }
 
-// The strip kernel of a launch (STAGE: planes through LDS).  FP16: the pass
-// after an in-run rescaling decision scales its reads; passes of a run with
-// probes record them.
-template <typename S, int V, int R, int L, bool FINAL, bool STAGE>
-auto strip_kernel(bool rescale, bool probe) {
-    using C = typename fdtd::ComputeOf<S>::type;
-    auto kern = probe ? fdtd::strip_sweep<S, C, V, R, L, FINAL, STAGE, true>
-                      : fdtd::strip_sweep<S, C, V, R, L, FINAL, STAGE, false>;
-    if constexpr (sizeof(S) == 2)
-        if (rescale)
-            kern = probe ? fdtd::strip_rescale_sweep<S, C, V, R, L, FINAL, STAGE, true>
-                         : fdtd::strip_rescale_sweep<S, C, V, R, L, FINAL, STAGE, false>;
-    return kern;
-}
-
-template <typename S, int V, int R, int L, bool FINAL>
-int launch_strip_v(fdtd_grid* g, int slot, int in, int out, void* const* in_b, void* const* ahead) {
-    using C = typename fdtd::ComputeOf<S>::type;
-    if constexpr (!strip_built(sizeof(C), V, R)) {
-        return fail(FDTD_ERR_UNSUPPORTED, "strip variant V=%d R=%d not built", V, R);
-    } else {
-        const BlockTuning& t = g->btune;
-        fdtd::StripArgs<S, C> a;
-        a.in = fields_of<S>(g, in);
-        if (in_b)
-            for (int d = 0; d < 3; ++d) a.in.b[d] = static_cast<S*>(in_b[d]);
-        a.out = fields_of<S>(g, out);
-        for (int d = 0; d < 3; ++d) a.ahead[d] = ahead ? static_cast<S*>(ahead[d]) : nullptr;
-        a.src = g->d_src;
-        a.kstart = g->d_kstart;
-        a.vals = g->d_vals ? g->d_vals + (size_t)slot * g->nsrc : nullptr;
-        a.nsrc = g->nsrc;
-        a.vstride = g->nsrc;
-        a.c = make_coefs<C>(g);
-        a.g = make_strip_geom(g, t);
-        for (int c = 0; c < 6; ++c) a.iscale[c] = g->pass_iscale[c];
-        a.probe = probe_args(g);
-        auto kern = strip_kernel<S, V, R, L, FINAL, false>(g->pass_rescale, probing(g));
-        if constexpr (fdtd::strip_stage_built(V, R, L))
-            if (a.g.depth > 0) kern = strip_kernel<S, V, R, L, FINAL, true>(g->pass_rescale, probing(g));
-        const size_t lds = fdtd::strip_lds_bytes(L, a.g.W, V, R, sizeof(C), sizeof(S), a.g.depth);
-        if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
-        hipLaunchKernelGGL(kern, dim3(8 * a.g.per_xcd), dim3(64 * a.g.W), lds, g->stream, a);
-        HIP_TRY(hipGetLastError());
-        if (a.probe.n > 0) g->probe_rows += L;
-        return FDTD_OK;
-    }
-}
-
-// Workgroups of a strip variant resident per CU (0 if it cannot launch).
-template <typename S, int V, int R, int L>
-int strip_occupancy_v(int W, int depth) {
-    using C = typename fdtd::ComputeOf<S>::type;
-    if constexpr (!strip_built(sizeof(C), V, R)) {
-        return 0;
-    } else {
-        auto kern = fdtd::strip_sweep<S, C, V, R, L, false, false>;
-        if constexpr (fdtd::strip_stage_built(V, R, L))
-            if (depth > 0) kern = fdtd::strip_sweep<S, C, V, R, L, false, true>;
-        const size_t lds = fdtd::strip_lds_bytes(L, W, V, R, sizeof(C), sizeof(S), depth);
-        if (allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds) != FDTD_OK) return 0;
-        int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, 64 * W, lds) != hipSuccess) {
-            (void)hipGetLastError();
-            return 0;
-        }
-        return n;
-    }
-}
-
-template <typename S, int V, int R>
-int strip_occupancy_l(int L, int W, int depth) {
-    switch (L) {
-        case 1: return strip_occupancy_v<S, V, R, 1>(W, depth);
-        case 2: return strip_occupancy_v<S, V, R, 2>(W, depth);
-        case 3: return strip_occupancy_v<S, V, R, 3>(W, depth);
-        default: return strip_occupancy_v<S, V, R, 4>(W, depth);
-    }
-}
-
-template <typename S>
-int strip_occupancy_s(const BlockTuning& t, int depth) {
-    const int W = t.TYg / t.R;
-    if (t.V == 1 && t.R == 2) return strip_occupancy_l<S, 1, 2>(t.L, W, depth);
-    if (t.V == 1 && t.R == 4) return strip_occupancy_l<S, 1, 4>(t.L, W, depth);
-    if (t.V == 2 && t.R == 2) return strip_occupancy_l<S, 2, 2>(t.L, W, depth);
-    return 0;
-}
-
 int strip_occupancy(const fdtd_grid* g, const BlockTuning& t) {
     const int depth = strip_stage_depth(t.L, t.V, t.R, t.TYg / t.R, g->Ni, g->precision);
     switch (g->precision) {
@@ -1032,26 +937,6 @@ int strip_default_kchunk(const fdtd_grid* g, const BlockTuning& t) {
     return best;
 }
 
-template <typename S, int V, int R, bool FINAL>
-int launch_strip_l(fdtd_grid* g, int slot, int in, int out, void* const* in_b, void* const* ahead) {
-    switch (g->btune.L) {
-        case 1: return launch_strip_v<S, V, R, 1, FINAL>(g, slot, in, out, in_b, ahead);
-        case 2: return launch_strip_v<S, V, R, 2, FINAL>(g, slot, in, out, in_b, ahead);
-        case 3: return launch_strip_v<S, V, R, 3, FINAL>(g, slot, in, out, in_b, ahead);
-        case 4: return launch_strip_v<S, V, R, 4, FINAL>(g, slot, in, out, in_b, ahead);
-        default: return fail(FDTD_ERR_UNSUPPORTED, "unsupported blocking depth %d", g->btune.L);
-    }
-}
-
-template <typename S, bool FINAL>
-int launch_strip_s(fdtd_grid* g, int slot, int in, int out, void* const* in_b, void* const* ahead) {
-    const int V = g->btune.V, R = g->btune.R;
-    if (V == 1 && R == 2) return launch_strip_l<S, 1, 2, FINAL>(g, slot, in, out, in_b, ahead);
-    if (V == 1 && R == 4) return launch_strip_l<S, 1, 4, FINAL>(g, slot, in, out, in_b, ahead);
-    if (V == 2 && R == 2) return launch_strip_l<S, 2, 2, FINAL>(g, slot, in, out, in_b, ahead);
-    return fail(FDTD_ERR_UNSUPPORTED, "unsupported strip shape V=%d R=%d", V, R);
-}
-
 template <typename S, int V, bool FINAL>
 int launch_blocked_l(fdtd_grid* g, int slot, int in, int out) {
     switch (g->btune.L) {
@@ -1064,9 +949,9 @@ int launch_blocked_l(fdtd_grid* g, int slot, int in, int out) {
 }
 
 template <typename S, bool FINAL>
-int launch_blocked_s(fdtd_grid* g, int slot, int in, int out, void* const* in_b,
-                     void* const* ahead) {
-    if (g->btune.R > 0) return launch_strip_s<S, FINAL>(g, slot, in, out, in_b, ahead);
+int launch_blocked_s(fdtd_grid* g, int slot, int in, int out, void* const* in_b, void* const* ahead,
+                     bool first) {
+    if (g->btune.R > 0) return launch_strip<S>(g, FINAL, first, slot, in, out, in_b, ahead);
     switch (g->btune.V) {
         case 1: return launch_blocked_l<S, 1, FINAL>(g, slot, in, out);
         case 2: return launch_blocked_l<S, 2, FINAL>(g, slot, in, out);
@@ -1076,20 +961,21 @@ int launch_blocked_s(fdtd_grid* g, int slot, int in, int out, void* const* in_b,
 
 // One pass of btune.L fused steps; its source values are rows slot ..
 // slot+L-1 of the value table.  Strip passes may read their B input from
-// in_b (a carried half step) and, when final, also store the next half step
-// to ahead; the patch kernel takes neither.
+// in_b (a carried half step) or take the run's first half step themselves
+// (first) and, when final, also store the next half step to ahead; the patch
+// kernel does none of it.
 int launch_blocked(fdtd_grid* g, bool final, int slot, int in, int out,
-                   void* const* in_b = nullptr, void* const* ahead = nullptr) {
+                   void* const* in_b = nullptr, void* const* ahead = nullptr, bool first = false) {
     switch (g->precision) {
         case FDTD_FP64:
-            return final ? launch_blocked_s<double, true>(g, slot, in, out, in_b, ahead)
-                         : launch_blocked_s<double, false>(g, slot, in, out, in_b, ahead);
+            return final ? launch_blocked_s<double, true>(g, slot, in, out, in_b, ahead, first)
+                         : launch_blocked_s<double, false>(g, slot, in, out, in_b, ahead, first);
         case FDTD_FP32:
-            return final ? launch_blocked_s<float, true>(g, slot, in, out, in_b, ahead)
-                         : launch_blocked_s<float, false>(g, slot, in, out, in_b, ahead);
+            return final ? launch_blocked_s<float, true>(g, slot, in, out, in_b, ahead, first)
+                         : launch_blocked_s<float, false>(g, slot, in, out, in_b, ahead, first);
         default:
-            return final ? launch_blocked_s<_Float16, true>(g, slot, in, out, in_b, ahead)
-                         : launch_blocked_s<_Float16, false>(g, slot, in, out, in_b, ahead);
+            return final ? launch_blocked_s<_Float16, true>(g, slot, in, out, in_b, ahead, first)
+                         : launch_blocked_s<_Float16, false>(g, slot, in, out, in_b, ahead, first);
     }
 }
 
@@ -1138,21 +1024,28 @@ void trace_end(fdtd_grid* g, hipEvent_t a, int kind, bool pass) {
 // n steps with temporal blocking: B/2 (or, for strip passes, the carried
 // half step), then n / L blocked passes, then the remaining n % L steps as
 // single fused sweeps.  Source tables are filled in whole passes.  Strip
-// runs carry the next half step out of their last pass or sweep, as the
-// unblocked path does.
+// passes that stage two planes in LDS take B/2 in their first pass; for them
+// a carried half step is dearer than the half step itself (512^3 FP32: the
+// carry costs the last pass 0.31 ms and three fields, the half step costs the
+// first pass 0.1), so FP64 and FP32 runs leave none.  Others carry the next
+// half step out of their last pass or sweep, as the unblocked path does; so
+// does FP16, where the carried value (rounded once) is not the half step from
+// the stored B.
 int run_blocked(fdtd_grid* g, int nsteps, hipEvent_t mid) {
     const bool strips = g->btune.R > 0;
     const int carried = strips ? g->ba_cur : -1;
+    const bool own_half = strips && make_strip_geom(g, g->btune).depth == 2;
     g->ba_cur = -1;
     int rc = FDTD_OK;
-    if (carried < 0) {
+    if (carried < 0 && !own_half) {
         TraceRange tr("b_half_prologue");
         hipEvent_t t0 = trace_begin(g);
         rc = plain_B(g);
         trace_end(g, t0, 0, false);
     }
     if (rc) return rc;
-    const bool carry_out = strips && g->carry && ensure_carry(g);
+    const bool carry_out = strips && g->carry && (!own_half || g->precision == FDTD_FP16) &&
+                           ensure_carry(g);
     const int ahead_buf = carried < 0 ? 0 : 1 - carried;
     if (mid) HIP_TRY(hipEventRecord(mid, g->stream));
     const int L = g->btune.L;
@@ -1185,7 +1078,8 @@ int run_blocked(fdtd_grid* g, int nsteps, hipEvent_t mid) {
         void* const* ahead = last && carry_out ? g->BA[ahead_buf] : nullptr;
         TraceRange tr(strips ? "strip_pass" : "patch_pass");
         hipEvent_t t0 = trace_begin(g);
-        rc = launch_blocked(g, last, s % chunk, in, out, in_b, ahead);
+        rc = launch_blocked(g, last, s % chunk, in, out, in_b, ahead,
+                            own_half && p == 0 && carried < 0);
         trace_end(g, t0, last ? 2 : 1, true);
         g->pass_rescale = false;
         for (int c = 0; c < 6; ++c) g->pass_iscale[c] = 1.0f;

@@ -4,7 +4,8 @@ the direct path beside them (any other row length).
 Tile edges: rows of one pack, the last column of a tile and the first of the
 next, a tile short of a pack, rows shorter than a tile (the window wraps
 several times), one-plane grids, odd and even wavefront counts, z chunks of
-one plane, several calls (the carried half step) and sources in the first
+one plane, several calls (each call's first pass takes the B half step itself,
+and may be its last) and sources in the first
 and last cells of tiles.  Every run must equal unblocked single sweeps bit
 for bit, in E, B and the probes.
 """
@@ -61,8 +62,8 @@ def test_strip_planes_through_lds(prec, shape, L, W, kchunk):
     for probes in (False, True):
         for g in (a, b):
             if probes:
-                g.set_probes(cells, 3 * L + 1)
-        for n in (2 * L, L + 1):
+                g.set_probes(cells, 4 * L + 1)
+        for n in (2 * L, L + 1, L):
             a.update_fields(n)
             b.update_fields(n)
             assert a.checksum() == b.checksum(), (probes, n)
@@ -81,7 +82,7 @@ def test_batch_strips_through_lds(prec, sides):
     for g in a:
         g.set_time_blocking_strips(0)
         g.set_step_carry(False)  # a batch call starts from the B/2 prologue
-    for n in (8, 5):
+    for n in (8, 5, 4):
         for g in a:
             g.update_fields(n)
         batch.update_fields(n)
