@@ -320,6 +320,36 @@ __device__ __forceinline__ void add_point_sources(C (&t)[3][V], const Coefs<C>& 
     }
 }
 
+// Single-cell currents passed with the launch itself, for steps whose
+// sources are all values the host knows (sorted by plane, at most
+// kInlineSources): a one-step call is then one launch, with no upload of the
+// list and no value table in front of it.
+constexpr int kInlineSources = 32;
+struct InlineSource {
+    int i, j, k, comp;
+    double value;
+};
+
+// Adds the J terms of plane k's inline sources, as add_point_sources does.
+template <typename C, int V>
+__device__ __forceinline__ void add_inline_sources(C (&t)[3][V], const Coefs<C>& c,
+                                                   const InlineSource* src, int n, int ib, int j,
+                                                   int k) {
+    for (int q = 0; q < n; ++q) {
+        if (src[q].k != k) continue;
+        const int comp = src[q].comp, di = src[q].i - ib;
+        if (src[q].j != j || di < 0 || di >= V) continue;
+        const C val = C(src[q].value);
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            if (di != v) continue;
+            if (comp == 0) t[0][v] = c.jx * val + t[0][v];
+            if (comp == 1) t[1][v] = c.jy * val + t[1][v];
+            if (comp == 2) t[2][v] = c.jz * val + t[2][v];
+        }
+    }
+}
+
 // Probes: single field values recorded in FP64 after every step.  A probe
 // of E at plane k is listed under plane key k, one of B at plane k under key
 // k+1 (mod Nk): the sweep iteration (or strip level) that computes E at
@@ -680,6 +710,12 @@ struct SweepArgs {
     ProbeArgs probe;  // values after this sweep's step (n = 0: none)
 };
 
+// Arguments of the sweeps that bring their sources along (nsrc is 0).
+struct InlineArgs {
+    int n;
+    InlineSource src[kInlineSources];
+};
+
 // Lane -> pack (V cells) order within a row of a PML sweep: the packs that
 // hold lower-layer cells (i < pi), then those holding upper-layer cells
 // (i >= Ni - pi), then the rest, so that in main-box rows the layer cells
@@ -697,10 +733,11 @@ __device__ __forceinline__ int pml_pack(int lane, int npacks, int pi, int V) {
     return lane - nhi;
 }
 
+// INL: the launch's own sources are added (inl is null otherwise).
 template <typename S, typename C, typename JT, int V, bool STEADY, bool PML = false,
-          bool AUTO = false, bool PROBE = false>
+          bool AUTO = false, bool PROBE = false, bool INL = false>
 __device__ __forceinline__ void fused_tile(const SweepArgs<S, C, JT>& a, int tile_y, int chunk,
-                                           C* __restrict__ lds) {
+                                           C* __restrict__ lds, const InlineArgs* inl = nullptr) {
     static_assert(!(PML && PROBE), "PML sweeps record no probes");
     const int Ni = a.g.Ni, Nj = a.g.Nj, Nk = a.g.Nk, TY = a.g.TY;
     const int lanes = Ni / V;
@@ -813,6 +850,13 @@ __device__ __forceinline__ void fused_tile(const SweepArgs<S, C, JT>& a, int til
         }
         widen<S, C, V>(m0, bm);
     }
+    // whether one of the launch's own sources lies on this chunk's planes
+    bool inl_here = false;
+    if constexpr (INL)
+        for (int q = 0; q < inl->n; ++q) {
+            const int k = inl->src[q].k;
+            inl_here = inl_here || (k >= k0 && k <= k1) || (k == 0 && k1 == Nk);
+        }
 
     // PML sweeps: the split fields of iteration kn (E splits of its plane,
     // B splits of plane kn-1 for steady sweeps), for lanes holding layer
@@ -914,6 +958,8 @@ __device__ __forceinline__ void fused_tile(const SweepArgs<S, C, JT>& a, int til
                 }
                 add_point_sources<C, V>(t, c, a.src, a.vals, q0, q1, ib, j, kw);
             }
+            if constexpr (INL)
+                if (inl_here) add_inline_sources<C, V>(t, c, inl->src, inl->n, ib, j, kw);
 #pragma unroll
             for (int v = 0; v < V; ++v) {
                 e1[0][v] = en[0][v] + sub_mul(t[0][v], c.ex_by, bn[1][v] - bP[1][v]);
@@ -1135,6 +1181,22 @@ fused_sweep(SweepArgs<S, C, JT> a) {
     const int chunk = t / a.g.ntile_y;
     fused_tile<S, C, JT, V, STEADY, false, AUTO, PROBE>(a, tile_y, chunk,
                                                        reinterpret_cast<C*>(lds_raw));
+}
+
+// The fused sweep that brings its sources along: the sweeps of one-step calls
+// whose currents the host sets (a kernel of its own, since the larger
+// argument block makes every launch longer).
+template <typename S, typename C, typename JT, int V, bool STEADY>
+__global__ void __launch_bounds__(fused_max_threads(V, sizeof(C)))
+fused_inline_sweep(SweepArgs<S, C, JT> a, InlineArgs inl) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    const int b = blockIdx.x;
+    const int t = (b & 7) * a.g.per_xcd + (b >> 3);
+    if (t >= a.g.ntiles) return;
+    const int tile_y = t % a.g.ntile_y;
+    const int chunk = t / a.g.ntile_y;
+    fused_tile<S, C, JT, V, STEADY, false, false, false, true>(a, tile_y, chunk,
+                                                              reinterpret_cast<C*>(lds_raw), &inl);
 }
 
 // The fused sweep of a grid with a PML layer (same tiles and LDS staging;
@@ -2094,7 +2156,8 @@ __device__ __forceinline__ void load_to_lds(gptr<T> base, unsigned off, unsigned
 // FIRST (staged path, two planes in LDS): the pass that starts from (E_n,
 // B_n) and takes the run's first B half step, (B_n + d), on the planes it
 // reads, instead of a sweep over E and B in front of the pass (512^3 FP32:
-// 0.93 ms, 4.8 GB).  Plane kk then needs E of plane kk+1, which is staged,
+// 0.93 ms, 4.8 GB; it makes the pass 0.3 ms longer, FP64 0.9 where the sweep
+// took 1.8).  Plane kk then needs E of plane kk+1, which is staged,
 // and one E column and row past the tile's high edges, which the edge lanes
 // and the last row group read from memory themselves.
 // RESCALE (FP16 storage only): the pass after an in-run rescaling decision,
@@ -2249,12 +2312,14 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
             int cc;
             size_t off;
             const bool ok = target(i * 64 * G.W + threadIdx.x, 0, G.TY, 6, &cc, &off, &st_lds[i]);
-            S* p = a.out.e[0];
-            if (cc == 1) p = a.out.e[1];
-            if (cc == 2) p = a.out.e[2];
-            if (cc == 3) p = a.out.b[0];
-            if (cc == 4) p = a.out.b[1];
-            if (cc == 5) p = a.out.b[2];
+            // (uniform_gptr: a plain select would index the argument struct,
+            // which batches would then keep in scratch memory)
+            S* p = generic(uniform_gptr(a.out.e[0]));
+            if (cc == 1) p = generic(uniform_gptr(a.out.e[1]));
+            if (cc == 2) p = generic(uniform_gptr(a.out.e[2]));
+            if (cc == 3) p = generic(uniform_gptr(a.out.b[0]));
+            if (cc == 4) p = generic(uniform_gptr(a.out.b[1]));
+            if (cc == 5) p = generic(uniform_gptr(a.out.b[2]));
             st_lag[i] = ok ? (cc >= 3 ? 1 : 0) : (1 << 30);
             stp[i] = reinterpret_cast<char*>(p) + off - (cc >= 3 ? pbytes64 : 0);
         }
@@ -2508,7 +2573,8 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
             if constexpr (FIRST) {
                 // E of plane kk+1, of row j+1 (the next group's first row; past
                 // the tile for the last group) and of column i+1 (past the tile
-                // for the edge lane)
+                // for the edge lane, unless the ghost band has a column to
+                // spare); loading the latter two a plane ahead changed nothing
                 const int sat1 = stage_at(kk + 1);
                 const size_t off = static_cast<size_t>(wrap_mod(kk, Nk)) * plane;
                 C ex_jp, ez_jp;
@@ -2523,7 +2589,7 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
                     C ey_ip = lane_next(en[1][r][0]), ez_ip = lane_next(en[2][r][0]);
-                    if (cx0 == RW - 1) {
+                    if (cx0 == RW - 1 && G.Gx + G.TX + L >= RW) {
                         const size_t ip = off + gj[r] * Ni + wrap_mod(gi0 + 1, Ni);
                         ey_ip = C(a.in.e[1][ip]);
                         ez_ip = C(a.in.e[2][ip]);

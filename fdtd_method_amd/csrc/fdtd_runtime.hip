@@ -261,6 +261,23 @@ int flush_sources(fdtd_grid* g) {
     return FDTD_OK;
 }
 
+// Whether the grid's sources are a few constants the sweeps can take with
+// their launch (all of them, sorted by plane): single-cell J values and no
+// waveform, on a periodic grid without probes or FP16 rescaling.  The
+// reference drivers' one-step calls then upload nothing (32^3 FP64, 24
+// values set before each step: 28 us per step, now 12).
+bool inline_sources(const fdtd_grid* g, std::vector<fdtd::InlineSource>* out) {
+    if (!g->waveforms.empty() || !g->jtab_keys.empty() || g->pml || g->nprobe > 0 ||
+        g->autoscale_interval > 0 || g->sparse_j.size() > (size_t)fdtd::kInlineSources)
+        return false;
+    out->clear();
+    for (const fdtd::PointSource& q : host_sources(g)) out->push_back({q.i, q.j, q.k, q.comp, q.amp});
+    std::stable_sort(out->begin(), out->end(), [](const fdtd::InlineSource& x, const fdtd::InlineSource& y) {
+        return x.k < y.k;
+    });
+    return true;
+}
+
 // J values of all point sources for steps step .. step+nsteps-1
 // (t = (n+1)*dt) into the value table, nsteps <= kValTable.
 int eval_sources(fdtd_grid* g, long long step, int nsteps) {
@@ -570,6 +587,7 @@ struct SweepExtra {
     unsigned* maxbits = nullptr;
     void* const* in_b = nullptr;
     void* const* ahead = nullptr;
+    const std::vector<fdtd::InlineSource>* inl = nullptr;  // instead of the source list
 };
 
 // Probes of the steps a run queues from here: the next row.
@@ -635,7 +653,23 @@ int launch_fused_a(fdtd_grid* g, const Tuning& t, int slot, int in, int out,
     for (int c = 0; c < 6; ++c) a.oscale[c] = C(x.oscale ? x.oscale[c] : 1.0);
     a.maxbits = x.maxbits;
     a.probe = PROBE ? probe_args(g) : fdtd::ProbeArgs{};
+    if (x.inl) {
+        a.nsrc = 0;
+        a.kstart = nullptr;
+    }
     const size_t lds = sweep_lds_bytes(g, t.TY);
+    if constexpr (!AUTO && !PROBE)
+        if (x.inl && !x.inl->empty()) {
+            auto ikern = fdtd::fused_inline_sweep<S, C, JT, V, STEADY>;
+            fdtd::InlineArgs inl;
+            inl.n = (int)x.inl->size();
+            std::copy(x.inl->begin(), x.inl->end(), inl.src);
+            if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(ikern), lds)) return rc;
+            hipLaunchKernelGGL(ikern, dim3(8 * a.g.per_xcd), dim3((t.TY + 1) * (g->Ni / V)), lds,
+                               g->stream, a, inl);
+            HIP_TRY(hipGetLastError());
+            return FDTD_OK;
+        }
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
     const int threads = (t.TY + 1) * (g->Ni / V);
     hipLaunchKernelGGL(kern, dim3(8 * a.g.per_xcd), dim3(threads), lds, g->stream, a);
@@ -1025,9 +1059,10 @@ void trace_end(fdtd_grid* g, hipEvent_t a, int kind, bool pass) {
 // half step), then n / L blocked passes, then the remaining n % L steps as
 // single fused sweeps.  Source tables are filled in whole passes.  Strip
 // passes that stage two planes in LDS take B/2 in their first pass; for them
-// a carried half step is dearer than the half step itself (512^3 FP32: the
-// carry costs the last pass 0.31 ms and three fields, the half step costs the
-// first pass 0.1), so FP64 and FP32 runs leave none.  Others carry the next
+// a carried half step is no cheaper than the half step itself (512^3 FP32:
+// either makes one pass 0.3 ms longer; the carry also holds three fields
+// twice and is lost whenever the caller touches E or B), so FP64 and FP32
+// runs leave none.  Others carry the next
 // half step out of their last pass or sweep, as the unblocked path does; so
 // does FP16, where the carried value (rounded once) is not the half step from
 // the stored B.
@@ -1035,8 +1070,9 @@ int run_blocked(fdtd_grid* g, int nsteps, hipEvent_t mid) {
     const bool strips = g->btune.R > 0;
     const int carried = strips ? g->ba_cur : -1;
     const bool own_half = strips && make_strip_geom(g, g->btune).depth == 2;
+    int rc = flush_sources(g);
+    if (rc) return rc;
     g->ba_cur = -1;
-    int rc = FDTD_OK;
     if (carried < 0 && !own_half) {
         TraceRange tr("b_half_prologue");
         hipEvent_t t0 = trace_begin(g);
@@ -1124,7 +1160,10 @@ int run_fused(fdtd_grid* g, int nsteps, hipEvent_t mid = nullptr) {
     // final sweep of the previous run computed (B_n + d) + d from the same
     // E_n); otherwise B/2 in place.
     const int carried = g->ba_cur;
-    int rc = FDTD_OK;
+    std::vector<fdtd::InlineSource> inl;
+    const bool use_inl = inline_sources(g, &inl);
+    int rc = use_inl ? FDTD_OK : flush_sources(g);
+    if (rc) return rc;
     if (carried < 0) {
         TraceRange tr("b_half_prologue");
         hipEvent_t t0 = trace_begin(g);
@@ -1156,7 +1195,7 @@ int run_fused(fdtd_grid* g, int nsteps, hipEvent_t mid = nullptr) {
         }
         if (track)
             if ((rc = zero_fill(g->d_max, 32, g->stream))) return rc;
-        if (s % kValTable == 0)
+        if (!use_inl && s % kValTable == 0)
             if ((rc = eval_sources(g, g->step + s, std::min(kValTable, nsteps - s)))) return rc;
         if (g->pml && g->pml_path == 1 && !decide && !track) {
             // the step as two in-place phase sweeps
@@ -1169,6 +1208,7 @@ int run_fused(fdtd_grid* g, int nsteps, hipEvent_t mid = nullptr) {
         }
         const int in = g->cur, out = 1 - g->cur;
         SweepExtra x;
+        x.inl = use_inl ? &inl : nullptr;
         x.oscale = decide ? f : nullptr;
         x.maxbits = track ? g->d_max : nullptr;
         if (s == 0 && carried >= 0) x.in_b = g->BA[carried];
@@ -1195,6 +1235,7 @@ int run_fused(fdtd_grid* g, int nsteps, hipEvent_t mid = nullptr) {
 }
 
 int run_3sweep(fdtd_grid* g, int nsteps) {
+    if (int rc = flush_sources(g)) return rc;
     g->ba_cur = -1;
     for (int s = 0; s < nsteps; ++s) {
         TraceRange tr("three_sweep_step");
@@ -1959,7 +2000,6 @@ int fdtd_set_point_sources(fdtd_grid* g, int n, const fdtd_point_source* src) {
 int fdtd_update_fields(fdtd_grid* g, int nsteps) {
     if (!g || nsteps < 0) return fail(FDTD_ERR_INVALID_ARGUMENT, "invalid argument");
     if (nsteps == 0) return FDTD_OK;
-    if (int rc = flush_sources(g)) return rc;
     g->stats[0] += nsteps;
     return run_steps(g, nsteps, false);
 }
@@ -2162,7 +2202,6 @@ int fdtd_get_stats(const fdtd_grid* g, long long out[4]) {
 int fdtd_update_fields_3sweep(fdtd_grid* g, int nsteps) {
     if (!g || nsteps < 0) return fail(FDTD_ERR_INVALID_ARGUMENT, "invalid argument");
     if (nsteps == 0) return FDTD_OK;
-    if (int rc = flush_sources(g)) return rc;
     return run_steps(g, nsteps, true);
 }
 
