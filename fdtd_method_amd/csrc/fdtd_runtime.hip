@@ -948,17 +948,20 @@ int device_cus() {
 // z chunk length of a strip pass: every tile costs kchunk + 2(L-1) planes
 // (the pipeline fills and drains over L-1 planes at each end), and the
 // tiles run in rounds of (resident workgroups per CU x CUs); the chunking
-// with the fewest plane-rounds wins (ties: fewer chunks).
-int strip_default_kchunk(const fdtd_grid* g, const BlockTuning& t) {
+// with the fewest plane-rounds wins (ties: fewer chunks).  A grid whose tiles
+// are few gets chunks of a few planes: a plane takes about 3 us however few
+// workgroups run, so 128^3 FP32 (18 tiles a plane) takes 10 planes, 16
+// plane-rounds, instead of 16 planes, 22 (65 us a pass).  planes, when set, is
+// the plane-rounds of the choice.
+int strip_default_kchunk(const fdtd_grid* g, const BlockTuning& t, long long* planes = nullptr) {
     BlockTuning u = t;
     u.kchunk = g->Nk;
     const fdtd::StripGeom G = make_strip_geom(g, u);
     const long long nxy = (long long)G.ntx * G.nty;
     const long long slots = (long long)std::max(1, strip_occupancy(g, t)) * device_cus();
-    const int maxchunks = std::max(1, g->Nk / 16);
     long long best_cost = -1;
     int best = g->Nk;
-    for (int nchunk = 1; nchunk <= maxchunks; ++nchunk) {
+    for (int nchunk = 1; nchunk <= g->Nk; ++nchunk) {
         const int kc = (g->Nk + nchunk - 1) / nchunk;
         const int nc = (g->Nk + kc - 1) / kc;
         const long long rounds = (nxy * nc + slots - 1) / slots;
@@ -968,7 +971,19 @@ int strip_default_kchunk(const fdtd_grid* g, const BlockTuning& t) {
             best = kc;
         }
     }
+    if (planes) *planes = best_cost;
     return best;
+}
+
+// Whether strip passes of t.L steps beat as many single sweeps on a grid, by
+// what both cost on grids that fit the caches: a plane-round of a pass about
+// 3.5 us (FP64 W = 8, FP32 W = 16), a sweep 6.5 us up to 26 MB of E and B read
+// and written, beyond that 5 us and its bytes at 4.8 TB/s (FP32 128^3 26 us,
+// 160^3 48; FP64 131x90x70 26, 200x151x97 65).
+bool strips_pay(const fdtd_grid* g, const BlockTuning& t, long long planes) {
+    const double mb = 12.0 * g->N * g->esize * 1e-6;
+    const double sweep = mb <= 26.0 ? 6.5 : 5.0 + mb / 4.8;
+    return 3.5 * planes < t.L * sweep;
 }
 
 template <typename S, int V, bool FINAL>
@@ -1056,8 +1071,13 @@ void trace_end(fdtd_grid* g, hipEvent_t a, int kind, bool pass) {
 }
 
 // n steps with temporal blocking: B/2 (or, for strip passes, the carried
-// half step), then n / L blocked passes, then the remaining n % L steps as
-// single fused sweeps.  Source tables are filled in whole passes.  Strip
+// half step), then n / L blocked passes, then the remaining n % L steps: two
+// or three as one strip pass of that many levels, one (or those after patch
+// passes) as single fused sweeps.  A strip pass takes about as long with fewer
+// levels, since memory bounds it, so it is the cheaper form from two steps on
+// (ms, pass against sweeps: 512^3 FP32, two steps 1.67 / 2.3, three 1.78 / 3.5;
+// FP64 3.3 / 5.3, 3.7 / 8.0; 251x190x131 FP32 0.099 / 0.173, 0.120 / 0.25).
+// Source tables are filled in whole passes.  Strip
 // passes that stage two planes in LDS take B/2 in their first pass; for them
 // a carried half step is no cheaper than the half step itself (512^3 FP32:
 // either makes one pass 0.3 ms longer; the carry also holds three fields
@@ -1085,11 +1105,18 @@ int run_blocked(fdtd_grid* g, int nsteps, hipEvent_t mid) {
     const int ahead_buf = carried < 0 ? 0 : 1 - carried;
     if (mid) HIP_TRY(hipEventRecord(mid, g->stream));
     const int L = g->btune.L;
-    const int npass = nsteps / L, rem = nsteps % L;
+    const int npass = nsteps / L;
+    BlockTuning tail = g->btune;  // the pass of the steps left over
+    tail.L = nsteps % L;
+    const bool use_tail = strips && tail.L >= 2 && strip_valid(g, tail);
+    const int rem = use_tail ? 0 : nsteps % L;
+    const int blocked = nsteps - rem;
     const int chunk = (kValTable / L) * L;
     int s = 0;
-    for (int p = 0; p < npass; ++p, s += L) {
-        if (g->autoscale_interval > 0 && s > 0 && (s / L) % std::max(1, g->autoscale_interval / L) == 0) {
+    for (int p = 0; s < blocked; ++p, s += L) {
+        const bool is_tail = p == npass;
+        if (!is_tail && g->autoscale_interval > 0 && s > 0 &&
+            (s / L) % std::max(1, g->autoscale_interval / L) == 0) {
             if (strips) {
                 // strip passes scale what they read (bit-identical to
                 // rescaling the current state in place first)
@@ -1107,23 +1134,26 @@ int run_blocked(fdtd_grid* g, int nsteps, hipEvent_t mid) {
             }
         }
         if (s % chunk == 0)
-            if ((rc = eval_sources(g, g->step + s, std::min(chunk, npass * L - s)))) return rc;
+            if ((rc = eval_sources(g, g->step + s, std::min(chunk, blocked - s)))) return rc;
         const int in = g->cur, out = 1 - g->cur;
-        const bool last = rem == 0 && p + 1 == npass;
+        const bool last = rem == 0 && s + L >= nsteps;
         void* const* in_b = p == 0 && carried >= 0 ? g->BA[carried] : nullptr;
         void* const* ahead = last && carry_out ? g->BA[ahead_buf] : nullptr;
         TraceRange tr(strips ? "strip_pass" : "patch_pass");
         hipEvent_t t0 = trace_begin(g);
+        const BlockTuning keep = g->btune;
+        if (is_tail) g->btune = tail;
         rc = launch_blocked(g, last, s % chunk, in, out, in_b, ahead,
                             own_half && p == 0 && carried < 0);
-        trace_end(g, t0, last ? 2 : 1, true);
+        g->btune = keep;
+        trace_end(g, t0, last ? 2 : 1, !is_tail);
         g->pass_rescale = false;
         for (int c = 0; c < 6; ++c) g->pass_iscale[c] = 1.0f;
         if (rc) return rc;
         g->cur = out;
     }
-    for (int q = 0; q < rem; ++q, ++s) {
-        if ((rc = eval_sources(g, g->step + s, 1))) return rc;
+    for (int q = 0; q < rem; ++q) {
+        if ((rc = eval_sources(g, g->step + blocked + q, 1))) return rc;
         const int in = g->cur, out = 1 - g->cur;
         SweepExtra x;
         if (q + 1 == rem && carry_out) x.ahead = g->BA[ahead_buf];
@@ -1559,12 +1589,15 @@ int create_grid(const fdtd_parameters* p, double dt, double pml_percent, int pre
         if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
             return cleanup(fail(FDTD_ERR_HIP, "hipEventCreate"));
     g->fused_ok = default_tuning(g, &g->tune);
-    // Periodic grids large enough to fill the device with strip tiles step
-    // in temporally blocked passes of 4 steps by default (bit-identical to
-    // single sweeps; FP16 with in-run rescaling to FP16 rounding), with the
-    // shape the autotuner picks at 512^3; fdtd_set_time_blocking_strips(grid,
-    // 0, ...) returns to single sweeps.
-    if (!g->pml && g->fused_ok && g->Ni >= 128 && g->Nj >= 64 && g->Nk >= 32) {
+    // Periodic grids large enough step in temporally blocked passes of 4 steps
+    // by default (bit-identical to single sweeps; FP16 with in-run rescaling to
+    // FP16 rounding), with the shape the autotuner picks at 512^3;
+    // fdtd_set_time_blocking_strips(grid, 0, ...) returns to single sweeps.
+    // Narrower grids do where the passes cost less (100^3 FP64: 16 plane-rounds
+    // against four sweeps of 25 us); FP16, whose rescaling points depend on the
+    // passes, does not.
+    const bool wide = g->Ni >= 128 && g->Nj >= 64 && g->Nk >= 32;
+    if (!g->pml && g->fused_ok && (wide || precision != FDTD_FP16)) {
         BlockTuning t;
         t.L = 4;
         t.V = 1;
@@ -1573,8 +1606,9 @@ int create_grid(const fdtd_parameters* p, double dt, double pml_percent, int pre
         t.TYg = (precision == FDTD_FP64 ? 8 : 16) * t.R;
         t.kchunk = 1;
         if (strip_valid(g, t)) {
-            t.kchunk = strip_default_kchunk(g, t);
-            g->btune = t;
+            long long planes = 0;
+            t.kchunk = strip_default_kchunk(g, t, &planes);
+            if (wide || strips_pay(g, t, planes)) g->btune = t;
         }
     }
     if (hipStreamSynchronize(g->stream) != hipSuccess)

@@ -212,8 +212,9 @@ int fdtd_update_fields_with_currents(fdtd_grid* grid, int nsteps, const int* cou
                                      const long long* index, const int* component,
                                      const double* value);
 
-/* Launch counters since creation: {steps, temporally blocked passes,
- * single-step sweeps, B half-step prologues}. */
+/* Launch counters since creation: {steps, temporally blocked passes of the
+ * grid's depth, single-step sweeps and shorter passes that take the steps left
+ * over, B half-step prologues}. */
 int fdtd_get_stats(const fdtd_grid* grid, long long out[4]);
 
 /* Probes: the FP64 values (physical units, as stored) of n single field
