@@ -18,7 +18,7 @@ LIB_NAME = "libfdtd_mi355x.so"
 LIB_PATH = os.path.join(PKG, LIB_NAME)
 
 HIP_SOURCES = ["fdtd_runtime.hip", "fdtd_batch.hip", "fdtd_strips_fp64.hip", "fdtd_strips_fp32.hip",
-               "fdtd_strips_fp16.hip"]
+               "fdtd_strips_fp16.hip", "fdtd_pml_strips.hip"]
 
 # -ffp-contract=off keeps every a*b+c unfused, as in the reference's CPU
 # build (no FMA): the FP64 path is then bit-identical to the reference.

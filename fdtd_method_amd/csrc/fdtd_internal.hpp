@@ -187,7 +187,13 @@ struct fdtd_grid {
     double pml_percent = 0;
     int pml_p[3] = {0, 0, 0};
     void* ES[2][6] = {};        // E splits Exy Exz Eyx Eyz Ezx Ezy, ping-pong with E
-    void* BS[6] = {};           // B splits Bxy Bxz Byx Byz Bzx Bzy, in place
+    // B splits Bxy Bxz Byx Byz Bzx Bzy: sweeps update BS[bs_cur] in place, strip
+    // passes write the other set (BS[1]: grids that run strip passes only)
+    void* BS[2][6] = {};
+    int bs_cur = 0;
+    void* split_slab = nullptr;  // ES and BS, split_stride bytes apart
+    size_t split_stride = 0;
+    int pml_strip_kchunk = 0;   // z chunk of a PML strip pass; 0: the grid runs none
     void* pml_tab = nullptr;    // per-axis decay/coefficient tables (compute type)
     // PML steps: 0 = the fused PML sweep (shape tune); 1 = the two in-place
     // phase sweeps (pml_e_phase, pml_b_phase) with launch shape ptune.  FP16
@@ -260,7 +266,7 @@ fdtd::Pml<S, C> make_pml(const fdtd_grid* g, int in, int out) {
     for (int q = 0; q < 6; ++q) {
         P.es_in[q] = static_cast<const S*>(g->ES[in][q]);
         P.es_out[q] = static_cast<S*>(g->ES[out][q]);
-        P.bs[q] = static_cast<S*>(g->BS[q]);
+        P.bs[q] = static_cast<S*>(g->BS[g->bs_cur][q]);
     }
     const C* t = static_cast<const C*>(g->pml_tab);
     P.tx = t;
@@ -286,6 +292,8 @@ int allow_dynamic_lds(const void* kernel, size_t bytes);
 int grid_blocks(size_t n);
 int max_threads(const fdtd_grid* g, int V);
 int default_kchunk(int Nj, int Nk, int TY);
+int strip_chunk(int Nk, long long nxy, long long slots, int L, long long* planes);
+int device_cus();
 // Sparse J values (as kind-0 sources) followed by the waveform sources.
 std::vector<fdtd::PointSource> host_sources(const fdtd_grid* g);
 // Uploads the grid's source list to its device copy when it changed.
@@ -313,6 +321,10 @@ int launch_strip(fdtd_grid* g, bool final, bool first, int slot, int in, int out
 // Workgroups of a strip shape resident per CU (0 if it cannot launch).
 template <typename S>
 int strip_occupancy_s(const BlockTuning& t, int depth);
+// Tiles of a PML strip pass, and one pass of two steps (fdtd_pml_strips.hpp):
+// from the current buffers to the others, which become the current ones.
+fdtd::StripGeom make_pml_strip_geom(const fdtd_grid* g, int kchunk);
+int launch_pml_strip(fdtd_grid* g, bool final, int slot);
 // The batched strip kernel of a shape (null: not built).
 template <typename S>
 const void* batch_strip_kernel(int V, int R, int L, bool final, bool stage, bool first);

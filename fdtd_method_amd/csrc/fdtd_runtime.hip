@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "fdtd_internal.hpp"
+#include "fdtd_pml_strips.hpp"
 
 namespace fdtd::rt {
 
@@ -452,6 +453,25 @@ int box_update(fdtd_grid* g, const fdtd::Box& box, bool e_step) {
     }
 }
 
+// Chunk of Nk planes with the fewest plane-rounds (planes, when set) for nxy
+// tiles a chunk and `slots` workgroups at a time (see strip_default_kchunk).
+int strip_chunk(int Nk, long long nxy, long long slots, int L, long long* planes) {
+    long long best_cost = -1;
+    int best = Nk;
+    for (int nchunk = 1; nchunk <= Nk; ++nchunk) {
+        const int kc = (Nk + nchunk - 1) / nchunk;
+        const int nc = (Nk + kc - 1) / kc;
+        const long long rounds = (nxy * nc + slots - 1) / slots;
+        const long long cost = rounds * (kc + 2 * (L - 1));
+        if (best_cost < 0 || cost < best_cost) {
+            best_cost = cost;
+            best = kc;
+        }
+    }
+    if (planes) *planes = best_cost;
+    return best;
+}
+
 // ---- PML layer ----------------------------------------------------------------
 
 // Layer width of an axis of n cells, src/FDTD/FDTD_PML.cpp:254-256.
@@ -513,17 +533,62 @@ int build_pml_tables(fdtd_grid* g) {
     return FDTD_OK;
 }
 
+// Tiles of a PML strip pass (fdtd_pml_strips.hpp).
+fdtd::StripGeom make_pml_strip_geom(const fdtd_grid* g, int kchunk) {
+    const int cs = (int)compute_size(g->precision);
+    fdtd::StripGeom G{};
+    G.Ni = g->Ni;
+    G.Nj = g->Nj;
+    G.Nk = g->Nk;
+    G.W = fdtd::kPmlStripW;
+    G.Gx = fdtd::pml_strip_ghost(cs);
+    G.TX = fdtd::pml_strip_columns(cs);
+    G.TY = fdtd::kPmlStripW * fdtd::kPmlStripR - 2 * fdtd::kPmlStripL;
+    G.kchunk = kchunk;
+    G.ntx = (g->Ni + G.TX - 1) / G.TX;
+    G.nty = (g->Nj + G.TY - 1) / G.TY;
+    G.ntiles = G.ntx * G.nty * ((g->Nk + kchunk - 1) / kchunk);
+    G.per_xcd = (G.ntiles + 7) / 8;
+    return G;
+}
+
+// z chunk of a PML grid's strip passes, the one with the fewest plane-rounds; 0
+// where two fused sweeps cost less.  A pass of few planes takes 7 us and 6.5 us
+// a plane-round, two sweeps 24 us up to 26 MB (24 words a cell), beyond that 22
+// us and 0.45 us a MB (us, pass against sweeps: FP64 64^3 45 / 43, 80^3 47 / 66,
+// 128^3 168 / 200; FP32 64^3 34 / 25, 80^3 38 / 48, 128^3 102 / 120).
+int pml_strip_chunk(const fdtd_grid* g) {
+    const unsigned long long pb = (unsigned long long)g->Ni * g->Nj * g->esize;
+    if (g->precision == FDTD_FP16 || pb >= (1ull << 31) || pb + g->split_stride >= (1ull << 32))
+        return 0;  // (32-bit offsets from a plane's start)
+    const int cs = (int)compute_size(g->precision);
+    const fdtd::StripGeom G = make_pml_strip_geom(g, g->Nk);
+    long long planes = 0;
+    int kc = strip_chunk(g->Nk, (long long)G.ntx * G.nty, fdtd::pml_strip_wgs(cs) * device_cus(),
+                         fdtd::kPmlStripL, &planes);
+    const double mb = 24e-6 * g->N * g->esize;
+    if (7.0 + 6.5 * planes > (mb <= 26.0 ? 24.0 : 22.0 + 0.45 * mb)) return 0;
+    while (fdtd::pml_strip_lds_bytes(cs, kc) * fdtd::pml_strip_wgs(cs) > kLdsLimit) kc = (kc + 1) / 2;  // (its z tables)
+    return kc;
+}
+
 // Storage of a PML grid's layer: split fields (zeroed) and tables.
 int alloc_pml(fdtd_grid* g) {
-    const size_t bytes = g->N * g->esize + 16;
-    for (int q = 0; q < 6; ++q) {
-        for (int b = 0; b < 2; ++b) {
-            HIP_TRY(hipMalloc(&g->ES[b][q], bytes));
-            if (int rc = zero_fill(g->ES[b][q], bytes, g->stream)) return rc;
-        }
-        HIP_TRY(hipMalloc(&g->BS[q], bytes));
-        if (int rc = zero_fill(g->BS[q], bytes, g->stream)) return rc;
+    g->split_stride = (g->N * g->esize + 16 + 255) / 256 * 256;
+    g->pml_strip_kchunk = pml_strip_chunk(g);
+    if (g->pml_strip_kchunk > 0 && hipMalloc(&g->split_slab, 24 * g->split_stride) != hipSuccess) {
+        (void)hipGetLastError();
+        g->split_slab = nullptr;
+        g->pml_strip_kchunk = 0;
     }
+    if (!g->split_slab) HIP_TRY(hipMalloc(&g->split_slab, 18 * g->split_stride));
+    const int nset = g->pml_strip_kchunk > 0 ? 2 : 1;
+    char* p = static_cast<char*>(g->split_slab);
+    for (int q = 0; q < 6; ++q) {
+        for (int b = 0; b < 2; ++b) g->ES[b][q] = p + (b * 6 + q) * g->split_stride;
+        for (int b = 0; b < nset; ++b) g->BS[b][q] = p + (12 + b * 6 + q) * g->split_stride;
+    }
+    if (int rc = zero_fill(p, (12 + 6 * nset) * g->split_stride, g->stream)) return rc;
     HIP_TRY(hipMalloc(&g->pml_tab, 5 * (size_t)(g->Ni + g->Nj + g->Nk) * compute_size(g->precision)));
     return build_pml_tables(g);
 }
@@ -531,7 +596,7 @@ int alloc_pml(fdtd_grid* g) {
 // Storage component (0..5) whose scale split q (0..5 E, 6..11 B) shares.
 int split_component(int q) { return q < 6 ? q / 2 : 3 + (q - 6) / 2; }
 
-void* split_ptr(fdtd_grid* g, int q) { return q < 6 ? g->ES[g->cur][q] : g->BS[q - 6]; }
+void* split_ptr(fdtd_grid* g, int q) { return q < 6 ? g->ES[g->cur][q] : g->BS[g->bs_cur][q - 6]; }
 
 void* field_ptr(fdtd_grid* g, int c);
 
@@ -959,20 +1024,7 @@ int strip_default_kchunk(const fdtd_grid* g, const BlockTuning& t, long long* pl
     const fdtd::StripGeom G = make_strip_geom(g, u);
     const long long nxy = (long long)G.ntx * G.nty;
     const long long slots = (long long)std::max(1, strip_occupancy(g, t)) * device_cus();
-    long long best_cost = -1;
-    int best = g->Nk;
-    for (int nchunk = 1; nchunk <= g->Nk; ++nchunk) {
-        const int kc = (g->Nk + nchunk - 1) / nchunk;
-        const int nc = (g->Nk + kc - 1) / kc;
-        const long long rounds = (nxy * nc + slots - 1) / slots;
-        const long long cost = rounds * (kc + 2 * (t.L - 1));
-        if (best_cost < 0 || cost < best_cost) {
-            best_cost = cost;
-            best = kc;
-        }
-    }
-    if (planes) *planes = best_cost;
-    return best;
+    return strip_chunk(g->Nk, nxy, slots, t.L, planes);
 }
 
 // Whether strip passes of t.L steps beat as many single sweeps on a grid, by
@@ -1169,6 +1221,28 @@ int run_blocked(fdtd_grid* g, int nsteps, hipEvent_t mid) {
     return FDTD_OK;
 }
 
+// The steps of a PML run after its first B update, two to a strip pass; of an
+// odd number the first as a fused sweep (its output is what a pass reads).
+int run_pml_strips(fdtd_grid* g, int nsteps) {
+    for (int s = 0; s < nsteps;) {
+        const bool pass = s > 0 || nsteps % 2 == 0;
+        const int odd = nsteps % 2, slot = (s - odd) % kValTable;
+        if (!pass || slot == 0)
+            if (int rc = eval_sources(g, g->step + s, pass ? std::min(kValTable, nsteps - s) : 1)) return rc;
+        TraceRange tr(pass ? "pml_strip_pass" : "fused_sweep");
+        hipEvent_t t0 = trace_begin(g);
+        const int in = g->cur;
+        const int rc = pass ? launch_pml_strip(g, s + 2 == nsteps, slot)
+                            : launch_fused(g, g->tune, true, 0, in, 1 - in, SweepExtra());
+        trace_end(g, t0, s + 2 == nsteps ? 2 : (pass ? 1 : 3), pass);
+        if (rc) return rc;
+        if (!pass) g->cur = 1 - in;
+        s += pass ? 2 : 1;
+    }
+    g->step += nsteps;
+    return FDTD_OK;
+}
+
 // n steps: B half step in place, then n fused sweeps between the buffers.
 // With FP16 autoscaling, the state between two sweeps, (E_n, B_{n+1/2}),
 // is rescaled by exact powers of two every autoscale_interval sweeps.
@@ -1205,6 +1279,8 @@ int run_fused(fdtd_grid* g, int nsteps, hipEvent_t mid = nullptr) {
     const int ahead_buf = carried < 0 ? 0 : 1 - carried;
     g->ba_cur = -1;
     if (mid) HIP_TRY(hipEventRecord(mid, g->stream));
+    if (g->pml && g->pml_path == 0 && g->pml_strip_kchunk > 0 && nsteps >= 2 && !g->j_dense_active)
+        return run_pml_strips(g, nsteps);
     const int iv = g->precision == FDTD_FP16 ? g->autoscale_interval : 0;
     for (int s = 0; s < nsteps; ++s) {
         const bool decide = iv > 0 && s > 0 && s % iv == 0 && s + 1 < nsteps;
@@ -1643,11 +1719,7 @@ int fdtd_destroy(fdtd_grid* g) {
             if (g->E[b][d]) (void)hipFree(g->E[b][d]);
             if (g->B[b][d]) (void)hipFree(g->B[b][d]);
         }
-    for (int q = 0; q < 6; ++q) {
-        for (int b = 0; b < 2; ++b)
-            if (g->ES[b][q]) (void)hipFree(g->ES[b][q]);
-        if (g->BS[q]) (void)hipFree(g->BS[q]);
-    }
+    if (g->split_slab) (void)hipFree(g->split_slab);
     if (g->pml_tab) (void)hipFree(g->pml_tab);
     for (int b = 0; b < 2; ++b)
         for (int d = 0; d < 3; ++d)
@@ -2492,7 +2564,7 @@ int apply_scales(fdtd_grid* g, const double s[6], bool current_only) {
                     for (int b = 0; b < 2; ++b)
                         if (!current_only || b == g->cur) scale(g->ES[b][q], f);
                 } else {
-                    scale(g->BS[q - 6], f);
+                    scale(g->BS[g->bs_cur][q - 6], f);
                 }
             }
         g->scales[c] = s[c];
@@ -2573,7 +2645,9 @@ int fdtd_zero_fields(fdtd_grid* g) {
         for (int q = 0; q < 6; ++q) {
             for (int b = 0; b < 2; ++b)
                 if (int rc = zero_fill(g->ES[b][q], bytes, g->stream)) return rc;
-            if (int rc = zero_fill(g->BS[q], bytes, g->stream)) return rc;
+            for (int b = 0; b < 2; ++b)
+                if (g->BS[b][q])
+                    if (int rc = zero_fill(g->BS[b][q], bytes, g->stream)) return rc;
         }
     if (g->j_device) {
         for (int d = 0; d < 3; ++d)

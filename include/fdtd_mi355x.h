@@ -104,7 +104,9 @@ int fdtd_create_pml(const fdtd_parameters* params, double dt, double pml_percent
                     fdtd_grid** out);
 /* How a PML grid's fused steps run (no counterpart in the reference, whose
  * step is FDTD_PML.cpp:343-365): path 0 (the default) as the single fused
- * PML sweep (shape: fdtd_set_tuning); path 1 as two in-place sweeps per
+ * PML sweep (shape: fdtd_set_tuning) or, on FP64 and FP32 grids of more than
+ * about 50 MB of state and with no dense J, two steps to a strip pass (same
+ * bits; 512^3 FP32 with a 0.2 layer 1.7 ms per step); path 1 as two in-place sweeps per
  * step, an E phase and a B phase, with V cells per lane, TY full rows per
  * workgroup and kchunk planes per z chunk (0: defaults; V*storage bytes at
  * most 16).  At 512^3 with a 0.2 layer the phases take 3.94 ms per FP32

@@ -1,0 +1,62 @@
+"""PML strip passes (two steps per read and write of the state): the same bits,
+splits included, as one-step calls, which take the fused sweep, on shapes
+around the tiles' edges."""
+import numpy as np
+import pytest
+
+from fdtd_method_amd import FDTD_PML, Parameters, Precision
+
+pytestmark = pytest.mark.gpu
+
+FP64, FP32 = Precision.FP64, Precision.FP32
+C = 3e10
+
+
+def make(shape, prec, percent):
+    dt = 0.5 / (C * np.sqrt(1.0 + 1.0 / 1.44 + 1.0 / 0.81))
+    g = FDTD_PML(Parameters(*shape, dx=1.0, dy=1.2, dz=0.9), dt, percent, prec)
+    rng = np.random.default_rng(9)
+    for c in range(6):
+        g.upload(c, rng.standard_normal(int(np.prod(shape))) * 1e-3)
+    g.set_point_sources([
+        dict(i=shape[0] // 2, j=shape[1] // 2, k=shape[2] // 2, comp=0, kind=0, amp=0.3 / dt),
+        dict(i=0, j=1, k=0, comp=1, kind=0, amp=0.2 / dt),          # in the layer: no effect
+        dict(i=shape[0] // 2 - 1, j=shape[1] // 2, k=shape[2] // 2 - 1, comp=2, kind=1,
+             amp=1e-3 / dt, period=9 * dt, t0=4 * dt, sigma=6 * dt)])
+    return g
+
+
+@pytest.mark.parametrize("prec,shape,percent", [
+    (FP64, (56, 60, 80), 0.2),       # whole tiles
+    (FP64, (57, 73, 90), 0.3),       # one column and one row more
+    (FP64, (122, 60, 44), 0.13),
+    (FP64, (40, 180, 171), 0.2),     # narrower than a tile
+    (FP64, (130, 40, 60), 0.5),      # all layer
+    (FP32, (48, 96, 120), 0.2),
+    (FP32, (65, 97, 161), 0.3),
+    (FP32, (200, 90, 33), 0.15),     # tiles of layer, main box and both
+    (FP32, (131, 57, 90), 0.05),
+    (FP32, (232, 40, 70), 0.13),     # packs of both kinds of cells
+    (FP32, (34, 300, 301), 0.03),     # one layer cell on each side in x
+])
+def test_strip_passes_equal_one_step_calls(prec, shape, percent):
+    a, b = make(shape, prec, percent), make(shape, prec, percent)
+    for n in (2, 5, 8, 1, 4):
+        for _ in range(n):
+            a.update_fields(1)
+        b.update_fields(n)
+        assert a.checksum() == b.checksum(), n
+    for q in range(12):
+        assert np.array_equal(a.split(q), b.split(q)), q
+    assert b.launch_stats()["passes"] == 1 + 2 + 4 + 2
+    a.close()
+    b.close()
+
+
+def test_more_steps_than_a_table_of_source_values():
+    a, b = make((96, 90, 100), FP32, 0.2), make((96, 90, 100), FP32, 0.2)
+    for _ in range(523):
+        a.update_fields(1)
+    b.update_fields(523)
+    assert a.checksum() == b.checksum()
+    assert b.launch_stats()["passes"] == 261
