@@ -2143,6 +2143,21 @@ __device__ __forceinline__ void load_to_lds(gptr<T> base, unsigned off, unsigned
                      "s"(base), "s"(lds) : "memory");
 }
 
+// Whether a probe lies among the columns and rows that a tile stores (long
+// lists are not searched).
+template <typename S, typename C>
+__device__ __forceinline__ bool tile_probes(const StripArgs<S, C>& a, int tile) {
+    if (a.probe.n > kTileSrcScan) return true;
+    const StripGeom& G = a.g;
+    const int rem = tile % (G.ntx * G.nty);
+    const int py0 = rem / G.ntx * G.TY, px0 = rem % G.ntx * G.TX;
+    const cptr<Probe> pr = as_const(a.probe.p);
+    bool any = false;
+    for (int q = 0; q < a.probe.n; ++q)
+        any = any || (pr[q].i >= px0 && pr[q].i < px0 + G.TX && pr[q].j >= py0 && pr[q].j < py0 + G.TY);
+    return any;
+}
+
 // One tile (index < a.g.ntiles) of a strip pass; every thread of the
 // workgroup calls it with the same tile.
 // STAGE: planes come in and go out through LDS.  Each wavefront moves its
@@ -2347,14 +2362,6 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
             const int di = wrap_mod(src[q].i - px0 + G.Gx, Ni), dj = wrap_mod(src[q].j - py0 + L, Nj);
             tile_src = tile_src || (di < RW && dj < ngroups * R);
         }
-    }
-    // Likewise for the probes and the cells this tile stores.
-    bool tile_probe = PROBE && a.probe.n > kTileSrcScan;
-    if (PROBE && !tile_probe) {
-        const cptr<Probe> pr = as_const(a.probe.p);
-        for (int q = 0; q < a.probe.n; ++q)
-            tile_probe = tile_probe || (pr[q].i >= px0 && pr[q].i < px0 + G.TX && pr[q].j >= py0 &&
-                                        pr[q].j < py0 + G.TY);
     }
     // Adds sources q0..q1-1 to the first curl terms, as add_point_sources
     // does.  The lane's cell is worked out here, from an opaque copy of the
@@ -2735,7 +2742,7 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
 #pragma unroll
                     for (int d = 0; d < 3; ++d) bnew[d][r][v] = as_stored<S>(bnew[d][r][v]);
                 }
-            if (PROBE && tile_probe) {
+            if (PROBE) {
                 // probes of step l: E of plane pkl, B of plane pkl-1, cells
                 // this tile stores
                 const int pe = kk - l, pkl = wrap_mod(pe, Nk);
@@ -2930,7 +2937,8 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
 
 // PROBE: the variant that records StripArgs::probe after each level (the
 // level's B is held in registers until then: up to 35 more VGPRs, which the
-// plain variant does without).
+// plain variant does without).  Tiles without a probe run the plain code in it:
+// 256^3 FP32 with 8 probes, 306 us per pass instead of 337.
 template <typename S, typename C, int V, int R, int L, bool FINAL, bool STAGE, bool FIRST,
           bool PROBE = false>
 __global__ void __launch_bounds__(strip_max_threads(V, R, L, sizeof(C)))
@@ -2939,7 +2947,10 @@ strip_sweep(StripArgs<S, C> a) {
     const int blk = blockIdx.x;
     const int tile = (blk & 7) * a.g.per_xcd + (blk >> 3);
     if (tile >= a.g.ntiles) return;  // whole workgroup
-    strip_tile<S, C, V, R, L, FINAL, STAGE, FIRST, false, PROBE>(a, tile, reinterpret_cast<C*>(lds_raw));
+    if (PROBE && tile_probes(a, tile))
+        strip_tile<S, C, V, R, L, FINAL, STAGE, FIRST, false, PROBE>(a, tile, reinterpret_cast<C*>(lds_raw));
+    else
+        strip_tile<S, C, V, R, L, FINAL, STAGE, FIRST>(a, tile, reinterpret_cast<C*>(lds_raw));
 }
 
 // FP16 storage: the strip pass after an in-run rescaling decision, reading
@@ -2952,7 +2963,10 @@ strip_rescale_sweep(StripArgs<S, C> a) {
     const int blk = blockIdx.x;
     const int tile = (blk & 7) * a.g.per_xcd + (blk >> 3);
     if (tile >= a.g.ntiles) return;  // whole workgroup
-    strip_tile<S, C, V, R, L, FINAL, STAGE, false, true, PROBE>(a, tile, reinterpret_cast<C*>(lds_raw));
+    if (PROBE && tile_probes(a, tile))
+        strip_tile<S, C, V, R, L, FINAL, STAGE, false, true, PROBE>(a, tile, reinterpret_cast<C*>(lds_raw));
+    else
+        strip_tile<S, C, V, R, L, FINAL, STAGE, false, true>(a, tile, reinterpret_cast<C*>(lds_raw));
 }
 
 // ---------------------------------------------------------------------------
@@ -3188,11 +3202,26 @@ __device__ __forceinline__ double block_max(double v, double* sh) {
     return r;
 }
 
-// Per-block partials of sum(x^2) (scaled by inv_scale) and max|x| for one array.
+// Per-block partials of sum(x^2) (scaled by inv_scale) and max|x| of six arrays,
+// blockIdx.y's partials at part + blockIdx.y * part_stride.  One launch for the six:
+// 256^3 FP32 76 us with the final pass, six pairs of launches 120.
+struct SixScales {
+    double inv[6];
+};
+
 template <typename S>
 __global__ void __launch_bounds__(kReduceThreads)
-sumsq_maxabs_partial(const S* __restrict__ x, size_t n, double inv_scale,
-                     double* __restrict__ part) {
+sumsq_maxabs_partial(Fields<S> f, size_t n, SixScales scales, double* __restrict__ part, int part_stride) {
+    const int comp = blockIdx.y;
+    const S* __restrict__ x = f.e[0];
+    double inv_scale = scales.inv[0];
+#pragma unroll
+    for (int c = 1; c < 6; ++c)
+        if (comp == c) {
+            x = c < 3 ? f.e[c < 3 ? c : 0] : f.b[c < 3 ? 0 : c - 3];
+            inv_scale = scales.inv[c];
+        }
+    part += static_cast<size_t>(comp) * part_stride;
     // x is an allocation's start (16-byte aligned): 16-byte packs (8 FP16,
     // 4 FP32 or 2 FP64 values), four in flight per thread, then the tail
     // element-wise.  A fixed grid keeps the summation order fixed.
@@ -3261,11 +3290,14 @@ diff_partial(const S* __restrict__ a, double inv_scale, const double* __restrict
 }
 
 // Final pass over `nblk` partial records of width w; column c is a sum
-// unless (max_mask >> c) & 1.  Deterministic: one block, fixed order.
+// unless (max_mask >> c) & 1.  Deterministic: one block, fixed order.  Block b
+// works on the records at part + b * stride and writes out[b*w ..].
 static __global__ void __launch_bounds__(kReduceThreads)
 reduce_partials(const double* __restrict__ part, int nblk, int w, unsigned max_mask,
-                double* __restrict__ out) {
+                double* __restrict__ out, int stride = 0) {
     __shared__ double sh[kReduceThreads];
+    part += static_cast<size_t>(blockIdx.x) * stride;
+    out += static_cast<size_t>(blockIdx.x) * w;
     for (int col = 0; col < w; ++col) {
         const bool is_max = (max_mask >> col) & 1u;
         double acc = 0.0;
@@ -3278,15 +3310,18 @@ reduce_partials(const double* __restrict__ part, int nblk, int w, unsigned max_m
     }
 }
 
-// out[0] = the sum of column 0 of `nblk` partial records of width w, in
-// reduce_partials' order (energy records equal fdtd_sum_squares bitwise).
+// out[b] = the sum of column 0 of `nblk` partial records of width w at part +
+// b * stride, in reduce_partials' order (energy records equal fdtd_sum_squares
+// bitwise).
 static __global__ void __launch_bounds__(kReduceThreads)
-sum_partials_col0(const double* __restrict__ part, int nblk, int w, double* __restrict__ out) {
+sum_partials_col0(const double* __restrict__ part, int nblk, int w, double* __restrict__ out,
+                  int stride) {
     __shared__ double sh[kReduceThreads];
+    part += static_cast<size_t>(blockIdx.x) * stride;
     double acc = 0.0;
     for (int b = threadIdx.x; b < nblk; b += kReduceThreads) acc = acc + part[b * w];
     const double r = block_sum(acc, sh);
-    if (threadIdx.x == 0) out[0] = r;
+    if (threadIdx.x == 0) out[blockIdx.x] = r;
 }
 
 // Probe values read from the fields in memory (the state after a step of

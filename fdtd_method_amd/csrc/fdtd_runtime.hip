@@ -1355,6 +1355,26 @@ int run_3sweep(fdtd_grid* g, int nsteps) {
     return FDTD_OK;
 }
 
+// Partials of the six fields' sums of squares and maxima, component c's at
+// parts + 2 * kReduceBlocks * c.
+void launch_partials(fdtd_grid* g, int nb, double* parts) {
+    fdtd::SixScales s;
+    for (int c = 0; c < 6; ++c) s.inv[c] = 1.0 / g->scales[c];
+    switch (g->precision) {
+        case FDTD_FP64:
+            hipLaunchKernelGGL(fdtd::sumsq_maxabs_partial<double>, dim3(nb, 6), dim3(256), 0, g->stream,
+                               fields_of<double>(g, g->cur), g->N, s, parts, 2 * kReduceBlocks);
+            break;
+        case FDTD_FP32:
+            hipLaunchKernelGGL(fdtd::sumsq_maxabs_partial<float>, dim3(nb, 6), dim3(256), 0, g->stream,
+                               fields_of<float>(g, g->cur), g->N, s, parts, 2 * kReduceBlocks);
+            break;
+        default:
+            hipLaunchKernelGGL(fdtd::sumsq_maxabs_partial<_Float16>, dim3(nb, 6), dim3(256), 0, g->stream,
+                               fields_of<_Float16>(g, g->cur), g->N, s, parts, 2 * kReduceBlocks);
+    }
+}
+
 // Energy record of the current state: the six sums of squares (physical
 // units) reduced into the next row of d_energy, queued without a wait, in
 // fdtd_sum_squares' summation order.
@@ -1363,26 +1383,9 @@ int record_energy(fdtd_grid* g) {
     if (row >= g->energy_cap) return fail(FDTD_ERR_INVALID_ARGUMENT, "energy records full");
     TraceRange tr("energy_record");
     const int nb = std::min<int>(kReduceBlocks, grid_blocks(g->N));
-    for (int c = 0; c < 6; ++c) {
-        const void* p = field_ptr(g, c);
-        const double inv = 1.0 / g->scales[c];
-        double* part = g->d_part + (size_t)2 * kReduceBlocks * c;
-        switch (g->precision) {
-            case FDTD_FP64:
-                hipLaunchKernelGGL(fdtd::sumsq_maxabs_partial<double>, dim3(nb), dim3(256), 0,
-                                   g->stream, static_cast<const double*>(p), g->N, inv, part);
-                break;
-            case FDTD_FP32:
-                hipLaunchKernelGGL(fdtd::sumsq_maxabs_partial<float>, dim3(nb), dim3(256), 0,
-                                   g->stream, static_cast<const float*>(p), g->N, inv, part);
-                break;
-            default:
-                hipLaunchKernelGGL(fdtd::sumsq_maxabs_partial<_Float16>, dim3(nb), dim3(256), 0,
-                                   g->stream, static_cast<const _Float16*>(p), g->N, inv, part);
-        }
-        hipLaunchKernelGGL(fdtd::sum_partials_col0, dim3(1), dim3(256), 0, g->stream, part, nb, 2,
-                           g->d_energy + 6 * row + c);
-    }
+    launch_partials(g, nb, g->d_part);
+    hipLaunchKernelGGL(fdtd::sum_partials_col0, dim3(6), dim3(256), 0, g->stream, g->d_part, nb, 2,
+                       g->d_energy + 6 * row, 2 * kReduceBlocks);
     HIP_TRY(hipGetLastError());
     g->energy_steps.push_back(g->step);
     return FDTD_OK;
@@ -1502,26 +1505,9 @@ void* field_ptr(fdtd_grid* g, int c);
 int reduce_fields_into(fdtd_grid* g, double* parts, double* res, double sumsq[6],
                        double maxabs[6]) {
     const int nb = std::min<int>(kReduceBlocks, grid_blocks(g->N));
-    for (int c = 0; c < 6; ++c) {
-        const void* p = field_ptr(g, c);
-        const double inv = 1.0 / g->scales[c];
-        double* part = parts + (size_t)2 * kReduceBlocks * c;
-        switch (g->precision) {
-            case FDTD_FP64:
-                hipLaunchKernelGGL(fdtd::sumsq_maxabs_partial<double>, dim3(nb), dim3(256), 0,
-                                   g->stream, static_cast<const double*>(p), g->N, inv, part);
-                break;
-            case FDTD_FP32:
-                hipLaunchKernelGGL(fdtd::sumsq_maxabs_partial<float>, dim3(nb), dim3(256), 0,
-                                   g->stream, static_cast<const float*>(p), g->N, inv, part);
-                break;
-            default:
-                hipLaunchKernelGGL(fdtd::sumsq_maxabs_partial<_Float16>, dim3(nb), dim3(256), 0,
-                                   g->stream, static_cast<const _Float16*>(p), g->N, inv, part);
-        }
-        hipLaunchKernelGGL(fdtd::reduce_partials, dim3(1), dim3(256), 0, g->stream, part, nb, 2,
-                           2u, res + 2 * c);
-    }
+    launch_partials(g, nb, parts);
+    hipLaunchKernelGGL(fdtd::reduce_partials, dim3(6), dim3(256), 0, g->stream, parts, nb, 2, 2u, res,
+                       2 * kReduceBlocks);
     HIP_TRY(hipGetLastError());
     double r[12];
     HIP_TRY(hipMemcpyAsync(r, res, sizeof r, hipMemcpyDeviceToHost, g->stream));
