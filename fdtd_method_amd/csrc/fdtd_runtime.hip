@@ -123,7 +123,11 @@ int default_kchunk(int Nj, int Nk, int TY) {
 
 // Widest V giving 16-byte lanes that divides Ni, then the largest TY with at
 // most 640 (FP32/FP16) or 768 (FP64) threads and 80 KiB of LDS per
-// workgroup; the autotuner refines this.
+// workgroup.  Grids of few planes take as few rows as give at most 192 tiles,
+// three quarters of the CUs (a sweep, us: 32^3 FP64 32 rows 5.6, 6 rows 4.8;
+// 64^3 FP32 39 rows 6.5, 22 rows 5.5; PML 48^3 FP64 20 rows 11.6, 12 rows 11.1;
+// a tile on every CU is 5% faster still alone, but 64^3 FP64 runs of several
+// grids at a time then take 1.41 ms instead of 1.20).  The autotuner refines this.
 bool default_tuning(const fdtd_grid* g, Tuning* t) {
     int vc[4];
     const int nv = v_candidates(g->precision, vc);
@@ -141,6 +145,8 @@ bool default_tuning(const fdtd_grid* g, Tuning* t) {
             for (int ty = std::min(g->Nj, mt / lanes - 1); ty >= 1; --ty)
                 if (sweep_lds_bytes(g, ty) <= lds_cap) { best = ty; break; }
             if (!best) continue;
+            const int least = g->pml ? 8 : 2;  // (PML 16^3: 16 rows 9.4 us, 4 rows 10.3)
+            while (best > least && (long long)((g->Nj + best - 2) / (best - 1)) * g->Nk <= 192) --best;
             t->V = V;
             t->TY = best;
             t->kchunk = default_kchunk(g->Nj, g->Nk, best);
