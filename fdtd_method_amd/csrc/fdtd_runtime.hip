@@ -278,10 +278,13 @@ bool inline_sources(const fdtd_grid* g, std::vector<fdtd::InlineSource>* out) {
         g->autoscale_interval > 0 || g->sparse_j.size() > (size_t)fdtd::kInlineSources)
         return false;
     out->clear();
-    for (const fdtd::PointSource& q : host_sources(g)) out->push_back({q.i, q.j, q.k, q.comp, q.amp});
-    std::stable_sort(out->begin(), out->end(), [](const fdtd::InlineSource& x, const fdtd::InlineSource& y) {
-        return x.k < y.k;
-    });
+    out->reserve(g->sparse_j.size());
+    const unsigned Ni = g->Ni, Nj = g->Nj;
+    for (const auto& kv : g->sparse_j) {  // in order of the cells' indices, hence by plane
+        const unsigned key = static_cast<unsigned>(kv.first / 3), row = key / Ni;
+        out->push_back({static_cast<int>(key - row * Ni), static_cast<int>(row % Nj),
+                        static_cast<int>(row / Nj), static_cast<int>(kv.first % 3), kv.second});
+    }
     return true;
 }
 
@@ -736,8 +739,9 @@ int launch_fused_a(fdtd_grid* g, const Tuning& t, int slot, int in, int out,
             inl.n = (int)x.inl->size();
             std::copy(x.inl->begin(), x.inl->end(), inl.src);
             if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(ikern), lds)) return rc;
-            hipLaunchKernelGGL(ikern, dim3(8 * a.g.per_xcd), dim3((t.TY + 1) * (g->Ni / V)), lds,
-                               g->stream, a, inl);
+            // whole wavefronts, each holding every source
+            const int threads = ((t.TY + 1) * (g->Ni / V) + 63) / 64 * 64;
+            hipLaunchKernelGGL(ikern, dim3(8 * a.g.per_xcd), dim3(threads), lds, g->stream, a, inl);
             HIP_TRY(hipGetLastError());
             return FDTD_OK;
         }
@@ -1035,12 +1039,12 @@ int strip_default_kchunk(const fdtd_grid* g, const BlockTuning& t, long long* pl
 
 // Whether strip passes of t.L steps beat as many single sweeps on a grid, by
 // what both cost on grids that fit the caches: a plane-round of a pass about
-// 3.5 us (FP64 W = 8, FP32 W = 16), a sweep 6.5 us up to 26 MB of E and B read
+// 3.5 us (FP64 W = 8, FP32 W = 16), a sweep 5 us up to 26 MB of E and B read
 // and written, beyond that 5 us and its bytes at 4.8 TB/s (FP32 128^3 26 us,
 // 160^3 48; FP64 131x90x70 26, 200x151x97 65).
 bool strips_pay(const fdtd_grid* g, const BlockTuning& t, long long planes) {
     const double mb = 12.0 * g->N * g->esize * 1e-6;
-    const double sweep = mb <= 26.0 ? 6.5 : 5.0 + mb / 4.8;
+    const double sweep = mb <= 26.0 ? 5.0 : 5.0 + mb / 4.8;
     return 3.5 * planes < t.L * sweep;
 }
 
