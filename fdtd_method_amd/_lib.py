@@ -107,8 +107,9 @@ def load():
         "fdtd_get_stream": ([_vp, ctypes.POINTER(_vp)], _i),
         "fdtd_update_b_box": ([_vp, ctypes.POINTER(_i), ctypes.POINTER(_i)], _i),
         "fdtd_update_e_box": ([_vp, ctypes.POINTER(_i), ctypes.POINTER(_i)], _i),
-        "fdtd_set_current_values": ([_vp, _i, ctypes.POINTER(ctypes.c_longlong),
-                                     ctypes.POINTER(_i), _dp], _i),
+        # (plain addresses: called before every step, where three pointer objects
+        # would cost more than the call)
+        "fdtd_set_current_values": ([_vp, _i, _vp, _vp, _vp], _i),
         "fdtd_set_point_sources": ([_vp, _i, ctypes.POINTER(PointSource)], _i),
         "fdtd_update_fields_with_currents": ([_vp, _i, ctypes.POINTER(_i),
                                               ctypes.POINTER(ctypes.c_longlong), ctypes.POINTER(_i),

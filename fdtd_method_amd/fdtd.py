@@ -38,6 +38,10 @@ def _dptr(a: np.ndarray):
     return a.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
 
 
+def _address(a: np.ndarray) -> int:
+    return a.__array_interface__["data"][0]
+
+
 class Field:
     """Host mirror of one component (the reference's ``Field&``)."""
 
@@ -227,9 +231,8 @@ class FDTD:
         idx = np.ascontiguousarray(index, dtype=np.int64)
         cc = np.ascontiguousarray(comp, dtype=np.int32)
         vv = np.ascontiguousarray(value, dtype=np.float64)
-        _lib.check(self._L.fdtd_set_current_values(
-            self._h, idx.size, idx.ctypes.data_as(ctypes.POINTER(ctypes.c_longlong)),
-            cc.ctypes.data_as(ctypes.POINTER(ctypes.c_int)), _dptr(vv)))
+        _lib.check(self._L.fdtd_set_current_values(self._h, idx.size, _address(idx), _address(cc),
+                                                   _address(vv)))
 
     def update_fields_with_currents(self, writes) -> None:
         """len(writes) steps; before step s the sparse currents writes[s] =
