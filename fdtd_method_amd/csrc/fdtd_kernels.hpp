@@ -636,6 +636,61 @@ pml_plain_update_B(Fields<S> f, Pml<S, C> P, Coefs<C> c, int Ni, int Nj, int Nk)
         pml_B_cell<S, C>(f, P, Ni, Nj, Nk, i, j, k);
 }
 
+// The same first B update in front of the sweeps of a run, marching up zc
+// planes per thread: Ex and Ey of plane k+1 are read once, a layer cell's B,
+// the sum of its splits, is not read, and only written (`totals`) where a sweep
+// follows that reads it.  15 words a layer cell instead of 23 with both planes
+// of E fetched: 512^3 FP32 with a 0.2 layer 1.78 ms instead of 2.24.
+template <typename S, typename C>
+__global__ void __launch_bounds__(256)
+pml_first_B(Fields<S> f, Pml<S, C> P, Coefs<C> c, int Ni, int Nj, int Nk, int zc, bool totals) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int j = blockIdx.y * blockDim.y + threadIdx.y;
+    if (i >= Ni || j >= Nj) return;
+    const int plane = Ni * Nj, row = i + j * Ni;
+    const int row_in = wrap(i + 1, Ni) + j * Ni, row_jn = i + wrap(j + 1, Nj) * Ni;
+    const bool xy = in_main(i, Ni, P.pi) && in_main(j, Nj, P.pj);
+    const C ax = P.tx[i], cyx = P.tx[3 * Ni + i], czx = P.tx[4 * Ni + i];
+    const C ay = P.ty[j], cxy = P.ty[3 * Nj + j], czy = P.ty[4 * Nj + j];
+    const int k0 = blockIdx.z * zc, k1 = min(k0 + zc, Nk);
+    C exn = f.e[0][row + k0 * plane], eyn = f.e[1][row + k0 * plane];
+    for (int k = k0; k < k1; ++k) {
+        const int off = k * plane, idx = row + off, next = row + wrap(k + 1, Nk) * plane;
+        const C ex = exn, ey = eyn, ez = f.e[2][idx];
+        exn = f.e[0][next];
+        eyn = f.e[1][next];
+        const C ey_ip = f.e[1][row_in + off], ez_ip = f.e[2][row_in + off];
+        const C ex_jp = f.e[0][row_jn + off], ez_jp = f.e[2][row_jn + off];
+        if (xy && in_main(k, Nk, P.pk)) {
+            const C dbx = sub_mul(c.bx_ey * (eyn - ey), c.bx_ez, ez_jp - ez);
+            const C dby = sub_mul(c.by_ez * (ez_ip - ez), c.by_ex, exn - ex);
+            const C dbz = sub_mul(c.bz_ex * (ex_jp - ex), c.bz_ey, ey_ip - ey);
+            f.b[0][idx] = static_cast<S>(C(f.b[0][idx]) + dbx);
+            f.b[1][idx] = static_cast<S>(C(f.b[1][idx]) + dby);
+            f.b[2][idx] = static_cast<S>(C(f.b[2][idx]) + dbz);
+        } else {
+            const C az = P.tz[k], cxz = P.tz[3 * Nk + k], cyz = P.tz[4 * Nk + k];
+            const C byx = stored<S, C>(C(P.bs[kByx][idx]) * ax + cyx * (ez_ip - ez));
+            const C bzx = stored<S, C>(C(P.bs[kBzx][idx]) * ax - czx * (ey_ip - ey));
+            const C bxy = stored<S, C>(C(P.bs[kBxy][idx]) * ay - cxy * (ez_jp - ez));
+            const C bzy = stored<S, C>(C(P.bs[kBzy][idx]) * ay + czy * (ex_jp - ex));
+            const C bxz = stored<S, C>(C(P.bs[kBxz][idx]) * az + cxz * (eyn - ey));
+            const C byz = stored<S, C>(C(P.bs[kByz][idx]) * az - cyz * (exn - ex));
+            P.bs[kByx][idx] = static_cast<S>(byx);
+            P.bs[kBzx][idx] = static_cast<S>(bzx);
+            P.bs[kBxy][idx] = static_cast<S>(bxy);
+            P.bs[kBzy][idx] = static_cast<S>(bzy);
+            P.bs[kBxz][idx] = static_cast<S>(bxz);
+            P.bs[kByz][idx] = static_cast<S>(byz);
+            if (totals) {
+                f.b[0][idx] = static_cast<S>(bxy + bxz);
+                f.b[1][idx] = static_cast<S>(byz + byx);
+                f.b[2][idx] = static_cast<S>(bzx + bzy);
+            }
+        }
+    }
+}
+
 // E on the main box (with J) and the split update on the layer,
 // FDTD_PML.cpp:354-362.
 template <typename S, typename C, typename JT>

@@ -389,6 +389,30 @@ int launch_plain_B(fdtd_grid* g, bool layer) {
     return FDTD_OK;
 }
 
+// The first B update of a PML run, 16 planes per thread where that leaves two
+// rounds of workgroups and more.
+template <typename S>
+int launch_pml_first_B(fdtd_grid* g, bool totals) {
+    using C = typename fdtd::ComputeOf<S>::type;
+    const dim3 block(64, 4, 1);
+    dim3 grid((g->Ni + 63) / 64, (g->Nj + 3) / 4, 1);
+    int zc = 16;
+    while (zc > 1 && (long long)grid.x * grid.y * ((g->Nk + zc - 1) / zc) < 16 * device_cus()) zc /= 2;
+    grid.z = (g->Nk + zc - 1) / zc;
+    hipLaunchKernelGGL((fdtd::pml_first_B<S, C>), grid, block, 0, g->stream, fields_of<S>(g, g->cur),
+                       make_pml<S, C>(g, g->cur, g->cur), make_coefs<C>(g), g->Ni, g->Nj, g->Nk, zc, totals);
+    HIP_TRY(hipGetLastError());
+    return FDTD_OK;
+}
+
+int pml_first_B(fdtd_grid* g, bool totals) {
+    switch (g->precision) {
+        case FDTD_FP64: return launch_pml_first_B<double>(g, totals);
+        case FDTD_FP32: return launch_pml_first_B<float>(g, totals);
+        default: return launch_pml_first_B<_Float16>(g, totals);
+    }
+}
+
 template <typename S>
 int launch_plain_E(fdtd_grid* g, long long step) {
     using C = typename fdtd::ComputeOf<S>::type;
@@ -1278,10 +1302,12 @@ int run_fused(fdtd_grid* g, int nsteps, hipEvent_t mid = nullptr) {
     const bool use_inl = inline_sources(g, &inl);
     int rc = use_inl ? FDTD_OK : flush_sources(g);
     if (rc) return rc;
+    const bool pml_strips = g->pml && g->pml_path == 0 && g->pml_strip_kchunk > 0 && nsteps >= 2 &&
+                            !g->j_dense_active;
     if (carried < 0) {
         TraceRange tr("b_half_prologue");
         hipEvent_t t0 = trace_begin(g);
-        rc = plain_B(g);
+        rc = g->pml ? pml_first_B(g, !pml_strips || nsteps % 2 != 0) : plain_B(g);
         trace_end(g, t0, 0, false);
     }
     if (rc) return rc;
@@ -1289,8 +1315,7 @@ int run_fused(fdtd_grid* g, int nsteps, hipEvent_t mid = nullptr) {
     const int ahead_buf = carried < 0 ? 0 : 1 - carried;
     g->ba_cur = -1;
     if (mid) HIP_TRY(hipEventRecord(mid, g->stream));
-    if (g->pml && g->pml_path == 0 && g->pml_strip_kchunk > 0 && nsteps >= 2 && !g->j_dense_active)
-        return run_pml_strips(g, nsteps);
+    if (pml_strips) return run_pml_strips(g, nsteps);
     const int iv = g->precision == FDTD_FP16 ? g->autoscale_interval : 0;
     for (int s = 0; s < nsteps; ++s) {
         const bool decide = iv > 0 && s > 0 && s % iv == 0 && s + 1 < nsteps;
