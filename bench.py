@@ -502,22 +502,25 @@ def bench_blocked(a):
     print(json.dumps(out), flush=True)
 
 
-def pml_bytes_per_step(shape, widths, word):
+def pml_bytes_per_step(shape, widths, word, steps_per_launch=1):
     """Algorithmic HBM bytes of one PML step: main-box cells read and write
-    E and B (12 words); layer cells also read and write their 12 split
-    fields (36 words)."""
+    E and B (12 words); layer cells read and write their 12 split fields, and a
+    sweep (one step per launch) B's totals as well (30 words).  A strip pass
+    takes two steps per read and write of the state (24 words a layer cell)."""
     Ni, Nj, Nk = shape
     main = 1
     for n, p in zip(shape, widths):
         main *= max(0, n - 2 * p)
     layer = Ni * Nj * Nk - main
-    return word * (12 * main + 36 * layer), main, layer
+    words = 12 * main + (30 if steps_per_launch == 1 else 24) * layer
+    return word * words / steps_per_launch, main, layer
 
 
 def bench_pml(a):
     """The PML workload on both PML step forms: the two in-place phase sweeps
-    per step (pml_e_phase, pml_b_phase) and the fused PML sweep.  `value` is
-    the grid's default form in FP32."""
+    per step (pml_e_phase, pml_b_phase) and the fused form, which takes strip
+    passes of two steps where the grid runs them, else the fused PML sweep.
+    `value` is the grid's default form in FP32."""
     from fdtd_method_amd import FDTD_PML
     n, K, pml = a.n, a.steps, a.pml
     dt = 0.5 / (C * np.sqrt(3.0))
@@ -547,12 +550,13 @@ def bench_pml(a):
         prec = {"fp32": Precision.FP32, "fp64": Precision.FP64, "fp16": Precision.FP16}[a.profile]
         g = make(prec, a.pml_form or default_form)
         r = run_path(g, K, a.warmup)
-        nbytes, main, layer = pml_bytes_per_step((n, n, n), g.pml_widths, WORD[prec])
+        spl = 2 if g.launch_stats()["passes"] else 1
+        nbytes, main, layer = pml_bytes_per_step((n, n, n), g.pml_widths, WORD[prec], spl)
         ms_copy = calibration_copy(1 << 30, 5)
         print(json.dumps(dict(profile=a.profile, workload="pml", n=n, pml=pml, steps=K,
                               form=a.pml_form or default_form, pml_path=g.get_pml_path(),
                               tuning=g.get_tuning(), widths=g.pml_widths,
-                              alg_bytes_per_step=nbytes, main_cells=main, layer_cells=layer,
+                              steps_per_launch=spl, alg_bytes_per_step=nbytes, main_cells=main, layer_cells=layer,
                               **r, calibration_copy=dict(bytes=1 << 30, ms=ms_copy))),
               flush=True)
         return
@@ -563,10 +567,12 @@ def bench_pml(a):
         for form in ("phases", "fused"):
             g = make(prec, form)
             r = run_path(g, K, a.warmup)
-            nbytes, main, layer = pml_bytes_per_step((n, n, n), g.pml_widths, WORD[prec])
-            gbs = nbytes / (r["steady_launch_ms"] * 1e-3) / 1e9
-            rec = dict(gcells=r["gcells"], ms_per_step=r["ms_per_step"],
-                       step_kernel_ms=r["steady_launch_ms"], alg_bytes_per_step=nbytes,
+            spl = 2 if g.launch_stats()["passes"] else 1
+            nbytes, main, layer = pml_bytes_per_step((n, n, n), g.pml_widths, WORD[prec], spl)
+            step_ms = r["steady_launch_ms"] / spl
+            gbs = nbytes / (step_ms * 1e-3) / 1e9
+            rec = dict(gcells=r["gcells"], ms_per_step=r["ms_per_step"], steps_per_launch=spl,
+                       step_kernel_ms=step_ms, alg_bytes_per_step=nbytes,
                        alg_gbs=gbs, frac_of_peak=gbs / PEAK_GBS)
             if form == "fused":
                 rec["launch_shape"] = g.get_tuning()
@@ -577,7 +583,7 @@ def bench_pml(a):
                 rec["phase_bytes_per_step"] = wd * (18 * main + 36 * layer)
             res[f"{prec.name.lower()}_{form}"] = rec
             log(f"pml {prec.name} {form}: {r['gcells']:.1f} Gcell/s, step kernels "
-                f"{r['steady_launch_ms']:.3f} ms, {gbs:.0f} GB/s algorithmic")
+                f"{step_ms:.3f} ms, {gbs:.0f} GB/s algorithmic")
             if form == default_form:
                 grids[prec] = g
             else:
@@ -585,10 +591,12 @@ def bench_pml(a):
     err = errors(grids[Precision.FP32], grids[Precision.FP64])
     widths = grids[Precision.FP32].pml_widths
     en = energy(grids[Precision.FP64])
-    nbytes, main, layer = pml_bytes_per_step((n, n, n), widths, 4)
     r32 = res[f"fp32_{default_form}"]
+    spl = r32["steps_per_launch"]
+    nbytes, main, layer = pml_bytes_per_step((n, n, n), widths, 4, spl)
     kern = ("fdtd::pml_e_phase<float,float,float,V> + fdtd::pml_b_phase<float,float,float,V,true>"
-            if default_form == "phases" else "fdtd::fused_pml_sweep<float,float,float,V,true>")
+            if default_form == "phases" else "fdtd::pml_strip_sweep<float,float,false>" if spl == 2
+            else "fdtd::fused_pml_sweep<float,float,float,V,true>")
     cpu = None if a.no_cpu_baseline else cpu_baseline(min(n, 256), pml)
     out = {
         "metric": "Gcell-updates/s and %HBM roofline of the PML (absorbing layer) step",
@@ -602,9 +610,11 @@ def bench_pml(a):
                    "main_box_cells": main, "layer_cells": layer, "pml_step_form": default_form},
         "roofline": {"bound": "hbm", "achieved": r32["alg_gbs"], "peak": PEAK_GBS, "unit": "GB/s",
                      "frac": r32["alg_gbs"] / PEAK_GBS,
+                     # (the committed record is the fused sweep's)
                      "traffic": committed_traffic(PML_TRAFFIC_FILE, n=n, pml=pml,
                                                   form=default_form,
-                                                  tuning=list(grids[Precision.FP32].get_tuning())),
+                                                  tuning=list(grids[Precision.FP32].get_tuning()))
+                     if spl == 1 else None,
                      "kernel": kern, "alg_bytes_per_step": nbytes,
                      "step_kernel_ms": r32["step_kernel_ms"]},
         "cpu_baseline": cpu,

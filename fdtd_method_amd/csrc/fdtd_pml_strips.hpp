@@ -30,9 +30,10 @@ namespace fdtd {
 // issued after its loads under way.
 //
 // What bounds it: memory.  512^3 FP32 with a 0.2 layer: 3.32 ms per pass, where
-// two fused sweeps take 6.4; about 15 GB of traffic (a cell's words once
-// would be 11.4; neighbouring tiles read their ghost cells from L2 or again),
-// 4.5 TB/s, the arithmetic alone takes 1.7 ms.  Registers and LDS hold no larger
+// two fused sweeps take 6.4; 18.6 GB of traffic (a cell's words once would be
+// 11.5; neighbouring tiles read their ghost cells again, and 52 columns touch
+// three 128-byte lines a row), 5.6 TB/s where a plain copy reaches 4.7; the
+// arithmetic alone takes 1.7 ms.  Registers and LDS hold no larger
 // tile: 42 words of state a cell.  FP32 tiles of 128 x 16 cells, one workgroup a
 // CU, took 3.73 ms, of 64 x 32 3.92.  FP64: 256^3 0.95 ms (two sweeps 1.59),
 // 128^3 0.168 (0.200).
