@@ -488,10 +488,13 @@ int box_update(fdtd_grid* g, const fdtd::Box& box, bool e_step) {
 
 // Chunk of Nk planes with the fewest plane-rounds (planes, when set) for nxy
 // tiles a chunk and `slots` workgroups at a time (see strip_default_kchunk).
+// Beyond 64 rounds shorter chunks only add planes, so a grid of millions of
+// planes is not searched through.
 int strip_chunk(int Nk, long long nxy, long long slots, int L, long long* planes) {
+    const int most = static_cast<int>(std::min<long long>(Nk, 64 + 64 * slots / std::max(1LL, nxy)));
     long long best_cost = -1;
     int best = Nk;
-    for (int nchunk = 1; nchunk <= Nk; ++nchunk) {
+    for (int nchunk = 1; nchunk <= most; ++nchunk) {
         const int kc = (Nk + nchunk - 1) / nchunk;
         const int nc = (Nk + kc - 1) / kc;
         const long long rounds = (nxy * nc + slots - 1) / slots;

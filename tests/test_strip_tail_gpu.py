@@ -57,6 +57,7 @@ def test_steps_left_over(prec, shape, L, counts):
     (FP32, (33, 150, 181), True),   # one tile across
     (FP32, (72, 70, 74), False),
     (FP16, (120, 120, 120), False),
+    (FP64, (3, 2, 200000), False),  # few tiles, many planes
 ])
 def test_default_of_narrow_grids(prec, shape, blocked):
     a, b = make(shape, prec), make(shape, prec)
