@@ -966,10 +966,12 @@ int strip_occupancy(const fdtd_grid* g, const BlockTuning& t) {
 // fdtd_autotune_blocking's picks, kept across processes in a text file (the
 // path of fdtd_set_tune_cache, else $FDTD_MI355X_TUNE_CACHE; none: off).
 // One line per pick, "<key> | L V lanes TYg kchunk R ms", the key naming
-// the cache format, shape, precision, device architecture and CU count;
+// the cache version, shape, precision, device architecture and CU count;
 // the last line of a key wins, and a pick that no longer validates is
-// timed again.
-constexpr int kTuneCacheVersion = 1;
+// timed again.  The version changes whenever a shape's tiles or its kernel do:
+// a pick timed on other code is not the fastest here, and its time is not this
+// code's.  (1: strip passes straight from memory, FP64 tiles of 64 columns.)
+constexpr int kTuneCacheVersion = 2;
 std::mutex g_tune_mu;
 std::string g_tune_path;
 bool g_tune_path_set = false;

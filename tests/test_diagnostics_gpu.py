@@ -95,3 +95,23 @@ def test_autotune_cache(tmp_path):
             g.close()
     finally:
         set_tune_cache(None)
+
+
+def test_autotune_cache_of_other_kernels(tmp_path):
+    """A pick recorded under an older version, valid as a shape, is not taken:
+    it was timed on other kernels."""
+    path = tmp_path / "tune.txt"
+    set_tune_cache(path)
+    try:
+        dt = courant_dt(1, 1, 1)
+        g = FDTD(Parameters(64, 48, 20), dt, Precision.FP64)
+        g.autotune_blocking(reps=1)
+        key = path.read_text().splitlines()[0].split("|")[0].strip()
+        old = " ".join(["v1"] + key.split()[1:])
+        path.write_text(f"{old} | 1 1 64 4 20 2 0.0001\n")
+        cfg, ms = g.autotune_blocking(reps=1)
+        assert ms != pytest.approx(0.0001)
+        assert len(path.read_text().splitlines()) == 2  # timed and recorded
+        g.close()
+    finally:
+        set_tune_cache(None)
