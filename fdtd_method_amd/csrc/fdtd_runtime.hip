@@ -488,6 +488,10 @@ int box_update(fdtd_grid* g, const fdtd::Box& box, bool e_step) {
 
 // Chunk of Nk planes with the fewest plane-rounds (planes, when set) for nxy
 // tiles a chunk and `slots` workgroups at a time (see strip_default_kchunk).
+// A chunk of kc planes is marched in kc + 2L-1: the one below it gives the
+// first plane its B, and each of the L levels ends one plane further on.  (Not
+// counted for L = 1, that plane made chunks of one plane look free: 256^3, us a
+// step FP32 326 instead of 225, FP16 261 instead of 144.)
 // Beyond 64 rounds shorter chunks only add planes, so a grid of millions of
 // planes is not searched through.
 int strip_chunk(int Nk, long long nxy, long long slots, int L, long long* planes) {
@@ -498,7 +502,7 @@ int strip_chunk(int Nk, long long nxy, long long slots, int L, long long* planes
         const int kc = (Nk + nchunk - 1) / nchunk;
         const int nc = (Nk + kc - 1) / kc;
         const long long rounds = (nxy * nc + slots - 1) / slots;
-        const long long cost = rounds * (kc + 2 * (L - 1));
+        const long long cost = rounds * (kc + 2 * L - 1);
         if (best_cost < 0 || cost < best_cost) {
             best_cost = cost;
             best = kc;
@@ -589,7 +593,7 @@ fdtd::StripGeom make_pml_strip_geom(const fdtd_grid* g, int kchunk) {
 }
 
 // z chunk of a PML grid's strip passes, the one with the fewest plane-rounds; 0
-// where two fused sweeps cost less.  A pass of few planes takes 7 us and 6.5 us
+// where two fused sweeps cost less.  A pass of few planes takes 0.5 us and 6.5 us
 // a plane-round, two sweeps 24 us up to 26 MB (24 words a cell), beyond that 22
 // us and 0.45 us a MB (us, pass against sweeps: FP64 64^3 45 / 43, 80^3 47 / 66,
 // 128^3 168 / 200; FP32 64^3 34 / 25, 80^3 38 / 48, 128^3 102 / 120).
@@ -603,7 +607,7 @@ int pml_strip_chunk(const fdtd_grid* g) {
     int kc = strip_chunk(g->Nk, (long long)G.ntx * G.nty, fdtd::pml_strip_wgs(cs) * device_cus(),
                          fdtd::kPmlStripL, &planes);
     const double mb = 24e-6 * g->N * g->esize;
-    if (7.0 + 6.5 * planes > (mb <= 26.0 ? 24.0 : 22.0 + 0.45 * mb)) return 0;
+    if (0.5 + 6.5 * planes > (mb <= 26.0 ? 24.0 : 22.0 + 0.45 * mb)) return 0;
     while (fdtd::pml_strip_lds_bytes(cs, kc) * fdtd::pml_strip_wgs(cs) > kLdsLimit) kc = (kc + 1) / 2;  // (its z tables)
     return kc;
 }
@@ -1049,13 +1053,13 @@ int device_cus() {
     return cus;
 }
 
-// z chunk length of a strip pass: every tile costs kchunk + 2(L-1) planes
-// (the pipeline fills and drains over L-1 planes at each end), and the
-// tiles run in rounds of (resident workgroups per CU x CUs); the chunking
+// z chunk length of a strip pass: every tile costs kchunk + 2L-1 planes
+// (the pipeline fills and drains over L-1 planes at each end, and starts one
+// plane below), and the tiles run in rounds of (resident workgroups per CU x CUs); the chunking
 // with the fewest plane-rounds wins (ties: fewer chunks).  A grid whose tiles
 // are few gets chunks of a few planes: a plane takes about 3 us however few
-// workgroups run, so 128^3 FP32 (18 tiles a plane) takes 10 planes, 16
-// plane-rounds, instead of 16 planes, 22 (65 us a pass).  planes, when set, is
+// workgroups run, so 128^3 FP32 (18 tiles a plane) takes 10 planes, 17
+// plane-rounds, instead of 16 planes, 23 (65 us a pass).  planes, when set, is
 // the plane-rounds of the choice.
 int strip_default_kchunk(const fdtd_grid* g, const BlockTuning& t, long long* planes = nullptr) {
     BlockTuning u = t;
@@ -1068,13 +1072,13 @@ int strip_default_kchunk(const fdtd_grid* g, const BlockTuning& t, long long* pl
 
 // Whether strip passes of t.L steps beat as many single sweeps on a grid, by
 // what both cost on grids that fit the caches: a plane-round of a pass about
-// 3.5 us (FP64 W = 8, FP32 W = 16), a sweep 5 us up to 26 MB of E and B read
+// 3.3 us (FP64 W = 8, FP32 W = 16), a sweep 5 us up to 26 MB of E and B read
 // and written, beyond that 5 us and its bytes at 4.8 TB/s (FP32 128^3 26 us,
 // 160^3 48; FP64 131x90x70 26, 200x151x97 65).
 bool strips_pay(const fdtd_grid* g, const BlockTuning& t, long long planes) {
     const double mb = 12.0 * g->N * g->esize * 1e-6;
     const double sweep = mb <= 26.0 ? 5.0 : 5.0 + mb / 4.8;
-    return 3.5 * planes < t.L * sweep;
+    return 3.3 * planes < t.L * sweep;
 }
 
 template <typename S, int V, bool FINAL>

@@ -269,3 +269,14 @@ def test_strip_blocking_fp16_in_run_rescaling():
     assert r_ref <= 5e-3
     assert r_ub <= 5e-3
 
+
+@pytest.mark.parametrize("prec", [Precision.FP64, Precision.FP32, Precision.FP16])
+@pytest.mark.parametrize("L", [1, 2, 3, 4])
+def test_default_z_chunk_marches_few_planes_twice(prec, L):
+    """A chunk of kc planes is marched in kc + 2L-1: on a grid whose tiles
+    fill the device several times over, no default chunk is shorter than the
+    planes it marches besides its own."""
+    g = FDTD(Parameters(256, 256, 256), courant_dt(1, 1, 1), prec)
+    g.set_time_blocking_strips(L, 1, 2, 8 if prec == Precision.FP64 else 16)
+    assert g.get_time_blocking_strips()["kchunk"] >= 2 * (2 * L - 1)
+    g.close()
