@@ -73,6 +73,7 @@ struct fdtd_batch {
     std::vector<fdtd::StripGeom> sgeom;
     int2* d_swork = nullptr;
     int snwork = 0;
+    int snblocks = 0;  // workgroups of a pass (a tile each, or as many as are resident)
     size_t slds = 0;
     int sdepth = 0;  // input planes the strip tiles stage in LDS (0: direct)
     void* d_sgrids = nullptr;
@@ -94,7 +95,7 @@ void drop_graph(fdtd_batch* b) {
 // The values a graph captured for nsteps steps depends on (see graph_key).
 std::vector<long long> graph_key_of(const fdtd_batch* b, int nsteps) {
     auto addr = [](const void* p) { return static_cast<long long>(reinterpret_cast<uintptr_t>(p)); };
-    return {nsteps, b->total_src, b->sL, b->sV, b->sR, b->sW, b->sdepth, b->snwork,
+    return {nsteps, b->total_src, b->sL, b->sV, b->sR, b->sW, b->sdepth, b->snwork, b->snblocks,
             b->nwork, b->nblocks, b->shape.V, b->shape.NT,
             addr(b->d_src), addr(b->d_vals), addr(b->d_kstart), addr(b->d_grids),
             addr(b->d_sgrids), addr(b->d_work), addr(b->d_swork), addr(b->d_counters),
@@ -276,11 +277,12 @@ int launch_batch_strip_s(fdtd_batch* b, bool final, bool first, int parity, cons
     a.vals = vals;
     a.vstride = b->total_src;
     a.pad = 0;
+    a.counters = b->d_counters;
     const void* kern = batch_strip_kernel<S>(b->sV, b->sR, b->sL, final, b->sdepth > 0, first);
     if (!kern) return fail(FDTD_ERR_UNSUPPORTED, "strip variant V=%d R=%d not built", b->sV, b->sR);
     if (int rc = allow_dynamic_lds(kern, b->slds)) return rc;
     void* args[] = {&a};
-    HIP_TRY(hipLaunchKernel(kern, dim3(b->snwork), dim3(64 * b->sW), args, b->slds, b->stream));
+    HIP_TRY(hipLaunchKernel(kern, dim3(b->snblocks), dim3(64 * b->sW), args, b->slds, b->stream));
     return FDTD_OK;
 }
 
@@ -296,7 +298,7 @@ int launch_batch_strip(fdtd_batch* b, bool final, bool first, int parity, const 
 }
 
 // Strip tiling of every grid (L, V, R rows per lane, W wavefronts), its
-// work list (most expensive tiles first) and the persistent grid size.
+// work list (most expensive tiles first) and the workgroups of a pass.
 // Every z chunk of a tile repeats the pipeline's 2(L-1) fill planes, while
 // fewer, longer tiles fill the device's resident workgroups in coarser
 // rounds.  For each candidate chunk length (whole grids down to about
@@ -411,6 +413,7 @@ int apply_strips(fdtd_batch* b, int L, int V, int R, int W) {
                       hipMemcpyHostToDevice));
     b->sgeom = geom;
     b->snwork = (int)sorted.size();
+    b->snblocks = depth > 0 ? b->snwork : (int)std::min(sorted.size(), slots);
     b->slds = lds;
     b->sdepth = depth;
     b->sL = L;

@@ -288,3 +288,30 @@ def test_batch_256_grid_workload_graph_strips():
     b.close()
     for g in grids + keep:
         g.close()
+
+
+@pytest.mark.parametrize("prec,L,W", [(Precision.FP64, 4, 8), (Precision.FP64, 2, 8),
+                                      (Precision.FP32, 4, 16), (Precision.FP32, 1, 16),
+                                      (Precision.FP16, 3, 16)])
+def test_batch_of_more_strip_tiles_than_workgroups(prec, L, W):
+    """Tiles straight from memory come from a queue: 600 of them, more than
+    workgroups are resident, of two costs, in several calls and replays."""
+    shapes = [(113, 49, 3 + q % 2) for q in range(67)]
+    singles = [make(s, prec, q) for q, s in enumerate(shapes)]
+    batched = [make(s, prec, q) for q, s in enumerate(shapes)]
+    b = Batch(batched)
+    b.set_time_blocking_strips(L, 1, 2, W)
+    for g in singles:
+        g.set_time_blocking_strips(0)
+        g.set_step_carry(False)  # a batch call starts from the B/2 prologue
+    for n in (2 * L, L + 1):
+        for g in singles:
+            g.update_fields(n)
+        b.update_fields(n)
+        assert [g.checksum() for g in singles] == [g.checksum() for g in batched], n
+    b.update_fields_graph(2 * L, 3)
+    for _ in range(3):
+        for g in singles:
+            g.update_fields(2 * L)
+    assert [g.checksum() for g in singles] == [g.checksum() for g in batched]
+    b.close()
