@@ -76,6 +76,7 @@ struct fdtd_batch {
     int snblocks = 0;  // workgroups of a pass (a tile each, or as many as are resident)
     size_t slds = 0;
     int sdepth = 0;  // input planes the strip tiles stage in LDS (0: direct)
+    int slanes = 64;  // lanes of their rows
     void* d_sgrids = nullptr;
     size_t sgrid_desc_bytes = 0;
     std::vector<unsigned char> h_sgrids;
@@ -95,7 +96,7 @@ void drop_graph(fdtd_batch* b) {
 // The values a graph captured for nsteps steps depends on (see graph_key).
 std::vector<long long> graph_key_of(const fdtd_batch* b, int nsteps) {
     auto addr = [](const void* p) { return static_cast<long long>(reinterpret_cast<uintptr_t>(p)); };
-    return {nsteps, b->total_src, b->sL, b->sV, b->sR, b->sW, b->sdepth, b->snwork, b->snblocks,
+    return {nsteps, b->total_src, b->sL, b->sV, b->sR, b->sW, b->sdepth, b->slanes, b->snwork, b->snblocks,
             b->nwork, b->nblocks, b->shape.V, b->shape.NT,
             addr(b->d_src), addr(b->d_vals), addr(b->d_kstart), addr(b->d_grids),
             addr(b->d_sgrids), addr(b->d_work), addr(b->d_swork), addr(b->d_counters),
@@ -258,11 +259,11 @@ int launch_batch(fdtd_batch* b, bool steady, int parity, const double* vals_row)
 
 // ---- strip passes --------------------------------------------------------
 
-const void* strip_kernel(int precision, int V, int R, int L, bool final, bool stage, bool first) {
+const void* strip_kernel(int precision, int V, int R, int L, int lanes, bool final, bool stage, bool first) {
     switch (precision) {
-        case FDTD_FP64: return batch_strip_kernel<double>(V, R, L, final, stage, first);
-        case FDTD_FP32: return batch_strip_kernel<float>(V, R, L, final, stage, first);
-        default: return batch_strip_kernel<_Float16>(V, R, L, final, stage, first);
+        case FDTD_FP64: return batch_strip_kernel<double>(V, R, L, lanes, final, stage, first);
+        case FDTD_FP32: return batch_strip_kernel<float>(V, R, L, lanes, final, stage, first);
+        default: return batch_strip_kernel<_Float16>(V, R, L, lanes, final, stage, first);
     }
 }
 
@@ -278,7 +279,7 @@ int launch_batch_strip_s(fdtd_batch* b, bool final, bool first, int parity, cons
     a.vstride = b->total_src;
     a.pad = 0;
     a.counters = b->d_counters;
-    const void* kern = batch_strip_kernel<S>(b->sV, b->sR, b->sL, final, b->sdepth > 0, first);
+    const void* kern = batch_strip_kernel<S>(b->sV, b->sR, b->sL, b->slanes, final, b->sdepth > 0, first);
     if (!kern) return fail(FDTD_ERR_UNSUPPORTED, "strip variant V=%d R=%d not built", b->sV, b->sR);
     if (int rc = allow_dynamic_lds(kern, b->slds)) return rc;
     void* args[] = {&a};
@@ -323,12 +324,28 @@ int apply_strips(fdtd_batch* b, int L, int V, int R, int W) {
     int depth = 2;
     for (const fdtd_grid* g : b->grids)
         depth = std::min(depth, strip_stage_depth(L, V, R, W, g->Ni, b->precision));
-    const int TY = fdtd::strip_tile_rows(W, R, cs) - 2 * L;
+    // row width, the same for every grid (see strip_direct_lanes)
+    int lanes = cs == 8 ? fdtd::strip_stage_lanes(cs) : 64;
+    if (cs == 8 && depth == 0) {
+        double cost[2] = {0, 0};
+        size_t cells = 0;
+        for (const fdtd_grid* g : b->grids) {
+            cells += g->N;
+            for (int q = 0; q < 2; ++q) {
+                int Gx, TX;
+                strip_x_geometry(L, V, b->precision, false, q ? 32 : 64, &Gx, &TX);
+                const int rows = fdtd::strip_tile_rows(W, R, q ? 32 : 64) - 2 * L;
+                cost[q] += (double)((g->Ni + TX - 1) / TX) * ((g->Nj + rows - 1) / rows) * (g->Nk + 2 * L - 1);
+            }
+        }
+        lanes = cost[1] * strip_narrow_cost(L, cells) < cost[0] ? 32 : 64;
+    }
+    const int TY = fdtd::strip_tile_rows(W, R, lanes) - 2 * L;
     const size_t lds = fdtd::strip_lds_bytes(L, W, V, R, cs, (int)storage_size(b->precision), depth);
     if (lds > kLdsLimit) return fail(FDTD_ERR_INVALID_ARGUMENT, "strip tiles need too much LDS");
     int per_cu = 0;
     for (bool final : {false, true}) {
-        const void* kern = strip_kernel(b->precision, V, R, L, final, depth > 0, false);
+        const void* kern = strip_kernel(b->precision, V, R, L, lanes, final, depth > 0, false);
         if (!kern) return fail(FDTD_ERR_UNSUPPORTED, "strip variant not built");
         if (int rc = allow_dynamic_lds(kern, lds)) return rc;
         if (!final) HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 64 * W, lds));
@@ -357,8 +374,8 @@ int apply_strips(fdtd_batch* b, int L, int V, int R, int W) {
             G.W = W;
             // the granule-aligned width where it needs no more tiles
             int Gx = 0, TX = 0;
-            strip_x_geometry(L, V, b->precision, depth > 0, &Gx, &TX, false);
-            strip_x_geometry(L, V, b->precision, depth > 0, &G.Gx, &G.TX, true);
+            strip_x_geometry(L, V, b->precision, depth > 0, lanes, &Gx, &TX, false);
+            strip_x_geometry(L, V, b->precision, depth > 0, lanes, &G.Gx, &G.TX, true);
             if ((g->Ni + TX - 1) / TX < (g->Ni + G.TX - 1) / G.TX) {
                 G.Gx = Gx;
                 G.TX = TX;
@@ -416,6 +433,7 @@ int apply_strips(fdtd_batch* b, int L, int V, int R, int W) {
     b->snblocks = depth > 0 ? b->snwork : (int)std::min(sorted.size(), slots);
     b->slds = lds;
     b->sdepth = depth;
+    b->slanes = lanes;
     b->sL = L;
     b->sV = V;
     b->sR = R;

@@ -55,6 +55,8 @@ struct Tuning {
 struct BlockTuning {
     int L = 0, V = 2, lanes = 64, TYg = 16, kchunk = 64;
     int R = 0;  // > 0: wavefront-strip kernel, R rows per lane, TYg / R wavefronts
+    // strip passes of l steps straight from memory: lanes of a tile row
+    int row_lanes[5] = {64, 64, 64, 64, 64};
 };
 
 inline size_t storage_size(int precision) {
@@ -77,10 +79,9 @@ inline int strip_stage_depth(int L, int V, int R, int W, int Ni, int precision) 
     return 0;
 }
 
-// x geometry of a strip tile: a window of 64*V columns (FP64: 32) with Gx
-// ghost columns on each side (at least L, a multiple of V) and TX stored
-// columns; tiles start at multiples of TX.  With 4-byte storage, TX is a
-// multiple of 16 columns, so every stored row is whole, aligned 64-byte
+// x geometry of a strip tile: a window of lanes*V columns with Gx ghost columns
+// on each side (at least L, a multiple of V) and TX stored columns; tiles start
+// at multiples of TX.  With 4-byte storage, TX is a multiple of 16 columns, so every stored row is whole, aligned 64-byte
 // granules: rows that begin mid-granule are written as 32-byte requests
 // (512^3 FP32 L = 4, staged: 2.01 ms per pass with 56 stored columns, 1.61
 // with 48).  FP64 rows of 24 doubles are whole granules already; FP16 keeps
@@ -90,9 +91,9 @@ inline int strip_stage_depth(int L, int V, int R, int W, int Ni, int precision) 
 // stores save (256-grid batch, both widths for all grids: 236.0 Gcell/s with
 // 56 stored columns, 221.5 with 48).
 // Staged tiles start and end on 16-byte packs: four ghost columns for every L.
-inline void strip_x_geometry(int L, int V, int precision, bool stage, int* Gx, int* TX,
+inline void strip_x_geometry(int L, int V, int precision, bool stage, int lanes, int* Gx, int* TX,
                              bool align = true) {
-    const int RW = fdtd::strip_row_lanes((int)compute_size(precision)) * V;
+    const int RW = lanes * V;
     *Gx = stage ? 4 : (L + V - 1) / V * V;
     *TX = RW - 2 * *Gx;
     if (align && storage_size(precision) == 4) {
@@ -310,6 +311,11 @@ constexpr bool strip_built(int csize, int V, int R) {
 }
 
 fdtd::StripGeom make_strip_geom(const fdtd_grid* g, const BlockTuning& t);
+// Lanes of a tile row of a pass of t.L steps.
+int strip_lanes(const BlockTuning& t, int precision, int depth);
+// What a plane of 32-lane rows costs against one of 64-lane rows (FP64 straight
+// from memory, see strip_direct_lanes).
+double strip_narrow_cost(int L, size_t cells);
 // Probes are recorded by the stepping entry points only.
 bool probing(const fdtd_grid* g);
 fdtd::ProbeArgs probe_args(const fdtd_grid* g);
@@ -327,6 +333,6 @@ fdtd::StripGeom make_pml_strip_geom(const fdtd_grid* g, int kchunk);
 int launch_pml_strip(fdtd_grid* g, bool final, int slot);
 // The batched strip kernel of a shape (null: not built).
 template <typename S>
-const void* batch_strip_kernel(int V, int R, int L, bool final, bool stage, bool first);
+const void* batch_strip_kernel(int V, int R, int L, int lanes, bool final, bool stage, bool first);
 
 }  // namespace fdtd::rt

@@ -2037,8 +2037,8 @@ blocked_sweep(BlockedArgs<S, C> a) {
 // Wavefront-strip temporally blocked sweep: L fused steps per pass over HBM.
 //
 // A workgroup of W wavefronts covers a tile of 64*V columns by W*R rows of
-// every plane (FP64: 32 columns by 2*W*R rows, two row groups of 32 lanes per
-// wavefront).  Lane l of row group w owns columns l*V .. l*V+V-1 of tile
+// every plane (FP64 also 32 columns by 2*W*R rows, two row groups of 32 lanes
+// per wavefront).  Lane l of row group w owns columns l*V .. l*V+V-1 of tile
 // rows w*R .. w*R+R-1 and keeps them in registers, so of the x and y
 // neighbours a cell update reads:
 //   - x: the neighbouring lane's cell, moved by a DPP wavefront shift
@@ -2116,16 +2116,20 @@ struct StripGeom {
     int depth;        // staged path: input planes in LDS (1 or 2)
 };
 
-// Lanes of a tile row.  Float compute: a wavefront is one row group of 64
-// lanes.  Double compute holds twice the register bytes per cell, so a
-// workgroup covers half as many cells; a 64 x 16 tile would store 56 x 8 of
-// them at L = 4 (2.29 cells computed per cell stored), a 32 x 32 tile
+// Lanes of a tile row on the staged path.  Float compute: a wavefront is one
+// row group of 64 lanes.  Double compute holds twice the register bytes per
+// cell, so a workgroup covers half as many cells; a 64 x 16 tile would store 56
+// x 8 of them at L = 4 (2.29 cells computed per cell stored), a 32 x 32 tile
 // stores 24 x 24 (1.78): there a wavefront is two row groups of 32 lanes.
-__host__ __device__ constexpr int strip_row_lanes(int csize) { return csize == 8 ? 32 : 64; }
+// FP64 rows straight from memory take either width (strip_direct_lanes).
+__host__ __device__ constexpr int strip_stage_lanes(int csize) { return csize == 8 ? 32 : 64; }
+__host__ __device__ constexpr bool strip_lanes_built(int csize, bool stage, int lanes) {
+    return stage ? lanes == strip_stage_lanes(csize) : lanes == 64 || (csize == 8 && lanes == 32);
+}
 
 // Tile rows of W wavefronts with R rows per lane.
-__host__ __device__ constexpr int strip_tile_rows(int W, int R, int csize) {
-    return W * R * (64 / strip_row_lanes(csize));
+__host__ __device__ constexpr int strip_tile_rows(int W, int R, int lanes) {
+    return W * R * (64 / lanes);
 }
 
 // LDS of a tile: the row exchange (per buffer two B and two E rows of every
@@ -2138,12 +2142,12 @@ __host__ __device__ inline size_t strip_exchange_bytes(int L, int W, int V, int 
     return static_cast<size_t>(4) * strip_exchange_bufs(L) * W * 64 * V * csize;
 }
 __host__ __device__ constexpr int strip_out_row_bytes(int csize, int ssize) {
-    return (strip_row_lanes(csize) - 8) * ssize;
+    return (strip_stage_lanes(csize) - 8) * ssize;
 }
 __host__ __device__ inline size_t strip_lds_bytes(int L, int W, int V, int R, int csize, int ssize,
                                                   int depth) {
     const size_t plane = static_cast<size_t>(6) * W * 64 * V * R * ssize;
-    const int stored = strip_tile_rows(W, R, csize) - 2 * L;
+    const int stored = strip_tile_rows(W, R, strip_stage_lanes(csize)) - 2 * L;
     return strip_exchange_bytes(L, W, V, csize) + depth * plane +
            (depth > 0 ? static_cast<size_t>(6) * stored * strip_out_row_bytes(csize, ssize) : 0);
 }
@@ -2260,11 +2264,13 @@ __device__ __forceinline__ bool tile_probes(const StripArgs<S, C>& a, int tile) 
 // and the last row group read from memory themselves.
 // RESCALE (FP16 storage only): the pass after an in-run rescaling decision,
 // which scales what it reads.
-template <typename S, typename C, int V, int R, int L, bool FINAL, bool STAGE, bool FIRST = false,
-          bool RESCALE = false, bool PROBE = false>
+// LN: lanes of a tile row.
+template <typename S, typename C, int V, int R, int L, bool FINAL, bool STAGE, int LN,
+          bool FIRST = false, bool RESCALE = false, bool PROBE = false>
 __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int tile,
                                            C* __restrict__ lds) {
     static_assert(!STAGE || strip_stage_built(V, R, L), "staged shape");
+    static_assert(strip_lanes_built(sizeof(C), STAGE, LN), "row width");
     static_assert(!FIRST || (STAGE && !RESCALE), "first passes are staged and rescale nothing");
     const StripGeom& G = a.g;
     const int txy = G.ntx * G.nty;
@@ -2273,7 +2279,6 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
     const int ty = rem / G.ntx;
     const int tx = rem - ty * G.ntx;
 
-    constexpr int LN = strip_row_lanes(sizeof(C));
     constexpr int GPW = 64 / LN;                       // row groups per wavefront
     constexpr int RW = LN * V;                         // tile columns
     const int Ni = G.Ni, Nj = G.Nj, Nk = G.Nk;
@@ -3022,7 +3027,7 @@ __device__ __forceinline__ void strip_tile(const StripArgs<S, C>& a, const int t
 // level's B is held in registers until then: up to 35 more VGPRs, which the
 // plain variant does without).  Tiles without a probe run the plain code in it:
 // 256^3 FP32 with 8 probes, 306 us per pass instead of 337.
-template <typename S, typename C, int V, int R, int L, bool FINAL, bool STAGE, bool FIRST,
+template <typename S, typename C, int V, int R, int L, bool FINAL, bool STAGE, int LN, bool FIRST,
           bool PROBE = false>
 __global__ void __launch_bounds__(strip_max_threads(V, R, L, sizeof(C)))
 strip_sweep(StripArgs<S, C> a) {
@@ -3031,9 +3036,9 @@ strip_sweep(StripArgs<S, C> a) {
     const int tile = (blk & 7) * a.g.per_xcd + (blk >> 3);
     if (tile >= a.g.ntiles) return;  // whole workgroup
     if (PROBE && tile_probes(a, tile))
-        strip_tile<S, C, V, R, L, FINAL, STAGE, FIRST, false, PROBE>(a, tile, reinterpret_cast<C*>(lds_raw));
+        strip_tile<S, C, V, R, L, FINAL, STAGE, LN, FIRST, false, PROBE>(a, tile, reinterpret_cast<C*>(lds_raw));
     else
-        strip_tile<S, C, V, R, L, FINAL, STAGE, FIRST>(a, tile, reinterpret_cast<C*>(lds_raw));
+        strip_tile<S, C, V, R, L, FINAL, STAGE, LN, FIRST>(a, tile, reinterpret_cast<C*>(lds_raw));
 }
 
 // FP16 storage: the strip pass after an in-run rescaling decision, reading
@@ -3047,9 +3052,9 @@ strip_rescale_sweep(StripArgs<S, C> a) {
     const int tile = (blk & 7) * a.g.per_xcd + (blk >> 3);
     if (tile >= a.g.ntiles) return;  // whole workgroup
     if (PROBE && tile_probes(a, tile))
-        strip_tile<S, C, V, R, L, FINAL, STAGE, false, true, PROBE>(a, tile, reinterpret_cast<C*>(lds_raw));
+        strip_tile<S, C, V, R, L, FINAL, STAGE, 64, false, true, PROBE>(a, tile, reinterpret_cast<C*>(lds_raw));
     else
-        strip_tile<S, C, V, R, L, FINAL, STAGE, false, true>(a, tile, reinterpret_cast<C*>(lds_raw));
+        strip_tile<S, C, V, R, L, FINAL, STAGE, 64, false, true>(a, tile, reinterpret_cast<C*>(lds_raw));
 }
 
 // ---------------------------------------------------------------------------
@@ -3232,7 +3237,7 @@ __device__ __forceinline__ StripArgs<S, C> load_batch_strip_grid(cptr<BatchStrip
     return a;
 }
 
-template <typename S, typename C, int V, int R, int L, bool FINAL, bool STAGE, bool FIRST>
+template <typename S, typename C, int V, int R, int L, bool FINAL, bool STAGE, int LN, bool FIRST>
 __global__ void __launch_bounds__(strip_max_threads(V, R, L, sizeof(C)))
 batch_strip_sweep(BatchStripArgs<S, C> a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -3241,7 +3246,7 @@ batch_strip_sweep(BatchStripArgs<S, C> a) {
         const int grid = work[2 * t], tile = work[2 * t + 1];
         const StripArgs<S, C> sa = load_batch_strip_grid<S, C>(as_const(a.grids) + grid, a.parity,
                                                                a.vals, a.vstride);
-        strip_tile<S, C, V, R, L, FINAL, STAGE, FIRST>(sa, tile, reinterpret_cast<C*>(lds_raw));
+        strip_tile<S, C, V, R, L, FINAL, STAGE, LN, FIRST>(sa, tile, reinterpret_cast<C*>(lds_raw));
     };
     if constexpr (STAGE) {
         run(blockIdx.x);

@@ -339,6 +339,11 @@ bool blocked_valid(const fdtd_grid* g, const BlockTuning& t) {
     return true;
 }
 
+int strip_lanes(const BlockTuning& t, int precision, int depth) {
+    const int cs = (int)compute_size(precision);
+    return depth > 0 ? fdtd::strip_stage_lanes(cs) : (cs == 8 ? t.row_lanes[t.L] : 64);
+}
+
 fdtd::StripGeom make_strip_geom(const fdtd_grid* g, const BlockTuning& t) {
     fdtd::StripGeom G;
     G.Ni = g->Ni;
@@ -346,8 +351,9 @@ fdtd::StripGeom make_strip_geom(const fdtd_grid* g, const BlockTuning& t) {
     G.Nk = g->Nk;
     G.W = t.TYg / t.R;
     G.depth = strip_stage_depth(t.L, t.V, t.R, G.W, g->Ni, g->precision);
-    strip_x_geometry(t.L, t.V, g->precision, G.depth > 0, &G.Gx, &G.TX);
-    G.TY = fdtd::strip_tile_rows(G.W, t.R, (int)compute_size(g->precision)) - 2 * t.L;
+    const int lanes = strip_lanes(t, g->precision, G.depth);
+    strip_x_geometry(t.L, t.V, g->precision, G.depth > 0, lanes, &G.Gx, &G.TX);
+    G.TY = fdtd::strip_tile_rows(G.W, t.R, lanes) - 2 * t.L;
     G.kchunk = t.kchunk;
     G.ntx = (g->Ni + G.TX - 1) / G.TX;
     G.nty = (g->Nj + G.TY - 1) / G.TY;
@@ -1070,6 +1076,50 @@ int strip_default_kchunk(const fdtd_grid* g, const BlockTuning& t, long long* pl
     return strip_chunk(g->Nk, nxy, slots, t.L, planes);
 }
 
+// Lanes of a tile row of an FP64 pass of L steps straight from memory, z chunks
+// of kchunk planes (0: the best of either width).  32-lane rows store more of the
+// cells they compute, or fit narrow grids better, and need fewer plane-rounds;
+// but a stored row is then 24 unaligned doubles, and a plane-round takes longer
+// the more of the state comes from memory: 4 steps, us of 32 against 64 lanes,
+// 30 MB of state 3.5 / 3.4, 330 MB 3.9 / 3.5, 780 MB 4.1 / 3.5, 2.6 GB 4.5 / 3.5,
+// 13 GB 5.2 / 3.7; with fewer steps a plane about twice that.  (us per pass,
+// 32 / 64 lanes: 4 steps 301^3 962 / 1072, 65x65x400 80 / 117, 511x301x200 1257 /
+// 1156, 511^3 5371 / 4810; 3 steps 151^3 106 / 117, 511^3 5086 / 3804; 2 steps
+// 401^3 2123 / 1446.)
+double strip_narrow_cost(int L, size_t cells) {
+    return 1.0 + (L == 4 ? 0.045 : 0.08) * std::max(0.0, std::log2(96.0 * cells / 50e6));
+}
+
+int strip_direct_lanes(const fdtd_grid* g, const BlockTuning& t, int L, int kchunk) {
+    const int W = t.TYg / t.R;
+    if (g->precision != FDTD_FP64 || strip_stage_depth(L, t.V, t.R, W, g->Ni, g->precision) > 0) return 64;
+    const long long slots = (long long)std::max(1, 8 / W) * device_cus();
+    double cost[2];
+    for (int q = 0; q < 2; ++q) {
+        const int lanes = q ? 32 : 64;
+        int Gx, TX;
+        strip_x_geometry(L, t.V, g->precision, false, lanes, &Gx, &TX);
+        const int TY = fdtd::strip_tile_rows(W, t.R, lanes) - 2 * L;
+        const long long nxy = (long long)((g->Ni + TX - 1) / TX) * ((g->Nj + TY - 1) / TY);
+        long long planes = 0;
+        if (kchunk > 0)
+            planes = (nxy * ((g->Nk + kchunk - 1) / kchunk) + slots - 1) / slots * (kchunk + 2 * L - 1);
+        else
+            strip_chunk(g->Nk, nxy, slots, L, &planes);
+        cost[q] = planes * (q ? strip_narrow_cost(L, g->N) : 1.0);
+    }
+    return cost[1] < cost[0] ? 32 : 64;
+}
+
+// A valid strip shape's row widths (its own, and those of the shorter passes
+// that take the steps left over) and z chunk (kchunk, or 0: the best).
+void plan_strips(const fdtd_grid* g, BlockTuning* t, int kchunk, long long* planes = nullptr) {
+    t->row_lanes[t->L] = strip_direct_lanes(g, *t, t->L, kchunk);
+    t->kchunk = kchunk > 0 ? kchunk : strip_default_kchunk(g, *t, planes);
+    for (int l = 1; l < t->L; ++l)
+        if (t->TYg > 2 * l) t->row_lanes[l] = strip_direct_lanes(g, *t, l, t->kchunk);
+}
+
 // Whether strip passes of t.L steps beat as many single sweeps on a grid, by
 // what both cost on grids that fit the caches: a plane-round of a pass about
 // 3.3 us (FP64 W = 8, FP32 W = 16), a sweep 5 us up to 26 MB of E and B read
@@ -1713,7 +1763,7 @@ int create_grid(const fdtd_parameters* p, double dt, double pml_percent, int pre
         t.kchunk = 1;
         if (strip_valid(g, t)) {
             long long planes = 0;
-            t.kchunk = strip_default_kchunk(g, t, &planes);
+            plan_strips(g, &t, 0, &planes);
             if (wide || strips_pay(g, t, planes)) g->btune = t;
         }
     }
@@ -2776,7 +2826,7 @@ int fdtd_set_time_blocking_strips(fdtd_grid* g, int L, int V, int R, int W, int 
     if (!strip_valid(g, t))
         return fail(FDTD_ERR_INVALID_ARGUMENT, "strip blocking L=%d V=%d R=%d W=%d invalid for this grid",
                     t.L, t.V, t.R, t.TYg / t.R);
-    t.kchunk = kchunk > 0 ? kchunk : strip_default_kchunk(g, t);
+    plan_strips(g, &t, kchunk);
     g->btune = t;
     return FDTD_OK;
 }
@@ -2908,7 +2958,10 @@ int fdtd_get_time_blocking(const fdtd_grid* g, int out[5]) {
     if (!g || !out) return fail(FDTD_ERR_INVALID_ARGUMENT, "null argument");
     out[0] = g->btune.L;
     out[1] = g->btune.V;
-    out[2] = g->btune.lanes;
+    // (strip passes: the lanes of a tile row)
+    out[2] = g->btune.L > 0 && g->btune.R > 0
+                 ? strip_lanes(g->btune, g->precision, make_strip_geom(g, g->btune).depth)
+                 : g->btune.lanes;
     out[3] = g->btune.TYg;
     out[4] = g->btune.kchunk;
     return FDTD_OK;

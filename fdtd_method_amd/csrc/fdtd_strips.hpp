@@ -13,11 +13,11 @@ namespace fdtd::rt {
 // run's first half step).  FP16: the pass
 // after an in-run rescaling decision scales its reads; passes of a run with
 // probes record them.
-template <typename S, int V, int R, int L, bool FINAL, bool STAGE, bool FIRST>
+template <typename S, int V, int R, int L, bool FINAL, bool STAGE, int LN, bool FIRST>
 auto strip_kernel(bool rescale, bool probe) {
     using C = typename fdtd::ComputeOf<S>::type;
-    auto kern = probe ? fdtd::strip_sweep<S, C, V, R, L, FINAL, STAGE, FIRST, true>
-                      : fdtd::strip_sweep<S, C, V, R, L, FINAL, STAGE, FIRST, false>;
+    auto kern = probe ? fdtd::strip_sweep<S, C, V, R, L, FINAL, STAGE, LN, FIRST, true>
+                      : fdtd::strip_sweep<S, C, V, R, L, FINAL, STAGE, LN, FIRST, false>;
     if constexpr (sizeof(S) == 2 && !FIRST)
         if (rescale)
             kern = probe ? fdtd::strip_rescale_sweep<S, C, V, R, L, FINAL, STAGE, true>
@@ -48,11 +48,15 @@ int launch_strip_v(fdtd_grid* g, bool first, int slot, int in, int out, void* co
         a.g = make_strip_geom(g, t);
         for (int c = 0; c < 6; ++c) a.iscale[c] = g->pass_iscale[c];
         a.probe = probe_args(g);
-        auto kern = strip_kernel<S, V, R, L, FINAL, false, false>(g->pass_rescale, probing(g));
+        constexpr int SL = fdtd::strip_stage_lanes(sizeof(C));
+        auto kern = strip_kernel<S, V, R, L, FINAL, false, 64, false>(g->pass_rescale, probing(g));
+        if constexpr (sizeof(C) == 8)
+            if (strip_lanes(t, g->precision, a.g.depth) == 32)
+                kern = strip_kernel<S, V, R, L, FINAL, false, 32, false>(false, probing(g));
         if constexpr (fdtd::strip_stage_built(V, R, L))
             if (a.g.depth > 0)
-                kern = first ? strip_kernel<S, V, R, L, FINAL, true, true>(false, probing(g))
-                             : strip_kernel<S, V, R, L, FINAL, true, false>(g->pass_rescale, probing(g));
+                kern = first ? strip_kernel<S, V, R, L, FINAL, true, SL, true>(false, probing(g))
+                             : strip_kernel<S, V, R, L, FINAL, true, SL, false>(g->pass_rescale, probing(g));
         const size_t lds = fdtd::strip_lds_bytes(L, a.g.W, V, R, sizeof(C), sizeof(S), a.g.depth);
         if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
         hipLaunchKernelGGL(kern, dim3(8 * a.g.per_xcd), dim3(64 * a.g.W), lds, g->stream, a);
@@ -64,14 +68,17 @@ int launch_strip_v(fdtd_grid* g, bool first, int slot, int in, int out, void* co
 
 // Workgroups of a strip variant resident per CU (0 if it cannot launch).
 template <typename S, int V, int R, int L>
-int strip_occupancy_v(int W, int depth) {
+int strip_occupancy_v(int W, int depth, int lanes) {
     using C = typename fdtd::ComputeOf<S>::type;
     if constexpr (!strip_built(sizeof(C), V, R)) {
         return 0;
     } else {
-        auto kern = fdtd::strip_sweep<S, C, V, R, L, false, false, false>;
+        auto kern = fdtd::strip_sweep<S, C, V, R, L, false, false, 64, false>;
+        if constexpr (sizeof(C) == 8)
+            if (lanes == 32) kern = fdtd::strip_sweep<S, C, V, R, L, false, false, 32, false>;
         if constexpr (fdtd::strip_stage_built(V, R, L))
-            if (depth > 0) kern = fdtd::strip_sweep<S, C, V, R, L, false, true, false>;
+            if (depth > 0)
+                kern = fdtd::strip_sweep<S, C, V, R, L, false, true, fdtd::strip_stage_lanes(sizeof(C)), false>;
         const size_t lds = fdtd::strip_lds_bytes(L, W, V, R, sizeof(C), sizeof(S), depth);
         if (allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds) != FDTD_OK) return 0;
         int n = 0;
@@ -84,21 +91,21 @@ int strip_occupancy_v(int W, int depth) {
 }
 
 template <typename S, int V, int R>
-int strip_occupancy_l(int L, int W, int depth) {
+int strip_occupancy_l(int L, int W, int depth, int lanes) {
     switch (L) {
-        case 1: return strip_occupancy_v<S, V, R, 1>(W, depth);
-        case 2: return strip_occupancy_v<S, V, R, 2>(W, depth);
-        case 3: return strip_occupancy_v<S, V, R, 3>(W, depth);
-        default: return strip_occupancy_v<S, V, R, 4>(W, depth);
+        case 1: return strip_occupancy_v<S, V, R, 1>(W, depth, lanes);
+        case 2: return strip_occupancy_v<S, V, R, 2>(W, depth, lanes);
+        case 3: return strip_occupancy_v<S, V, R, 3>(W, depth, lanes);
+        default: return strip_occupancy_v<S, V, R, 4>(W, depth, lanes);
     }
 }
 
 template <typename S>
 int strip_occupancy_s(const BlockTuning& t, int depth) {
-    const int W = t.TYg / t.R;
-    if (t.V == 1 && t.R == 2) return strip_occupancy_l<S, 1, 2>(t.L, W, depth);
-    if (t.V == 1 && t.R == 4) return strip_occupancy_l<S, 1, 4>(t.L, W, depth);
-    if (t.V == 2 && t.R == 2) return strip_occupancy_l<S, 2, 2>(t.L, W, depth);
+    const int W = t.TYg / t.R, lanes = t.row_lanes[t.L];
+    if (t.V == 1 && t.R == 2) return strip_occupancy_l<S, 1, 2>(t.L, W, depth, lanes);
+    if (t.V == 1 && t.R == 4) return strip_occupancy_l<S, 1, 4>(t.L, W, depth, lanes);
+    if (t.V == 2 && t.R == 2) return strip_occupancy_l<S, 2, 2>(t.L, W, depth, lanes);
     return 0;
 }
 
@@ -126,35 +133,39 @@ int launch_strip_f(fdtd_grid* g, bool first, int slot, int in, int out, void* co
 
 // The batched strip kernel of a shape (null: not built).
 template <typename S, int V, int R, int L, bool FINAL>
-const void* batch_strip_kernel_v(bool stage, bool first) {
+const void* batch_strip_kernel_v(int lanes, bool stage, bool first) {
     using C = typename fdtd::ComputeOf<S>::type;
     if constexpr (!strip_built(sizeof(C), V, R)) {
         return nullptr;
     } else {
         if constexpr (fdtd::strip_stage_built(V, R, L)) {
+            constexpr int SL = fdtd::strip_stage_lanes(sizeof(C));
             if (stage)
-                return first ? reinterpret_cast<const void*>(fdtd::batch_strip_sweep<S, C, V, R, L, FINAL, true, true>)
-                             : reinterpret_cast<const void*>(fdtd::batch_strip_sweep<S, C, V, R, L, FINAL, true, false>);
+                return first ? reinterpret_cast<const void*>(fdtd::batch_strip_sweep<S, C, V, R, L, FINAL, true, SL, true>)
+                             : reinterpret_cast<const void*>(fdtd::batch_strip_sweep<S, C, V, R, L, FINAL, true, SL, false>);
         }
-        return reinterpret_cast<const void*>(fdtd::batch_strip_sweep<S, C, V, R, L, FINAL, false, false>);
+        if constexpr (sizeof(C) == 8)
+            if (lanes == 32)
+                return reinterpret_cast<const void*>(fdtd::batch_strip_sweep<S, C, V, R, L, FINAL, false, 32, false>);
+        return reinterpret_cast<const void*>(fdtd::batch_strip_sweep<S, C, V, R, L, FINAL, false, 64, false>);
     }
 }
 
 template <typename S, int V, int R, bool FINAL>
-const void* batch_strip_kernel_l(int L, bool stage, bool first) {
+const void* batch_strip_kernel_l(int L, int lanes, bool stage, bool first) {
     switch (L) {
-        case 1: return batch_strip_kernel_v<S, V, R, 1, FINAL>(stage, first);
-        case 2: return batch_strip_kernel_v<S, V, R, 2, FINAL>(stage, first);
-        case 3: return batch_strip_kernel_v<S, V, R, 3, FINAL>(stage, first);
-        default: return batch_strip_kernel_v<S, V, R, 4, FINAL>(stage, first);
+        case 1: return batch_strip_kernel_v<S, V, R, 1, FINAL>(lanes, stage, first);
+        case 2: return batch_strip_kernel_v<S, V, R, 2, FINAL>(lanes, stage, first);
+        case 3: return batch_strip_kernel_v<S, V, R, 3, FINAL>(lanes, stage, first);
+        default: return batch_strip_kernel_v<S, V, R, 4, FINAL>(lanes, stage, first);
     }
 }
 
 template <typename S, bool FINAL>
-const void* batch_strip_kernel_s(int V, int R, int L, bool stage, bool first) {
-    if (V == 1 && R == 2) return batch_strip_kernel_l<S, 1, 2, FINAL>(L, stage, first);
-    if (V == 1 && R == 4) return batch_strip_kernel_l<S, 1, 4, FINAL>(L, stage, first);
-    if (V == 2 && R == 2) return batch_strip_kernel_l<S, 2, 2, FINAL>(L, stage, first);
+const void* batch_strip_kernel_s(int V, int R, int L, int lanes, bool stage, bool first) {
+    if (V == 1 && R == 2) return batch_strip_kernel_l<S, 1, 2, FINAL>(L, lanes, stage, first);
+    if (V == 1 && R == 4) return batch_strip_kernel_l<S, 1, 4, FINAL>(L, lanes, stage, first);
+    if (V == 2 && R == 2) return batch_strip_kernel_l<S, 2, 2, FINAL>(L, lanes, stage, first);
     return nullptr;
 }
 
@@ -166,9 +177,9 @@ int launch_strip(fdtd_grid* g, bool final, bool first, int slot, int in, int out
 }
 
 template <typename S>
-const void* batch_strip_kernel(int V, int R, int L, bool final, bool stage, bool first) {
-    return final ? batch_strip_kernel_s<S, true>(V, R, L, stage, first)
-                 : batch_strip_kernel_s<S, false>(V, R, L, stage, first);
+const void* batch_strip_kernel(int V, int R, int L, int lanes, bool final, bool stage, bool first) {
+    return final ? batch_strip_kernel_s<S, true>(V, R, L, lanes, stage, first)
+                 : batch_strip_kernel_s<S, false>(V, R, L, lanes, stage, first);
 }
 
 }  // namespace fdtd::rt

@@ -280,3 +280,46 @@ def test_default_z_chunk_marches_few_planes_twice(prec, L):
     g.set_time_blocking_strips(L, 1, 2, 8 if prec == Precision.FP64 else 16)
     assert g.get_time_blocking_strips()["kchunk"] >= 2 * (2 * L - 1)
     g.close()
+
+
+@pytest.mark.parametrize("shape,L,lanes", [
+    ((25, 24, 2000), 4, 32),   # one column more than a 32-lane tile stores
+    ((23, 25, 2000), 4, 32),   # one row more
+    ((47, 47, 1200), 4, 32),
+    ((71, 23, 1500), 4, 32),
+    ((25, 25, 2000), 4, 64),
+    ((57, 8, 300), 4, 64),     # one column more than a 64-lane tile stores
+    ((55, 9, 300), 4, 64),
+    ((27, 26, 1800), 3, 32),
+    ((59, 11, 40), 3, 64),
+    ((29, 28, 1800), 2, 32),
+    ((61, 13, 40), 2, 64),
+    ((31, 30, 1500), 1, 32),
+    ((63, 15, 40), 1, 64),
+])
+def test_fp64_row_widths(shape, L, lanes):
+    """FP64 rows that cannot be staged: tiles of 32 or 64 columns, whichever
+    needs fewer plane-rounds, around the tiles' edges, with the shorter passes
+    that take the steps left over: the same bits as single sweeps."""
+    n, dt = int(np.prod(shape)), courant_dt(1, 1, 1, factor=0.5)
+    a, b = (FDTD(Parameters(*shape), dt, Precision.FP64) for _ in range(2))
+    for c, v in enumerate(random_state(n, 17)):
+        for g in (a, b):
+            g.upload(c, v)
+    for g in (a, b):
+        g.set_point_sources([dict(i=shape[0] - 1, j=q % shape[1], k=(7 * q) % shape[2], comp=q % 3,
+                                  kind=0, amp=0.2 / dt) for q in range(70)])
+        g.set_probes([(0, 0, 0, 0), (shape[0] - 1, shape[1] - 1, shape[2] - 1, 5)], 4 * L + 6)
+    a.set_time_blocking_strips(0)
+    b.set_time_blocking_strips(L, 1, 2, 8)
+    assert b.get_time_blocking()["lanes"] == lanes
+    for steps in (2 * L, L + 2, L + 3):
+        a.update_fields(steps)
+        b.update_fields(steps)
+        assert a.checksum() == b.checksum(), steps
+        if steps == L + 2:
+            for g in (a, b):
+                g.rewind_records()
+    assert np.array_equal(a.read_probes(), b.read_probes())
+    a.close()
+    b.close()
