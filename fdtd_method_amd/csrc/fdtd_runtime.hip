@@ -1215,13 +1215,24 @@ void trace_end(fdtd_grid* g, hipEvent_t a, int kind, bool pass) {
     g->trace->recs.push_back({kind, a, e});
 }
 
+// Whether a pass takes the l (2 or 3) steps left over faster than single sweeps.
+// A pass takes about as long with fewer levels, FP64 and FP32 because memory
+// bounds it, FP16 because its planes' latency does; FP16 sweeps of whole 4-cell
+// lanes move so little that two of them cost less from the size of the last-level
+// cache on (us, sweeps / pass: two steps 128^3 37 / 31, 256^3 189 / 202, 320^3 334
+// / 415, 512^3 1270 / 2036; three steps 256^3 283 / 200, 512^3 1905 / 2102, 640^3
+// 4143 / 3935; rows of single-cell lanes, two steps 401^3 1442 / 842).
+bool tail_pass_pays(const fdtd_grid* g, int l) {
+    const double mb = 12e-6 * g->N * g->esize;
+    return g->precision != FDTD_FP16 || g->Ni % 4 != 0 || l != 2 || mb <= 256.0;
+}
+
 // n steps with temporal blocking: B/2 (or, for strip passes, the carried
 // half step), then n / L blocked passes, then the remaining n % L steps: two
-// or three as one strip pass of that many levels, one (or those after patch
-// passes) as single fused sweeps.  A strip pass takes about as long with fewer
-// levels, since memory bounds it, so it is the cheaper form from two steps on
-// (ms, pass against sweeps: 512^3 FP32, two steps 1.67 / 2.3, three 1.78 / 3.5;
-// FP64 3.3 / 5.3, 3.7 / 8.0; 251x190x131 FP32 0.099 / 0.173, 0.120 / 0.25).
+// or three as one strip pass of that many levels where that pays
+// (tail_pass_pays; ms, pass against sweeps: 512^3 FP32, two steps 1.67 / 2.3,
+// three 1.78 / 3.5; FP64 3.3 / 5.3, 3.7 / 8.0; 251x190x131 FP32 0.099 / 0.173,
+// 0.120 / 0.25), else, or after patch passes, as single fused sweeps.
 // Source tables are filled in whole passes.  Strip
 // passes that stage two planes in LDS take B/2 in their first pass; for them
 // a carried half step is no cheaper than the half step itself (512^3 FP32:
@@ -1253,7 +1264,7 @@ int run_blocked(fdtd_grid* g, int nsteps, hipEvent_t mid) {
     const int npass = nsteps / L;
     BlockTuning tail = g->btune;  // the pass of the steps left over
     tail.L = nsteps % L;
-    const bool use_tail = strips && tail.L >= 2 && strip_valid(g, tail);
+    const bool use_tail = strips && tail.L >= 2 && tail_pass_pays(g, tail.L) && strip_valid(g, tail);
     const int rem = use_tail ? 0 : nsteps % L;
     const int blocked = nsteps - rem;
     const int chunk = (kValTable / L) * L;

@@ -69,3 +69,24 @@ def test_default_of_narrow_grids(prec, shape, blocked):
         assert a.checksum() == b.checksum(), n
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("prec,shape,n,sweeps", [
+    (FP16, (256, 256, 192), 6, 2),   # beyond the last-level cache: two sweeps
+    (FP16, (256, 256, 192), 7, 1),   # three steps: a pass
+    (FP16, (128, 128, 64), 6, 1),
+    (FP16, (257, 256, 192), 6, 1),   # single-cell lanes
+    (FP32, (256, 256, 128), 6, 1),
+    (FP64, (256, 128, 128), 6, 1),
+])
+def test_form_of_the_steps_left_over(prec, shape, n, sweeps):
+    a, b = make(shape, prec), make(shape, prec)
+    a.set_time_blocking_strips(0)
+    for _ in range(2):
+        a.update_fields(n)
+        b.update_fields(n)
+        assert a.checksum() == b.checksum()
+    s = b.launch_stats()
+    assert (s["passes"], s["sweeps"]) == (2, 2 * sweeps)
+    a.close()
+    b.close()
