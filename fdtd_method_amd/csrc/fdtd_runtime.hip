@@ -1238,7 +1238,9 @@ bool tail_pass_pays(const fdtd_grid* g, int l) {
 // a carried half step is no cheaper than the half step itself (512^3 FP32:
 // either makes one pass 0.3 ms longer; the carry also holds three fields
 // twice and is lost whenever the caller touches E or B), so FP64 and FP32
-// runs leave none.  Others carry the next
+// runs leave none unless they found one: a call of one step left it, and the
+// next such call would start with a sweep over E and B instead (512^3 FP32, calls
+// of four steps and of one in turn: 4.07 ms, with the carry 3.43).  Others carry the next
 // half step out of their last pass or sweep, as the unblocked path does; so
 // does FP16, where the carried value (rounded once) is not the half step from
 // the stored B.
@@ -1256,8 +1258,8 @@ int run_blocked(fdtd_grid* g, int nsteps, hipEvent_t mid) {
         trace_end(g, t0, 0, false);
     }
     if (rc) return rc;
-    const bool carry_out = strips && g->carry && (!own_half || g->precision == FDTD_FP16) &&
-                           ensure_carry(g);
+    const bool carry_out = strips && g->carry &&
+                           (!own_half || g->precision == FDTD_FP16 || carried >= 0) && ensure_carry(g);
     const int ahead_buf = carried < 0 ? 0 : 1 - carried;
     if (mid) HIP_TRY(hipEventRecord(mid, g->stream));
     const int L = g->btune.L;

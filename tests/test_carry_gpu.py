@@ -119,3 +119,25 @@ def test_host_writes_scales_and_batches_drop_the_carried_step():
     rel = np.sqrt(sum(e[0] for e in err) / sum(e[1] for e in err))
     print("fp16 after a scale change: relL2 vs FP64", rel)
     assert rel < 5e-3
+
+
+@pytest.mark.parametrize("prec,shape", [
+    (Precision.FP64, (128, 64, 32)), (Precision.FP32, (128, 66, 33)),
+    (Precision.FP32, (127, 66, 33)), (Precision.FP16, (128, 64, 32))])
+def test_calls_of_one_step_between_passes_keep_the_carry(prec, shape):
+    """Calls of one step and of whole passes in turn: only the first call
+    takes a B half step of its own (FP64 and FP32 passes leave the next one
+    when they found one)."""
+    n, dt = int(np.prod(shape)), courant_dt(1, 1, 1, factor=0.5)
+    a, b = (FDTD(Parameters(*shape), dt, prec) for _ in range(2))
+    for c, v in enumerate(random_state(n, 23)):
+        for g in (a, b):
+            g.upload(c, v)
+    a.set_time_blocking_strips(0)
+    for steps in (1, 4, 1, 6, 1, 5, 1, 1, 4, 4, 1):
+        a.update_fields(steps)
+        b.update_fields(steps)
+        assert a.checksum() == b.checksum(), steps
+    assert b.launch_stats()["prologues"] == 1
+    a.close()
+    b.close()
