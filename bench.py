@@ -517,10 +517,10 @@ def pml_bytes_per_step(shape, widths, word, steps_per_launch=1):
 
 
 def bench_pml(a):
-    """The PML workload on both PML step forms: the two in-place phase sweeps
-    per step (pml_e_phase, pml_b_phase) and the fused form, which takes strip
-    passes of two steps where the grid runs them, else the fused PML sweep.
-    `value` is the grid's default form in FP32."""
+    """The PML workload on the PML step forms: the two in-place phase sweeps per
+    step (pml_e_phase, pml_b_phase), the autotuned fused PML sweep on every step,
+    and the default, which takes strip passes of two steps where the grid runs
+    them.  `value` is the grid's default form in FP32."""
     from fdtd_method_amd import FDTD_PML
     n, K, pml = a.n, a.steps, a.pml
     dt = 0.5 / (C * np.sqrt(3.0))
@@ -533,8 +533,8 @@ def bench_pml(a):
         g.set_point_sources([src])
         if form == "phases":
             g.set_pml_path(1)
-        if form == "fused":
-            g.set_pml_path(0)
+        if form in ("sweeps", "fused"):
+            g.set_pml_path(2 if form == "sweeps" else 0)
             if a.tuning:
                 g.set_tuning(*[int(x) for x in a.tuning.split(",")])
             else:
@@ -564,7 +564,7 @@ def bench_pml(a):
     res = {}
     grids = {}
     for prec in (Precision.FP32, Precision.FP64):
-        for form in ("phases", "fused"):
+        for form in ("phases", "sweeps", "fused"):
             g = make(prec, form)
             r = run_path(g, K, a.warmup)
             spl = 2 if g.launch_stats()["passes"] else 1
@@ -574,8 +574,9 @@ def bench_pml(a):
             rec = dict(gcells=r["gcells"], ms_per_step=r["ms_per_step"], steps_per_launch=spl,
                        step_kernel_ms=step_ms, alg_bytes_per_step=nbytes,
                        alg_gbs=gbs, frac_of_peak=gbs / PEAK_GBS)
-            if form == "fused":
-                rec["launch_shape"] = g.get_tuning()
+            if form != "phases":
+                if spl == 1:  # (passes have no launch shape)
+                    rec["launch_shape"] = g.get_tuning()
             else:
                 rec["phase_shape"] = g.get_pml_path()
                 # the phases read E and B of main cells once more per step
@@ -645,7 +646,7 @@ def main():
     ap.add_argument("--workload", choices=["point", "batch", "precision", "blocked", "pml"],
                     default="point")
     ap.add_argument("--pml", type=float, default=0.2, help="pml_percent of --workload pml")
-    ap.add_argument("--pml-form", choices=["phases", "fused"], default=None,
+    ap.add_argument("--pml-form", choices=["phases", "sweeps", "fused"], default=None,
                     help="PML step form for --workload pml --profile (default: the grid's)")
     ap.add_argument("--dims", default="1024,1024,256", help="grid of --workload blocked")
     ap.add_argument("--grids", type=int, default=256)

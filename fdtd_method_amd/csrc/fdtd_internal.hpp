@@ -196,8 +196,9 @@ struct fdtd_grid {
     size_t split_stride = 0;
     int pml_strip_kchunk = 0;   // z chunk of a PML strip pass; 0: the grid runs none
     void* pml_tab = nullptr;    // per-axis decay/coefficient tables (compute type)
-    // PML steps: 0 = the fused PML sweep (shape tune); 1 = the two in-place
-    // phase sweeps (pml_e_phase, pml_b_phase) with launch shape ptune.  FP16
+    // PML steps: 0 = strip passes where the grid runs them, else the fused PML
+    // sweep (shape tune); 1 = the two in-place phase sweeps (pml_e_phase,
+    // pml_b_phase) with launch shape ptune; 2 = the fused PML sweep.  FP16
     // sweeps that rescale or track the max take the fused sweep either way.
     int pml_path = 0;
     fdtd::rt::Tuning ptune;

@@ -2845,10 +2845,10 @@ int fdtd_set_time_blocking_strips(fdtd_grid* g, int L, int V, int R, int W, int 
 }
 
 int fdtd_set_pml_path(fdtd_grid* g, int path, int V, int TY, int kchunk) {
-    if (!g || (path != 0 && path != 1)) return fail(FDTD_ERR_INVALID_ARGUMENT, "invalid argument");
+    if (!g || path < 0 || path > 2) return fail(FDTD_ERR_INVALID_ARGUMENT, "invalid argument");
     if (!g->pml) return fail(FDTD_ERR_UNSUPPORTED, "the grid has no PML layer");
-    if (path == 0) {
-        g->pml_path = 0;
+    if (path != 1) {
+        g->pml_path = path;
         return FDTD_OK;
     }
     Tuning t = pml_phase_default(g);

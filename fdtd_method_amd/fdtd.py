@@ -575,7 +575,9 @@ class FDTD_PML(FDTD):
         return tuple(w)
 
     def set_pml_path(self, path: int, V: int = 0, TY: int = 0, kchunk: int = 0) -> None:
-        """0: the fused PML sweep (default); 1: two in-place phase sweeps per step."""
+        """0: the fused PML sweep, or strip passes of two steps where they pay
+        (default); 1: two in-place phase sweeps per step; 2: the fused PML sweep
+        on every step."""
         _lib.check(self._L.fdtd_set_pml_path(self._h, int(path), int(V), int(TY), int(kchunk)))
 
     def get_pml_path(self):

@@ -105,12 +105,13 @@ int fdtd_create_pml(const fdtd_parameters* params, double dt, double pml_percent
 /* How a PML grid's fused steps run (no counterpart in the reference, whose
  * step is FDTD_PML.cpp:343-365): path 0 (the default) as the single fused
  * PML sweep (shape: fdtd_set_tuning) or, on FP64 and FP32 grids of more than
- * about 50 MB of state and with no dense J, two steps to a strip pass (same
- * bits; 512^3 FP32 with a 0.2 layer 1.7 ms per step); path 1 as two in-place sweeps per
- * step, an E phase and a B phase, with V cells per lane, TY full rows per
- * workgroup and kchunk planes per z chunk (0: defaults; V*storage bytes at
+ * about 50 MB of state, with no dense J and no probes, two steps to a strip pass
+ * (same bits; 512^3 FP32 with a 0.2 layer 1.7 ms per step; fdtd_get_stats counts
+ * the passes); path 2 as the fused sweep on every step; path 1 as two in-place
+ * sweeps per step, an E phase and a B phase, with V cells per lane, TY full rows
+ * per workgroup and kchunk planes per z chunk (0: defaults; V*storage bytes at
  * most 16).  At 512^3 with a 0.2 layer the phases take 3.94 ms per FP32
- * step against the fused sweep's 3.56 (FP64: 7.51 both).  FP64
+ * step against the fused sweep's 3.2 (FP64: 7.5 and 7.4).  FP64
  * and FP32 results are bit-identical either way (and FP64 to the
  * reference); with FP16 storage the phase path's B update reads E as
  * stored where the fused sweep uses it before rounding, so the two agree
@@ -341,7 +342,10 @@ int fdtd_set_step_carry(fdtd_grid* grid, int enable);
 
 /* Fused-sweep launch shape: V cells per lane along x, TY rows per tile,
  * kchunk planes per z chunk (0 = keep current).  fdtd_autotune times the
- * candidate shapes on scratch buffers and keeps the fastest. */
+ * candidate shapes on scratch buffers and keeps the fastest (best_ms: ms per
+ * sweep).  Runs of strip passes use it for the steps outside the passes only:
+ * fdtd_set_time_blocking_strips(grid, 0, ...) or, with a PML layer,
+ * fdtd_set_pml_path(grid, 2, ...) runs every step as a sweep of this shape. */
 int fdtd_set_tuning(fdtd_grid* grid, int V, int TY, int kchunk);
 int fdtd_get_tuning(const fdtd_grid* grid, int out[3]);
 int fdtd_autotune(fdtd_grid* grid, int reps, int out[3], float* best_ms);

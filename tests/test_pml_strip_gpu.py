@@ -60,3 +60,27 @@ def test_more_steps_than_a_table_of_source_values():
     b.update_fields(523)
     assert a.checksum() == b.checksum()
     assert b.launch_stats()["passes"] == 261
+
+
+@pytest.mark.parametrize("prec", [FP64, FP32])
+def test_path_2_runs_every_step_as_a_sweep(prec):
+    """set_pml_path(2) turns the passes off, 0 on again: the same bits, and the
+    sweeps take the shape that set_tuning gives."""
+    a, b = make((96, 90, 100), prec, 0.2), make((96, 90, 100), prec, 0.2)
+    passes = 0
+    for path, n in ((2, 6), (0, 4), (2, 5), (1, 3), (0, 6)):
+        b.set_pml_path(path)
+        assert b.get_pml_path()["path"] == path
+        if path == 2:
+            b.set_tuning(1, 5, 7)
+        a.update_fields(n)
+        b.update_fields(n)
+        assert a.checksum() == b.checksum(), (path, n)
+        passes += n // 2 if path == 0 else 0
+        assert b.launch_stats()["passes"] == passes
+    for q in range(12):
+        assert np.array_equal(a.split(q), b.split(q)), q
+    with pytest.raises(Exception):
+        b.set_pml_path(3)
+    a.close()
+    b.close()
