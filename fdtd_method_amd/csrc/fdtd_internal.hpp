@@ -294,7 +294,7 @@ int allow_dynamic_lds(const void* kernel, size_t bytes);
 int grid_blocks(size_t n);
 int max_threads(const fdtd_grid* g, int V);
 int default_kchunk(int Nj, int Nk, int TY);
-int strip_chunk(int Nk, long long nxy, long long slots, int L, long long* planes);
+int strip_chunk(int Nk, long long nxy, long long slots, int fill, long long* planes);
 int device_cus();
 // Sparse J values (as kind-0 sources) followed by the waveform sources.
 std::vector<fdtd::PointSource> host_sources(const fdtd_grid* g);

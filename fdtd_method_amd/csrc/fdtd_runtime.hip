@@ -493,14 +493,11 @@ int box_update(fdtd_grid* g, const fdtd::Box& box, bool e_step) {
 }
 
 // Chunk of Nk planes with the fewest plane-rounds (planes, when set) for nxy
-// tiles a chunk and `slots` workgroups at a time (see strip_default_kchunk).
-// A chunk of kc planes is marched in kc + 2L-1: the one below it gives the
-// first plane its B, and each of the L levels ends one plane further on.  (Not
-// counted for L = 1, that plane made chunks of one plane look free: 256^3, us a
-// step FP32 326 instead of 225, FP16 261 instead of 144.)
+// tiles a chunk, `slots` workgroups at a time and `fill` planes marched besides a
+// chunk's own (see strip_default_kchunk).
 // Beyond 64 rounds shorter chunks only add planes, so a grid of millions of
 // planes is not searched through.
-int strip_chunk(int Nk, long long nxy, long long slots, int L, long long* planes) {
+int strip_chunk(int Nk, long long nxy, long long slots, int fill, long long* planes) {
     const int most = static_cast<int>(std::min<long long>(Nk, 64 + 64 * slots / std::max(1LL, nxy)));
     long long best_cost = -1;
     int best = Nk;
@@ -508,7 +505,7 @@ int strip_chunk(int Nk, long long nxy, long long slots, int L, long long* planes
         const int kc = (Nk + nchunk - 1) / nchunk;
         const int nc = (Nk + kc - 1) / kc;
         const long long rounds = (nxy * nc + slots - 1) / slots;
-        const long long cost = rounds * (kc + 2 * L - 1);
+        const long long cost = rounds * (kc + fill);
         if (best_cost < 0 || cost < best_cost) {
             best_cost = cost;
             best = kc;
@@ -599,9 +596,11 @@ fdtd::StripGeom make_pml_strip_geom(const fdtd_grid* g, int kchunk) {
 }
 
 // z chunk of a PML grid's strip passes, the one with the fewest plane-rounds; 0
-// where two fused sweeps cost less.  A pass of few planes takes 0.5 us and 6.5 us
-// a plane-round, two sweeps 24 us up to 26 MB (24 words a cell), beyond that 22
-// us and 0.45 us a MB (us, pass against sweeps: FP64 64^3 45 / 43, 80^3 47 / 66,
+// where two fused sweeps cost less.  (The plane below a chunk is not counted
+// here: counted, it makes one chunk of all planes the choice at 512^3 FP32, where
+// neighbouring tiles drift apart: 4.43 ms a pass, with chunks of 37 planes 3.36.)
+// A pass of few planes takes 7 us and 6.5 us a plane-round, two sweeps 24 us up
+// to 26 MB (24 words a cell), beyond that 22 us and 0.45 us a MB (us, pass against sweeps: FP64 64^3 45 / 43, 80^3 47 / 66,
 // 128^3 168 / 200; FP32 64^3 34 / 25, 80^3 38 / 48, 128^3 102 / 120).
 int pml_strip_chunk(const fdtd_grid* g) {
     const unsigned long long pb = (unsigned long long)g->Ni * g->Nj * g->esize;
@@ -611,9 +610,9 @@ int pml_strip_chunk(const fdtd_grid* g) {
     const fdtd::StripGeom G = make_pml_strip_geom(g, g->Nk);
     long long planes = 0;
     int kc = strip_chunk(g->Nk, (long long)G.ntx * G.nty, fdtd::pml_strip_wgs(cs) * device_cus(),
-                         fdtd::kPmlStripL, &planes);
+                         2 * (fdtd::kPmlStripL - 1), &planes);
     const double mb = 24e-6 * g->N * g->esize;
-    if (0.5 + 6.5 * planes > (mb <= 26.0 ? 24.0 : 22.0 + 0.45 * mb)) return 0;
+    if (7.0 + 6.5 * planes > (mb <= 26.0 ? 24.0 : 22.0 + 0.45 * mb)) return 0;
     while (fdtd::pml_strip_lds_bytes(cs, kc) * fdtd::pml_strip_wgs(cs) > kLdsLimit) kc = (kc + 1) / 2;  // (its z tables)
     return kc;
 }
@@ -1060,8 +1059,10 @@ int device_cus() {
 }
 
 // z chunk length of a strip pass: every tile costs kchunk + 2L-1 planes
-// (the pipeline fills and drains over L-1 planes at each end, and starts one
-// plane below), and the tiles run in rounds of (resident workgroups per CU x CUs); the chunking
+// (the pipeline fills and drains over L-1 planes at each end, and the plane
+// below the chunk gives its first one B; not counted, that plane made chunks of
+// one plane look free for L = 1: 256^3, us a step FP32 326 instead of 225, FP16
+// 261 instead of 144), and the tiles run in rounds of (resident workgroups per CU x CUs); the chunking
 // with the fewest plane-rounds wins (ties: fewer chunks).  A grid whose tiles
 // are few gets chunks of a few planes: a plane takes about 3 us however few
 // workgroups run, so 128^3 FP32 (18 tiles a plane) takes 10 planes, 17
@@ -1073,7 +1074,7 @@ int strip_default_kchunk(const fdtd_grid* g, const BlockTuning& t, long long* pl
     const fdtd::StripGeom G = make_strip_geom(g, u);
     const long long nxy = (long long)G.ntx * G.nty;
     const long long slots = (long long)std::max(1, strip_occupancy(g, t)) * device_cus();
-    return strip_chunk(g->Nk, nxy, slots, t.L, planes);
+    return strip_chunk(g->Nk, nxy, slots, 2 * t.L - 1, planes);
 }
 
 // Lanes of a tile row of an FP64 pass of L steps straight from memory, z chunks
@@ -1105,7 +1106,7 @@ int strip_direct_lanes(const fdtd_grid* g, const BlockTuning& t, int L, int kchu
         if (kchunk > 0)
             planes = (nxy * ((g->Nk + kchunk - 1) / kchunk) + slots - 1) / slots * (kchunk + 2 * L - 1);
         else
-            strip_chunk(g->Nk, nxy, slots, L, &planes);
+            strip_chunk(g->Nk, nxy, slots, 2 * L - 1, &planes);
         cost[q] = planes * (q ? strip_narrow_cost(L, g->N) : 1.0);
     }
     return cost[1] < cost[0] ? 32 : 64;

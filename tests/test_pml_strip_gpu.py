@@ -84,3 +84,18 @@ def test_path_2_runs_every_step_as_a_sweep(prec):
         b.set_pml_path(3)
     a.close()
     b.close()
+
+
+def test_passes_of_large_grids_march_short_chunks():
+    """A pass whose tiles all march the whole grid lets neighbours drift apart
+    (512^3 FP32: 4.4 ms against 3.4, two sweeps 6.4)."""
+    dt = 0.5 / (C * np.sqrt(3.0))
+    g = FDTD_PML(Parameters(512, 512, 512, dx=1.0, dy=1.0, dz=1.0), dt, 0.2, FP32)
+    ms = {}
+    for path in (2, 0):
+        g.set_pml_path(path)
+        g.update_fields(4)
+        runs = [g.time_update_fields_kernels(12)["steady"] for _ in range(4)]
+        ms[path] = min(t / count for t, count in runs)
+    assert ms[0] < 0.62 * 2 * ms[2], ms
+    g.close()
