@@ -189,12 +189,13 @@ struct fdtd_grid {
     int pml_p[3] = {0, 0, 0};
     void* ES[2][6] = {};        // E splits Exy Exz Eyx Eyz Ezx Ezy, ping-pong with E
     // B splits Bxy Bxz Byx Byz Bzx Bzy: sweeps update BS[bs_cur] in place, strip
-    // passes write the other set (BS[1]: grids that run strip passes only)
+    // passes write the other set (BS[1]: null where the grid runs none)
     void* BS[2][6] = {};
     int bs_cur = 0;
-    void* split_slab = nullptr;  // ES and BS, split_stride bytes apart
+    void* split_slab = nullptr;  // ES and BS[0], split_stride bytes apart
+    void* pass_slab = nullptr;   // BS[1], the same
     size_t split_stride = 0;
-    int pml_strip_kchunk = 0;   // z chunk of a PML strip pass; 0: the grid runs none
+    int pml_strip_kchunk = 0;   // z chunk of a PML strip pass; 0: sweeps cost less
     void* pml_tab = nullptr;    // per-axis decay/coefficient tables (compute type)
     // PML steps: 0 = strip passes where the grid runs them, else the fused PML
     // sweep (shape tune); 1 = the two in-place phase sweeps (pml_e_phase,

@@ -600,8 +600,9 @@ fdtd::StripGeom make_pml_strip_geom(const fdtd_grid* g, int kchunk) {
 // here: counted, it makes one chunk of all planes the choice at 512^3 FP32, where
 // neighbouring tiles drift apart: 4.43 ms a pass, with chunks of 37 planes 3.36.)
 // A pass of few planes takes 7 us and 6.5 us a plane-round, two sweeps 24 us up
-// to 26 MB (24 words a cell), beyond that 22 us and 0.45 us a MB (us, pass against sweeps: FP64 64^3 45 / 43, 80^3 47 / 66,
-// 128^3 168 / 200; FP32 64^3 34 / 25, 80^3 38 / 48, 128^3 102 / 120).
+// to 26 MB (24 words a cell), beyond that 22 us and 0.45 us a MB (us, pass
+// against sweeps: FP64 64^3 45 / 43, 80^3 47 / 66, 128^3 168 / 200; FP32 64^3 34
+// / 25, 80^3 38 / 48, 128^3 102 / 120).
 int pml_strip_chunk(const fdtd_grid* g) {
     const unsigned long long pb = (unsigned long long)g->Ni * g->Nj * g->esize;
     if (g->precision == FDTD_FP16 || pb >= (1ull << 31) || pb + g->split_stride >= (1ull << 32))
@@ -621,21 +622,61 @@ int pml_strip_chunk(const fdtd_grid* g) {
 int alloc_pml(fdtd_grid* g) {
     g->split_stride = (g->N * g->esize + 16 + 255) / 256 * 256;
     g->pml_strip_kchunk = pml_strip_chunk(g);
-    if (g->pml_strip_kchunk > 0 && hipMalloc(&g->split_slab, 24 * g->split_stride) != hipSuccess) {
-        (void)hipGetLastError();
-        g->split_slab = nullptr;
-        g->pml_strip_kchunk = 0;
-    }
-    if (!g->split_slab) HIP_TRY(hipMalloc(&g->split_slab, 18 * g->split_stride));
-    const int nset = g->pml_strip_kchunk > 0 ? 2 : 1;
+    HIP_TRY(hipMalloc(&g->split_slab, 18 * g->split_stride));
     char* p = static_cast<char*>(g->split_slab);
     for (int q = 0; q < 6; ++q) {
         for (int b = 0; b < 2; ++b) g->ES[b][q] = p + (b * 6 + q) * g->split_stride;
-        for (int b = 0; b < nset; ++b) g->BS[b][q] = p + (12 + b * 6 + q) * g->split_stride;
+        g->BS[0][q] = p + (12 + q) * g->split_stride;
     }
-    if (int rc = zero_fill(p, (12 + 6 * nset) * g->split_stride, g->stream)) return rc;
+    if (int rc = zero_fill(p, 18 * g->split_stride, g->stream)) return rc;
     HIP_TRY(hipMalloc(&g->pml_tab, 5 * (size_t)(g->Ni + g->Nj + g->Nk) * compute_size(g->precision)));
     return build_pml_tables(g);
+}
+
+// The second set of B splits (6 words a cell on top of 30), without which a
+// grid's runs take sweeps.  It is taken where it leaves half of the device's
+// memory free, for whatever else the program holds, and given back when an
+// allocation of the grid finds no room (grid_malloc).
+int take_pass_splits(fdtd_grid* g) {
+    if (g->pass_slab || g->pml_strip_kchunk == 0) return FDTD_OK;
+    const size_t bytes = 6 * g->split_stride;
+    size_t free = 0, total = 0;
+    if (hipMemGetInfo(&free, &total) != hipSuccess || free < total / 2 + bytes ||
+        hipMalloc(&g->pass_slab, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        g->pass_slab = nullptr;
+        return FDTD_OK;
+    }
+    for (int q = 0; q < 6; ++q) g->BS[1][q] = static_cast<char*>(g->pass_slab) + q * g->split_stride;
+    return zero_fill(g->pass_slab, bytes, g->stream);
+}
+
+int drop_pass_splits(fdtd_grid* g) {
+    if (!g->pass_slab) return FDTD_OK;
+    if (g->bs_cur == 1)
+        HIP_TRY(hipMemcpyAsync(g->BS[0][0], g->BS[1][0], 6 * g->split_stride, hipMemcpyDeviceToDevice,
+                               g->stream));
+    HIP_TRY(hipStreamSynchronize(g->stream));
+    g->bs_cur = 0;
+    for (int q = 0; q < 6; ++q) g->BS[1][q] = nullptr;
+    HIP_TRY(hipFree(g->pass_slab));
+    g->pass_slab = nullptr;
+    return FDTD_OK;
+}
+
+// hipMalloc for a grid that exists; short of memory, the grid gives back the
+// second set of B splits first, if that makes the room.  (A refusal is reported
+// here, and not once more by the next launch's check.)
+template <typename T>
+hipError_t grid_malloc(fdtd_grid* g, T** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return e;
+    size_t free = 0, total = 0;
+    if (e == hipErrorOutOfMemory && g->pass_slab && hipMemGetInfo(&free, &total) == hipSuccess &&
+        free + 6 * g->split_stride >= bytes && drop_pass_splits(g) == FDTD_OK)
+        e = hipMalloc(p, bytes);
+    (void)hipGetLastError();
+    return e;
 }
 
 // Storage component (0..5) whose scale split q (0..5 E, 6..11 B) shares.
@@ -661,7 +702,7 @@ public:
         const int n = g_->pml ? 18 : 6;
         for (int d = 0; d < n; ++d) {
             void* p = nullptr;
-            HIP_TRY(hipMalloc(&p, bytes()));
+            HIP_TRY(grid_malloc(g_, &p, bytes()));
             saved_.push_back(p);
             HIP_TRY(hipMemcpyAsync(p, state_ptr(d), bytes(), hipMemcpyDeviceToDevice, g_->stream));
         }
@@ -1375,8 +1416,7 @@ int run_fused(fdtd_grid* g, int nsteps, hipEvent_t mid = nullptr) {
     const bool use_inl = inline_sources(g, &inl);
     int rc = use_inl ? FDTD_OK : flush_sources(g);
     if (rc) return rc;
-    const bool pml_strips = g->pml && g->pml_path == 0 && g->pml_strip_kchunk > 0 && nsteps >= 2 &&
-                            !g->j_dense_active;
+    const bool pml_strips = g->pass_slab && g->pml_path == 0 && nsteps >= 2 && !g->j_dense_active;
     if (carried < 0) {
         TraceRange tr("b_half_prologue");
         hipEvent_t t0 = trace_begin(g);
@@ -1560,7 +1600,7 @@ int run_steps(fdtd_grid* g, int nsteps, bool three_sweep) {
 // ---- conversions and reductions ------------------------------------------------
 
 int ensure_staging(fdtd_grid* g) {
-    if (!g->staging) HIP_TRY(hipMalloc(&g->staging, g->N * sizeof(double)));
+    if (!g->staging) HIP_TRY(grid_malloc(g, &g->staging, g->N * sizeof(double)));
     return FDTD_OK;
 }
 
@@ -1600,7 +1640,7 @@ int zero_fill(void* p, size_t bytes, hipStream_t s) {
 int ensure_dense_j(fdtd_grid* g) {
     const size_t bytes = g->N * current_size(g->precision);
     for (int d = 0; d < 3; ++d)
-        if (!g->J[d]) HIP_TRY(hipMalloc(&g->J[d], bytes + 16));
+        if (!g->J[d]) HIP_TRY(grid_malloc(g, &g->J[d], bytes + 16));
     return FDTD_OK;
 }
 
@@ -1781,6 +1821,8 @@ int create_grid(const fdtd_parameters* p, double dt, double pml_percent, int pre
             if (wide || strips_pay(g, t, planes)) g->btune = t;
         }
     }
+    if (g->pml && g->fused_ok)
+        if (int rc = take_pass_splits(g)) return cleanup(rc);
     if (hipStreamSynchronize(g->stream) != hipSuccess)
         return cleanup(fail(FDTD_ERR_HIP, "initialisation failed"));
     *out = g;
@@ -1814,6 +1856,7 @@ int fdtd_destroy(fdtd_grid* g) {
             if (g->B[b][d]) (void)hipFree(g->B[b][d]);
         }
     if (g->split_slab) (void)hipFree(g->split_slab);
+    if (g->pass_slab) (void)hipFree(g->pass_slab);
     if (g->pml_tab) (void)hipFree(g->pml_tab);
     for (int b = 0; b < 2; ++b)
         for (int d = 0; d < 3; ++d)
@@ -2131,7 +2174,7 @@ int fdtd_set_current_values(fdtd_grid* g, int n, const long long* index, const i
             g->d_jw = nullptr;
             g->d_jw_cap = 0;
             const size_t cap = std::max<size_t>(64, 2 * w.size());
-            HIP_TRY(hipMalloc(&g->d_jw, cap * sizeof(fdtd::CurrentWrite)));
+            HIP_TRY(grid_malloc(g, &g->d_jw, cap * sizeof(fdtd::CurrentWrite)));
             g->d_jw_cap = cap;
         }
         HIP_TRY(hipMemcpyAsync(g->d_jw, w.data(), w.size() * sizeof(fdtd::CurrentWrite),
@@ -2260,7 +2303,7 @@ int fdtd_update_fields_with_currents(fdtd_grid* g, int nsteps, const int* counts
         if (g->d_jtab) HIP_TRY(hipFree(g->d_jtab));
         g->d_jtab = nullptr;
         g->d_jtab_cap = 0;
-        HIP_TRY(hipMalloc(&g->d_jtab, sizeof(double) * tab.size()));
+        HIP_TRY(grid_malloc(g, &g->d_jtab, sizeof(double) * tab.size()));
         g->d_jtab_cap = tab.size();
     }
     // the table is read by this call's source evaluations, queued on the
@@ -2320,9 +2363,9 @@ int fdtd_set_probes(fdtd_grid* g, int n, const long long* index, const int* comp
     g->probe_cap = 0;
     g->probe_rows = 0;
     if (n == 0) return FDTD_OK;
-    HIP_TRY(hipMalloc(&g->d_probe, sizeof(fdtd::Probe) * n));
-    HIP_TRY(hipMalloc(&g->d_pstart, sizeof(int) * (g->Nk + 1)));
-    HIP_TRY(hipMalloc(&g->d_probe_out, sizeof(double) * n * capacity));
+    HIP_TRY(grid_malloc(g, &g->d_probe, sizeof(fdtd::Probe) * n));
+    HIP_TRY(grid_malloc(g, &g->d_pstart, sizeof(int) * (g->Nk + 1)));
+    HIP_TRY(grid_malloc(g, &g->d_probe_out, sizeof(double) * n * capacity));
     HIP_TRY(hipMemcpy(g->d_probe, list.data(), sizeof(fdtd::Probe) * n, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(g->d_pstart, start.data(), sizeof(int) * (g->Nk + 1), hipMemcpyHostToDevice));
     // rows not yet written read as NaN (all bits set)
@@ -2360,7 +2403,7 @@ int fdtd_set_energy_interval(fdtd_grid* g, int every, long long capacity) {
     g->energy_cap = 0;
     g->energy_steps.clear();
     if (every == 0) return FDTD_OK;
-    HIP_TRY(hipMalloc(&g->d_energy, sizeof(double) * 6 * capacity));
+    HIP_TRY(grid_malloc(g, &g->d_energy, sizeof(double) * 6 * capacity));
     g->energy_every = every;
     g->energy_cap = capacity;
     return FDTD_OK;
@@ -2850,7 +2893,7 @@ int fdtd_set_pml_path(fdtd_grid* g, int path, int V, int TY, int kchunk) {
     if (!g->pml) return fail(FDTD_ERR_UNSUPPORTED, "the grid has no PML layer");
     if (path != 1) {
         g->pml_path = path;
-        return FDTD_OK;
+        return path == 0 ? take_pass_splits(g) : drop_pass_splits(g);
     }
     Tuning t = pml_phase_default(g);
     if (V > 0) {
@@ -2866,7 +2909,7 @@ int fdtd_set_pml_path(fdtd_grid* g, int path, int V, int TY, int kchunk) {
                     t.V, t.TY, t.kchunk);
     g->ptune = t;
     g->pml_path = 1;
-    return FDTD_OK;
+    return drop_pass_splits(g);
 }
 
 int fdtd_get_pml_path(const fdtd_grid* g, int out[4]) {

@@ -107,7 +107,9 @@ int fdtd_create_pml(const fdtd_parameters* params, double dt, double pml_percent
  * PML sweep (shape: fdtd_set_tuning) or, on FP64 and FP32 grids of more than
  * about 50 MB of state, with no dense J and no probes, two steps to a strip pass
  * (same bits; 512^3 FP32 with a 0.2 layer 1.7 ms per step; fdtd_get_stats counts
- * the passes); path 2 as the fused sweep on every step; path 1 as two in-place
+ * the passes; they hold 36 words a cell instead of 30, taken where that leaves
+ * half of the device's memory free and given back when an allocation of the grid
+ * finds no room: it then runs sweeps until path 0 is set again); path 2 as the fused sweep on every step; path 1 as two in-place
  * sweeps per step, an E phase and a B phase, with V cells per lane, TY full rows
  * per workgroup and kchunk planes per z chunk (0: defaults; V*storage bytes at
  * most 16).  At 512^3 with a 0.2 layer the phases take 3.94 ms per FP32

@@ -68,7 +68,7 @@ def test_path_2_runs_every_step_as_a_sweep(prec):
     sweeps take the shape that set_tuning gives."""
     a, b = make((96, 90, 100), prec, 0.2), make((96, 90, 100), prec, 0.2)
     passes = 0
-    for path, n in ((2, 6), (0, 4), (2, 5), (1, 3), (0, 6)):
+    for path, n in ((2, 6), (0, 4), (2, 5), (1, 3), (0, 6), (2, 3), (0, 7), (1, 2)):
         b.set_pml_path(path)
         assert b.get_pml_path()["path"] == path
         if path == 2:
@@ -82,6 +82,43 @@ def test_path_2_runs_every_step_as_a_sweep(prec):
         assert np.array_equal(a.split(q), b.split(q)), q
     with pytest.raises(Exception):
         b.set_pml_path(3)
+    a.close()
+    b.close()
+
+
+@pytest.mark.torch
+def test_memory_of_the_passes_is_given_back():
+    """A grid whose memory is short gives up the passes' second set of B splits,
+    with the state in either set, rather than refuse: a record buffer that
+    fits only without it is allocated, the runs go on as sweeps with the same
+    bits, and passes come back when asked for."""
+    import torch
+
+    shape = (256, 256, 256)
+    a, b = make(shape, FP64, 0.2), make(shape, FP64, 0.2)
+    a.set_pml_path(2)
+    a.update_fields(6)
+    b.update_fields(6)
+    assert b.launch_stats()["passes"] == 3
+    free = torch.cuda.mem_get_info()[0]
+    b.set_energy_interval(1 << 30, (free + (600 << 20)) // 48)  # of the 768 MiB of that set
+    b.set_energy_interval(0)
+    assert a.checksum() == b.checksum()
+    for q in range(12):
+        assert np.array_equal(a.split(q), b.split(q)), q
+    a.update_fields(3)
+    b.update_fields(3)
+    assert a.checksum() == b.checksum()
+    assert b.launch_stats()["passes"] == 3
+    # a request that no release could meet is refused and costs nothing
+    b.set_pml_path(0)
+    with pytest.raises(Exception):
+        b.set_energy_interval(1 << 30, 1 << 40)
+    b.set_energy_interval(0)
+    a.update_fields(5)
+    b.update_fields(5)
+    assert a.checksum() == b.checksum()
+    assert b.launch_stats()["passes"] == 5
     a.close()
     b.close()
 
