@@ -599,10 +599,12 @@ fdtd::StripGeom make_pml_strip_geom(const fdtd_grid* g, int kchunk) {
 // where two fused sweeps cost less.  (The plane below a chunk is not counted
 // here: counted, it makes one chunk of all planes the choice at 512^3 FP32, where
 // neighbouring tiles drift apart: 4.43 ms a pass, with chunks of 37 planes 3.36.)
-// A pass of few planes takes 7 us and 6.5 us a plane-round, two sweeps 24 us up
-// to 26 MB (24 words a cell), beyond that 22 us and 0.45 us a MB (us, pass
-// against sweeps: FP64 64^3 45 / 43, 80^3 47 / 66, 128^3 168 / 200; FP32 64^3 34
-// / 25, 80^3 38 / 48, 128^3 102 / 120).
+// A pass of few planes takes 7 us and 6.5 us a plane-round, a fifth more and up
+// where packs of a row hold both kinds of cells; two sweeps 24 us up to 40 MB (24
+// words a cell), beyond that 22 us and 0.45 us a MB (us, pass against sweeps,
+// layer of 0.1, where not said with packs of one kind: FP64 64^3 40 / 42, 72^3 of
+// both 50 / 46, 80^3 46 / 65, 128^3 133 / 188; FP32 64^3 of both 39 / 25, 72^3 of
+// both 40 / 27, 80^3 38 / 48, 100^3 of both 73 / 72, 128^3 83 / 119).
 int pml_strip_chunk(const fdtd_grid* g) {
     const unsigned long long pb = (unsigned long long)g->Ni * g->Nj * g->esize;
     if (g->precision == FDTD_FP16 || pb >= (1ull << 31) || pb + g->split_stride >= (1ull << 32))
@@ -613,7 +615,9 @@ int pml_strip_chunk(const fdtd_grid* g) {
     int kc = strip_chunk(g->Nk, (long long)G.ntx * G.nty, fdtd::pml_strip_wgs(cs) * device_cus(),
                          2 * (fdtd::kPmlStripL - 1), &planes);
     const double mb = 24e-6 * g->N * g->esize;
-    if (7.0 + 6.5 * planes > (mb <= 26.0 ? 24.0 : 22.0 + 0.45 * mb)) return 0;
+    const int pack = 16 / cs;
+    const double mixed = g->Ni % pack == 0 && g->pml_p[0] % pack != 0 ? 1.2 : 1.0;
+    if (mixed * (7.0 + 6.5 * planes) > (mb <= 40.0 ? 24.0 : 22.0 + 0.45 * mb)) return 0;
     while (fdtd::pml_strip_lds_bytes(cs, kc) * fdtd::pml_strip_wgs(cs) > kLdsLimit) kc = (kc + 1) / 2;  // (its z tables)
     return kc;
 }

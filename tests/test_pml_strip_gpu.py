@@ -136,3 +136,23 @@ def test_passes_of_large_grids_march_short_chunks():
         ms[path] = min(t / count for t, count in runs)
     assert ms[0] < 0.62 * 2 * ms[2], ms
     g.close()
+
+
+@pytest.mark.parametrize("prec,side,percent,passes", [
+    (FP32, 72, 0.1, False),    # the caches hold the state, packs of both kinds of cells
+    (FP64, 72, 0.3, False),    # packs of both kinds
+    (FP32, 100, 0.3, False),
+    (FP32, 80, 0.1, True), (FP64, 80, 0.3, True), (FP32, 128, 0.1, True),
+])
+def test_grids_that_take_passes(prec, side, percent, passes):
+    """Passes run where they are the faster form, and only there (72^3 FP32: a
+    pass 40 us, its two sweeps 27)."""
+    a, b = make((side,) * 3, prec, percent), make((side,) * 3, prec, percent)
+    a.set_pml_path(2)
+    for n in (4, 7):
+        a.update_fields(n)
+        b.update_fields(n)
+        assert a.checksum() == b.checksum()
+    assert b.launch_stats()["passes"] == (5 if passes else 0)
+    a.close()
+    b.close()
