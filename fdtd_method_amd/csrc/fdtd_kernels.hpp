@@ -809,9 +809,10 @@ __device__ __forceinline__ int pml_pack(int lane, int npacks, int pi, int V) {
     return lane - nhi;
 }
 
-// INL: the launch's own sources are added (inl is null otherwise).
+// INL: the launch's own sources are added (inl is null otherwise).  SKIP: PML
+// sweeps leave out the layer's E totals.
 template <typename S, typename C, typename JT, int V, bool STEADY, bool PML = false,
-          bool AUTO = false, bool PROBE = false, bool INL = false>
+          bool AUTO = false, bool PROBE = false, bool INL = false, bool SKIP = false>
 __device__ __forceinline__ void fused_tile(const SweepArgs<S, C, JT>& a, int tile_y, int chunk,
                                            C* __restrict__ lds, const InlineArgs* inl = nullptr) {
     static_assert(!(PML && PROBE), "PML sweeps record no probes");
@@ -886,13 +887,14 @@ __device__ __forceinline__ void fused_tile(const SweepArgs<S, C, JT>& a, int til
     // The Ey slot is one load for every thread with a selected address (a
     // branch whose two sides load into the same registers would make the
     // halo row wait for the whole prefetch).
-    // PML sweeps: E of a layer cell is the sum of its splits, so lanes whose
-    // cells all lie in the layer read no E totals, and the steady sweeps of a
+    // PML sweeps with SKIP: E of a layer cell is the sum of its splits, so lanes
+    // whose cells all lie in the layer read no E totals, and the steady sweeps of a
     // run, whose totals no later sweep reads there, write none (layer cell:
     // 30 words instead of 36; 512^3 FP32 with a 0.2 layer: 16.5 -> 13.9 GB per
     // step).  The last sweep of a run writes them all; the rescaling variants
     // read and write them as before.
-    constexpr bool kSkipE = PML && !AUTO;
+    constexpr bool kSkipE = PML && SKIP;
+    static_assert(!(SKIP && AUTO), "rescaling sweeps read and write every total");
     const bool xlayer = kSkipE && (ib + V <= a.pml.pi || ib >= Ni - a.pml.pi);
     auto layer_only = [&](int kw) {
         return kSkipE && (xlayer || !(in_main(kw, Nk, a.pml.pk) && in_main(j, Nj, a.pml.pj)));
@@ -1293,7 +1295,7 @@ __host__ __device__ constexpr int fused_pml_max_threads(int V, int csize) {
     return V * csize >= 16 ? 512 : 768;
 }
 
-template <typename S, typename C, typename JT, int V, bool STEADY, bool AUTO = false>
+template <typename S, typename C, typename JT, int V, bool STEADY, bool AUTO, bool SKIP>
 __global__ void __launch_bounds__(fused_pml_max_threads(V, sizeof(C)))
 fused_pml_sweep(SweepArgs<S, C, JT> a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -1302,7 +1304,8 @@ fused_pml_sweep(SweepArgs<S, C, JT> a) {
     if (t >= a.g.ntiles) return;
     const int tile_y = t % a.g.ntile_y;
     const int chunk = t / a.g.ntile_y;
-    fused_tile<S, C, JT, V, STEADY, true, AUTO>(a, tile_y, chunk, reinterpret_cast<C*>(lds_raw));
+    fused_tile<S, C, JT, V, STEADY, true, AUTO, false, false, SKIP>(a, tile_y, chunk,
+                                                                    reinterpret_cast<C*>(lds_raw));
 }
 
 // ---------------------------------------------------------------------------

@@ -781,6 +781,16 @@ int gather_probes(fdtd_grid* g) {
     }
 }
 
+// Whether a PML grid's sweeps leave out the layer's E totals: the traffic saved
+// pays once it is what bounds a sweep, before that the lanes' branches around
+// their loads cost more, the narrower the storage (us a step, layer 0.1, without /
+// with: FP32 16^3 9.4 / 10.3, 32^3 10.0 / 10.4, 48^3 11.9 / 11.4; FP16 256^3 269 /
+// 282, 512^3 2264 / 2196; FP64 32^3 10.5 / 9.7).
+bool pml_skips_totals(const fdtd_grid* g) {
+    const double mb = 24e-6 * g->N * g->esize;
+    return mb > (g->precision == FDTD_FP64 ? 0.0 : g->precision == FDTD_FP32 ? 6.0 : 2000.0);
+}
+
 template <typename S, int V, bool STEADY, bool AUTO, bool PROBE>
 int launch_fused_a(fdtd_grid* g, const Tuning& t, int slot, int in, int out,
                    const SweepExtra& x) {
@@ -788,7 +798,11 @@ int launch_fused_a(fdtd_grid* g, const Tuning& t, int slot, int in, int out,
     using JT = C;
     auto kern = fdtd::fused_sweep<S, C, JT, V, STEADY, AUTO, PROBE>;
     if constexpr (!PROBE)
-        if (g->pml) kern = fdtd::fused_pml_sweep<S, C, JT, V, STEADY, AUTO>;
+        if (g->pml) {
+            kern = fdtd::fused_pml_sweep<S, C, JT, V, STEADY, AUTO, false>;
+            if constexpr (!AUTO)
+                if (pml_skips_totals(g)) kern = fdtd::fused_pml_sweep<S, C, JT, V, STEADY, AUTO, true>;
+        }
     fdtd::SweepArgs<S, C, JT> a;
     a.in = fields_of<S>(g, in);
     a.out = fields_of<S>(g, out);

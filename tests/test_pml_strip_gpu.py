@@ -156,3 +156,51 @@ def test_grids_that_take_passes(prec, side, percent, passes):
     assert b.launch_stats()["passes"] == (5 if passes else 0)
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("prec,side", [(FP32, 24), (FP32, 64), (Precision.FP16, 40)])
+def test_sweeps_with_and_without_the_layers_totals(prec, side):
+    """Sweeps that leave out the layer's E totals between the steps of a run,
+    or not, by the size of the state: after a run every layer total is the sum
+    of its splits, and two such runs agree bit for bit."""
+    a, b = make((side,) * 3, prec, 0.2), make((side,) * 3, prec, 0.2)
+    for g in (a, b):
+        g.set_pml_path(2)
+        g.update_fields(5)
+    assert a.checksum() == b.checksum()
+    for c, (p, q) in enumerate([("Exy", "Exz"), ("Eyx", "Eyz"), ("Ezx", "Ezy")]):
+        e, s = a.download(c), a.split(p) + a.split(q)
+        layer = np.ones((side,) * 3, bool)
+        w = a.pml_widths
+        layer[w[2]:side - w[2], w[1]:side - w[1], w[0]:side - w[0]] = False
+        d = np.abs(e - s)[layer.ravel()]
+        unit = 2.0 ** (-24 if prec == FP32 else -11)
+        assert d.max() <= unit * np.abs(s).max()
+    a.close()
+    b.close()
+
+
+def test_fp16_sweeps_of_large_grids():
+    """FP16 sweeps leave out the layer's totals on large grids, rescaling ones
+    never do: a run of both kinds stays within FP16's 5e-3 (relative L2) of FP32
+    on planes inside and across the layer, and its last sweep's layer totals are
+    the sums of the splits."""
+    n = 348
+    dt = 0.5 / (C * np.sqrt(3.0))
+    grids = []
+    for prec in (FP32, Precision.FP16):
+        g = FDTD_PML(Parameters(n, n, n, dx=1.0, dy=1.0, dz=1.0), dt, 0.1, prec)
+        g.add_plane_wave([2, 3, 1], 0.7, 0.3, [0.3, -1.0, 0.5])
+        if prec == Precision.FP16:
+            g.autoscale(10)
+            g.set_autoscale_interval(2, 10)
+        g.update_fields(7)
+        grids.append(g)
+    a, b = grids
+    for k in (0, 33, 34, 35, n // 2, n - 36, n - 1):
+        x = [np.concatenate([g.download_plane(c, k).ravel() for c in range(6)]) for g in grids]
+        assert np.linalg.norm(x[1] - x[0]) <= 5e-3 * np.linalg.norm(x[0]), k
+    e, s = b.download(0)[:n * n], (b.split("Exy") + b.split("Exz"))[:n * n]  # plane 0: all layer
+    assert np.abs(e - s).max() <= 2.0 ** -11 * np.abs(s).max()
+    a.close()
+    b.close()
