@@ -2221,16 +2221,16 @@ __device__ __forceinline__ double lane_next(double x) {
 // LDS offset lds + i*BYTES (base and lds are uniform; lanes switched off
 // write nothing).  No register is written: the data is there once the
 // wavefront has waited for vmcnt.  In assembly, because the compiler makes
-// every later LDS read wait for the builtin's transfer.
+// every later LDS read wait for the builtin's transfer.  (m0, the LDS address, is
+// an operand: written inside, the compiler would take a value it put there before
+// for still in place.)
 template <int BYTES, typename T>
 __device__ __forceinline__ void load_to_lds(gptr<T> base, unsigned off, unsigned lds) {
     static_assert(BYTES == 4 || BYTES == 16, "4 or 16 bytes per lane");
     if constexpr (BYTES == 16)
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off),
-                     "s"(base), "s"(lds) : "memory");
+        asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(lds) : "memory");
     else
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off),
-                     "s"(base), "s"(lds) : "memory");
+        asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "{m0}"(lds) : "memory");
 }
 
 // Whether a probe lies among the columns and rows that a tile stores (long

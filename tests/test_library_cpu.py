@@ -107,3 +107,37 @@ def test_pml_profile_matches_the_oracle(n, pct, d):
         assert decay[i] == a
         c = (1.0 - math.exp(-ref[i] * dt * O.C)) / (ref[i] * d) if ref[i] != 0.0 else O.C * dt / d
         assert coef[i] == c
+
+
+def test_lds_transfers_leave_m0_to_the_compiler(tmp_path):
+    """Around a plane's transfer to LDS the compiler sets m0, which holds the
+    transfer's LDS address, again for its own next use: in a kernel that uses
+    it before and after, three settings for three transfers."""
+    import subprocess
+    from fdtd_method_amd import build
+    src = tmp_path / "m0.hip"
+    src.write_text("""
+#include "fdtd_kernels.hpp"
+extern "C" __global__ void probe(const float* in, float* out) {
+    __shared__ float lds[256];
+    auto own = [&](int at) {
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(in + at + threadIdx.x),
+                                         (__attribute__((address_space(3))) void*)lds, 4, 0, 0);
+    };
+    own(0);
+    fdtd::load_to_lds<4>(fdtd::uniform_gptr<const float>(in), threadIdx.x * 4, 512);
+    own(64);
+    __builtin_amdgcn_s_waitcnt(0);
+    out[threadIdx.x] = lds[threadIdx.x];
+}
+""")
+    asm = tmp_path / "m0.s"
+    subprocess.run([build.hipcc(), *build.HIPCC_FLAGS, f"-I{build.INCLUDE}", f"-I{build.CSRC}",
+                    "--offload-device-only", "-S", str(src), "-o", str(asm)], check=True,
+                   capture_output=True)
+    code = [line.split(";")[0].split() for line in asm.read_text().splitlines()]
+    ops = ["set" if len(c) > 1 and c[1].startswith("m0") else "load" for c in code
+           if c and ((c[0].startswith("s_mov") and len(c) > 1 and c[1].startswith("m0"))
+                     or c[0].startswith("global_load_lds"))]
+    assert ops == ["set", "load"] * 3, ops
+
