@@ -259,11 +259,11 @@ int launch_batch(fdtd_batch* b, bool steady, int parity, const double* vals_row)
 
 // ---- strip passes --------------------------------------------------------
 
-const void* strip_kernel(int precision, int V, int R, int L, int lanes, bool final, bool stage, bool first) {
+const void* strip_kernel(int precision, int V, int R, int L, int lanes, bool final, int depth, bool first) {
     switch (precision) {
-        case FDTD_FP64: return batch_strip_kernel<double>(V, R, L, lanes, final, stage, first);
-        case FDTD_FP32: return batch_strip_kernel<float>(V, R, L, lanes, final, stage, first);
-        default: return batch_strip_kernel<_Float16>(V, R, L, lanes, final, stage, first);
+        case FDTD_FP64: return batch_strip_kernel<double>(V, R, L, lanes, final, depth, first);
+        case FDTD_FP32: return batch_strip_kernel<float>(V, R, L, lanes, final, depth, first);
+        default: return batch_strip_kernel<_Float16>(V, R, L, lanes, final, depth, first);
     }
 }
 
@@ -279,7 +279,7 @@ int launch_batch_strip_s(fdtd_batch* b, bool final, bool first, int parity, cons
     a.vstride = b->total_src;
     a.pad = 0;
     a.counters = b->d_counters;
-    const void* kern = batch_strip_kernel<S>(b->sV, b->sR, b->sL, b->slanes, final, b->sdepth > 0, first);
+    const void* kern = batch_strip_kernel<S>(b->sV, b->sR, b->sL, b->slanes, final, b->sdepth, first);
     if (!kern) return fail(FDTD_ERR_UNSUPPORTED, "strip variant V=%d R=%d not built", b->sV, b->sR);
     if (int rc = allow_dynamic_lds(kern, b->slds)) return rc;
     void* args[] = {&a};
@@ -345,7 +345,7 @@ int apply_strips(fdtd_batch* b, int L, int V, int R, int W) {
     if (lds > kLdsLimit) return fail(FDTD_ERR_INVALID_ARGUMENT, "strip tiles need too much LDS");
     int per_cu = 0;
     for (bool final : {false, true}) {
-        const void* kern = strip_kernel(b->precision, V, R, L, lanes, final, depth > 0, false);
+        const void* kern = strip_kernel(b->precision, V, R, L, lanes, final, depth, false);
         if (!kern) return fail(FDTD_ERR_UNSUPPORTED, "strip variant not built");
         if (int rc = allow_dynamic_lds(kern, lds)) return rc;
         if (!final) HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 64 * W, lds));

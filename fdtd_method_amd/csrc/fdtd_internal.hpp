@@ -333,8 +333,9 @@ int strip_occupancy_s(const BlockTuning& t, int depth);
 // from the current buffers to the others, which become the current ones.
 fdtd::StripGeom make_pml_strip_geom(const fdtd_grid* g, int kchunk);
 int launch_pml_strip(fdtd_grid* g, bool final, int slot);
-// The batched strip kernel of a shape (null: not built).
+// The batched strip kernel of a shape (null: not built).  first: the pass reads E
+// of the next plane from the stage too, so it needs two planes there.
 template <typename S>
-const void* batch_strip_kernel(int V, int R, int L, int lanes, bool final, bool stage, bool first);
+const void* batch_strip_kernel(int V, int R, int L, int lanes, bool final, int depth, bool first);
 
 }  // namespace fdtd::rt

@@ -1307,7 +1307,14 @@ bool tail_pass_pays(const fdtd_grid* g, int l) {
 int run_blocked(fdtd_grid* g, int nsteps, hipEvent_t mid) {
     const bool strips = g->btune.R > 0;
     const int carried = strips ? g->ba_cur : -1;
-    const bool own_half = strips && make_strip_geom(g, g->btune).depth == 2;
+    const int L = g->btune.L;
+    const int npass = nsteps / L;
+    BlockTuning tail = g->btune;  // the pass of the steps left over
+    tail.L = nsteps % L;
+    const bool use_tail = strips && tail.L >= 2 && tail_pass_pays(g, tail.L) && strip_valid(g, tail);
+    // whether the first pass takes the half step, by the planes it stages
+    const bool own_half = strips && (npass > 0 || use_tail) &&
+                          make_strip_geom(g, npass > 0 ? g->btune : tail).depth == 2;
     int rc = flush_sources(g);
     if (rc) return rc;
     g->ba_cur = -1;
@@ -1322,11 +1329,6 @@ int run_blocked(fdtd_grid* g, int nsteps, hipEvent_t mid) {
                            (!own_half || g->precision == FDTD_FP16 || carried >= 0) && ensure_carry(g);
     const int ahead_buf = carried < 0 ? 0 : 1 - carried;
     if (mid) HIP_TRY(hipEventRecord(mid, g->stream));
-    const int L = g->btune.L;
-    const int npass = nsteps / L;
-    BlockTuning tail = g->btune;  // the pass of the steps left over
-    tail.L = nsteps % L;
-    const bool use_tail = strips && tail.L >= 2 && tail_pass_pays(g, tail.L) && strip_valid(g, tail);
     const int rem = use_tail ? 0 : nsteps % L;
     const int blocked = nsteps - rem;
     const int chunk = (kValTable / L) * L;

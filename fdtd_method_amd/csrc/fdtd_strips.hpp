@@ -48,6 +48,8 @@ int launch_strip_v(fdtd_grid* g, bool first, int slot, int in, int out, void* co
         a.g = make_strip_geom(g, t);
         for (int c = 0; c < 6; ++c) a.iscale[c] = g->pass_iscale[c];
         a.probe = probe_args(g);
+        if (first && a.g.depth != 2)  // (it reads E of the next plane from the stage)
+            return fail(FDTD_ERR_UNSUPPORTED, "a first pass stages two planes, this one %d", a.g.depth);
         constexpr int SL = fdtd::strip_stage_lanes(sizeof(C));
         auto kern = strip_kernel<S, V, R, L, FINAL, false, 64, false>(g->pass_rescale, probing(g));
         if constexpr (sizeof(C) == 8)
@@ -177,7 +179,9 @@ int launch_strip(fdtd_grid* g, bool final, bool first, int slot, int in, int out
 }
 
 template <typename S>
-const void* batch_strip_kernel(int V, int R, int L, int lanes, bool final, bool stage, bool first) {
+const void* batch_strip_kernel(int V, int R, int L, int lanes, bool final, int depth, bool first) {
+    if (first && depth != 2) return nullptr;
+    const bool stage = depth > 0;
     return final ? batch_strip_kernel_s<S, true>(V, R, L, lanes, stage, first)
                  : batch_strip_kernel_s<S, false>(V, R, L, lanes, stage, first);
 }

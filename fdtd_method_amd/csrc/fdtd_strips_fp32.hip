@@ -4,5 +4,5 @@
 namespace fdtd::rt {
 template int launch_strip<float>(fdtd_grid*, bool, bool, int, int, int, void* const*, void* const*);
 template int strip_occupancy_s<float>(const BlockTuning&, int);
-template const void* batch_strip_kernel<float>(int, int, int, int, bool, bool, bool);
+template const void* batch_strip_kernel<float>(int, int, int, int, bool, int, bool);
 }  // namespace fdtd::rt

@@ -141,3 +141,18 @@ extern "C" __global__ void probe(const float* in, float* out) {
                      or c[0].startswith("global_load_lds"))]
     assert ops == ["set", "load"] * 3, ops
 
+
+def test_first_passes_need_two_staged_planes():
+    """The pass that takes a run's first B half step reads E of the next plane
+    from the stage: no kernel is given for it with fewer planes there."""
+    L = _lib.load()
+    for name in ("If", "Id", "IDF16_"):
+        fn = getattr(L, f"_ZN4fdtd2rt18batch_strip_kernel{name}EEPKviiiibib")
+        fn.restype = ctypes.c_void_p
+        lanes = 32 if name == "Id" else 64
+        for levels in (2, 3, 4):
+            for final in (False, True):
+                got = {(d, f): fn(1, 2, levels, lanes, ctypes.c_bool(final), d, ctypes.c_bool(f))
+                       for d in (0, 1, 2) for f in (False, True)}
+                assert all(got[d, False] for d in (0, 1, 2))
+                assert got[2, True] and not got[1, True] and not got[0, True]
