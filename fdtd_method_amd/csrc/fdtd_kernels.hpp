@@ -350,7 +350,9 @@ __device__ __forceinline__ double from_lane(double x, int lane) {
 }
 
 // Adds the J terms of the sources held by the lanes set in `lanes`, as
-// add_point_sources does.
+// add_point_sources does.  Called where every lane of the wavefront is on: a copy
+// of the sources' registers made by the compiler where some are off would lose
+// what those hold.
 template <typename C, int V>
 __device__ __forceinline__ void add_lane_sources(C (&t)[3][V], const Coefs<C>& c,
                                                  const LaneSource<C>& s, unsigned long long lanes,
@@ -823,9 +825,12 @@ __device__ __forceinline__ void fused_tile(const SweepArgs<S, C, JT>& a, int til
     const int k0 = chunk * a.g.kchunk;
     const int k1 = min(k0 + a.g.kchunk, Nk);
     const int tid = threadIdx.x;
-    const int r = tid / lanes;
-    const int ib = (PML ? pml_pack(tid - r * lanes, lanes, a.pml.pi, V) : tid - r * lanes) * V;
-    const bool active = r <= ty;
+    const int tr = tid / lanes;
+    // INL: lanes past the halo row do its work once more, so that wavefronts work
+    // with all lanes or not at all (see add_lane_sources)
+    const int r = INL ? min(tr, ty) : tr;
+    const int ib = (PML ? pml_pack(tid - tr * lanes, lanes, a.pml.pi, V) : tid - tr * lanes) * V;
+    const bool active = INL ? (tid & ~63) / lanes <= ty : r <= ty;
     const bool own = r < ty;  // row r == ty is the halo row
     const int j = (j0 + r >= Nj) ? j0 + r - Nj : j0 + r;  // halo row wraps
     const int jm = (j0 == 0) ? Nj - 1 : j0 - 1;
