@@ -323,3 +323,53 @@ def test_fp64_row_widths(shape, L, lanes):
     assert np.array_equal(a.read_probes(), b.read_probes())
     a.close()
     b.close()
+
+
+def many_sources(shape, dt, m, plane=None):
+    rng = np.random.default_rng(m)
+    i, j, k = (rng.integers(0, s, m) for s in shape)
+    i[:2], j[:2] = shape[0] - 1, shape[1] - 1
+    if plane is not None:
+        k[:] = plane
+    return [dict(i=int(i[q]), j=int(j[q]), k=int(k[q]), comp=q % 3, kind=1, amp=1e-3 / dt, period=9 * dt,
+                 t0=4 * dt, sigma=6 * dt) for q in range(m)]
+
+
+@pytest.mark.parametrize("prec", [Precision.FP64, Precision.FP32, Precision.FP16])
+@pytest.mark.parametrize("shape,m,plane", [
+    ((72, 70, 74), 200, 73),    # three to four sources in a row of the last plane
+    ((72, 70, 74), 1, 0),
+    ((72, 70, 74), 64, None),
+    ((101, 99, 12), 65, None),  # one more than a wavefront searches at a time
+    ((24, 9, 20), 130, 4),      # rows of the grid that come twice in a tile
+    ((7, 5, 20), 40, None),
+])
+def test_many_sources(prec, shape, m, plane):
+    """Passes add the sources of a long list as the sweeps do, cell by cell."""
+    dt = courant_dt(1, 1, 1, factor=0.5)
+    state = random_state(int(np.prod(shape)), 5)
+    a, b = (grid(shape, dt, state, prec, many_sources(shape, dt, m, plane)) for _ in range(2))
+    a.set_time_blocking_strips(0)
+    b.set_time_blocking_strips(4, 1, 2, 8 if prec == Precision.FP64 else 16)
+    for steps in (8, 7, 4):
+        a.update_fields(steps)
+        b.update_fields(steps)
+        assert a.checksum() == b.checksum(), steps
+    a.close()
+    b.close()
+
+
+def test_many_sources_in_a_plane_cost_passes_no_more_than_sweeps():
+    """Wavefronts pass over the sources of other wavefronts' rows (FP64
+    72 x 70 x 74, 200 in one plane, 24 steps: sweeps 1.00 ms, passes 0.70, and
+    1.63 where every wavefront took every source of its plane)."""
+    shape, dt = (72, 70, 74), courant_dt(1, 1, 1, factor=0.5)
+    g = FDTD(Parameters(*shape), dt, Precision.FP64)
+    g.set_point_sources(many_sources(shape, dt, 200, 37))
+    ms = []
+    for L in (4, 0):
+        g.set_time_blocking_strips(L, 1, 2, 8)
+        g.update_fields(24)
+        ms.append(min(g.time_update_fields(24)[0] for _ in range(8)))
+    assert ms[0] < 1.1 * ms[1], ms
+    g.close()
