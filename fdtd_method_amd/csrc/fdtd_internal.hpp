@@ -57,6 +57,9 @@ struct BlockTuning {
     int R = 0;  // > 0: wavefront-strip kernel, R rows per lane, TYg / R wavefronts
     // strip passes of l steps straight from memory: lanes of a tile row
     int row_lanes[5] = {64, 64, 64, 64, 64};
+    // us that a pass saves over single sweeps, where a grid takes passes by
+    // default only for that (0: it takes them in any case)
+    float saves = 0;
 };
 
 inline size_t storage_size(int precision) {
@@ -161,7 +164,7 @@ struct fdtd_grid {
     hipEvent_t src_ev[2] = {};
     bool src_ev_used[2] = {false, false};
     int src_slot = 0;
-    int nsrc = 0;
+    int nsrc = 0, src_planes = 0;  // sources in d_src, z planes that hold one
     bool src_dirty = true;
     fdtd::rt::Tuning tune;
     fdtd::rt::BlockTuning btune;

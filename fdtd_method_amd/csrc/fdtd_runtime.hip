@@ -264,6 +264,8 @@ int flush_sources(fdtd_grid* g) {
         g->d_kstart = g->d_kst_buf[slot];
     }
     g->nsrc = (int)all.size();
+    g->src_planes = 0;
+    for (int k = 0; k < g->Nk; ++k) g->src_planes += kstart[k + 1] > kstart[k];
     g->src_dirty = false;
     return FDTD_OK;
 }
@@ -1180,15 +1182,24 @@ void plan_strips(const fdtd_grid* g, BlockTuning* t, int kchunk, long long* plan
         if (t->TYg > 2 * l) t->row_lanes[l] = strip_direct_lanes(g, *t, l, t->kchunk);
 }
 
-// Whether strip passes of t.L steps beat as many single sweeps on a grid, by
-// what both cost on grids that fit the caches: a plane-round of a pass about
+// us that a strip pass of t.L steps saves over as many single sweeps on a grid,
+// by what both cost on grids that fit the caches: a plane-round of a pass about
 // 3.3 us (FP64 W = 8, FP32 W = 16), a sweep 5 us up to 26 MB of E and B read
 // and written, beyond that 5 us and its bytes at 4.8 TB/s (FP32 128^3 26 us,
 // 160^3 48; FP64 131x90x70 26, 200x151x97 65).
-bool strips_pay(const fdtd_grid* g, const BlockTuning& t, long long planes) {
+double strips_save(const fdtd_grid* g, const BlockTuning& t, long long planes) {
     const double mb = 12.0 * g->N * g->esize * 1e-6;
     const double sweep = mb <= 26.0 ? 5.0 : 5.0 + mb / 4.8;
-    return 3.3 * planes < t.L * sweep;
+    return t.L * sweep - 3.3 * planes;
+}
+
+// Whether a run of a grid's default passes is faster with its sources.  m point
+// sources all over the grid add some 2.5 sqrt(m) us to a pass, whose tiles
+// march through them one by one (FP32 101x99x97: 80 of them 22 us, 200 34, 500
+// 58; FP64 72x70x74 18, 27, 49), and next to nothing to sweeps.  Sources in few
+// planes hold up sweeps just as much.
+bool passes_pay(const fdtd_grid* g) {
+    return g->btune.saves <= 0 || 2 * g->src_planes < g->Nk || 2.5 * std::sqrt((double)g->nsrc) < g->btune.saves;
 }
 
 template <typename S, int V, bool FINAL>
@@ -1426,8 +1437,10 @@ int run_fused(fdtd_grid* g, int nsteps, hipEvent_t mid = nullptr) {
     // (uploaded J) runs single sweeps, which read it.
     // Probes are recorded by strip passes, not by patch passes.
     if (g->btune.L >= 1 && nsteps >= g->btune.L && !g->pml && !g->j_dense_active &&
-        (g->btune.R > 0 || !probing(g)))
-        return run_blocked(g, nsteps, mid);
+        (g->btune.R > 0 || !probing(g))) {
+        if (int rc = flush_sources(g)) return rc;
+        if (passes_pay(g)) return run_blocked(g, nsteps, mid);
+    }
     // A carried half step replaces the B/2 prologue (bit-identical: the
     // final sweep of the previous run computed (B_n + d) + d from the same
     // E_n); otherwise B/2 in place.
@@ -1838,7 +1851,9 @@ int create_grid(const fdtd_parameters* p, double dt, double pml_percent, int pre
         if (strip_valid(g, t)) {
             long long planes = 0;
             plan_strips(g, &t, 0, &planes);
-            if (wide || strips_pay(g, t, planes)) g->btune = t;
+            const double saves = strips_save(g, t, planes);
+            if (!wide) t.saves = static_cast<float>(saves);
+            if (wide || saves > 0) g->btune = t;
         }
     }
     if (g->pml && g->fused_ok)

@@ -373,3 +373,34 @@ def test_many_sources_in_a_plane_cost_passes_no_more_than_sweeps():
         ms.append(min(g.time_update_fields(24)[0] for _ in range(8)))
     assert ms[0] < 1.1 * ms[1], ms
     g.close()
+
+
+@pytest.mark.parametrize("prec,shape,m,plane,passes", [
+    (Precision.FP32, (101, 99, 97), 500, None, 0),  # 386 us by sweeps, 572 by passes
+    (Precision.FP64, (72, 70, 74), 200, None, 0),   # 321, 371
+    (Precision.FP32, (101, 99, 97), 16, None, 3),   # 330, 282
+    (Precision.FP32, (101, 99, 97), 500, 50, 3),    # 2.52 ms, 1.93
+    (Precision.FP64, (101, 99, 97), 200, None, 3),  # 660 us, 570
+])
+def test_narrow_grids_with_sources_all_over(prec, shape, m, plane, passes):
+    """Grids that take passes by default only because these cost less take
+    sweeps where sources all over the grid hold the passes up; a blocking that
+    was asked for stays."""
+    dt = courant_dt(1, 1, 1, factor=0.5)
+    state = random_state(int(np.prod(shape)), 5)
+    a, b, c = (grid(shape, dt, state, prec, many_sources(shape, dt, m, plane)) for _ in range(3))
+    a.set_time_blocking_strips(0)
+    c.set_time_blocking_strips(4, 1, 2, 8 if prec == Precision.FP64 else 16)
+    for steps in (8, 1, 4):
+        for g in (a, b, c):
+            g.update_fields(steps)
+        assert a.checksum() == b.checksum() == c.checksum(), steps
+    assert b.launch_stats()["passes"] == passes
+    assert c.launch_stats()["passes"] == 3
+    for g in (b, c):  # without its sources a grid is back to passes
+        g.set_point_sources([])
+        g.update_fields(4)
+    assert b.launch_stats()["passes"] == passes + 1
+    assert b.checksum() == c.checksum()
+    for g in (a, b, c):
+        g.close()
