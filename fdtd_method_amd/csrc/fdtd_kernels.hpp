@@ -641,8 +641,9 @@ pml_plain_update_B(Fields<S> f, Pml<S, C> P, Coefs<C> c, int Ni, int Nj, int Nk)
 // The same first B update in front of the sweeps of a run, marching up zc
 // planes per thread: Ex and Ey of plane k+1 are read once, a layer cell's B,
 // the sum of its splits, is not read, and only written (`totals`) where a sweep
-// follows that reads it.  15 words a layer cell instead of 23 with both planes
-// of E fetched: 512^3 FP32 with a 0.2 layer 1.78 ms instead of 2.24.
+// follows that reads it.  15 words a layer cell, 18 with the totals, instead of
+// 20 (E of one plane read, the splits moved, the totals written): 512^3 FP32
+// with a 0.2 layer 1.78 ms instead of 2.24.
 template <typename S, typename C>
 __global__ void __launch_bounds__(256)
 pml_first_B(Fields<S> f, Pml<S, C> P, Coefs<C> c, int Ni, int Nj, int Nk, int zc, bool totals) {
@@ -2067,13 +2068,14 @@ blocked_sweep(BlockedArgs<S, C> a) {
 // before the barrier in front of level l.  One barrier per level and plane
 // (two for L = 1).
 //
-// What bounds it (512^3 FP32, L = 4, one MI355X, staged path): 1.53 ms per
-// pass = 5.3 TB/s of real traffic (4.8 GB read: the minimum times 1.49, since
+// What bounds it (512^3 FP32, L = 4, one MI355X, staged path): 1.50 ms per
+// pass = 5.4 TB/s of real traffic (4.8 GB read: the minimum times 1.49, since
 // neighbouring tiles drift apart by more planes than an L2 holds; 3.3 GB
-// written), with the VALU busy about three quarters of the time; the
-// arithmetic alone, without loads and stores, takes 1.1 ms.  Before planes
-// went through LDS: 1.83 ms.  FP64 (64 x 16 tiles, direct): 4.62 ms, now 3.38;
-// FP16 1.74 -> 1.62 ms.
+// written), where a single sweep reaches 5.7, with the VALU busy 63% of the
+// time; the arithmetic alone, without loads and stores, takes 1.1 ms.  Before
+// planes went through LDS: 1.83 ms.  FP64: 3.38 ms (4.62 before, 64 x 16 tiles)
+// at 5.1 TB/s, 10.95 GB read (the minimum times 1.70), the VALU busy 37%: neither
+// is full, waves wait.  FP16 1.74 -> 1.62 ms.
 
 // p advanced by a 32-bit unsigned byte offset (zero-extended): lets the
 // compiler address memory as a scalar base plus a 32-bit lane offset.
@@ -2279,7 +2281,7 @@ __device__ __forceinline__ bool tile_probes(const StripArgs<S, C>& a, int tile) 
 // FIRST (staged path, two planes in LDS): the pass that starts from (E_n,
 // B_n) and takes the run's first B half step, (B_n + d), on the planes it
 // reads, instead of a sweep over E and B in front of the pass (512^3 FP32:
-// 0.93 ms, 4.8 GB; it makes the pass 0.3 ms longer, FP64 0.9 where the sweep
+// 0.93 ms, 4.8 GB; it makes the pass 0.3 ms longer, FP64 1.0 where the sweep
 // took 1.8).  Plane kk then needs E of plane kk+1, which is staged,
 // and one E column and row past the tile's high edges, which the edge lanes
 // and the last row group read from memory themselves.

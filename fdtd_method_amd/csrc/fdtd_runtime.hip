@@ -274,7 +274,7 @@ int flush_sources(fdtd_grid* g) {
 // their launch (all of them, sorted by plane): single-cell J values and no
 // waveform, on a periodic grid without probes or FP16 rescaling.  The
 // reference drivers' one-step calls then upload nothing (32^3 FP64, 24
-// values set before each step: 28 us per step, now 12).
+// values set before each step: 28 us per step, now 8.8).
 bool inline_sources(const fdtd_grid* g, std::vector<fdtd::InlineSource>* out) {
     if (!g->waveforms.empty() || !g->jtab_keys.empty() || g->pml || g->nprobe > 0 ||
         g->autoscale_interval > 0 || g->sparse_j.size() > (size_t)fdtd::kInlineSources)
@@ -1287,8 +1287,8 @@ void trace_end(fdtd_grid* g, hipEvent_t a, int kind, bool pass) {
 }
 
 // Whether a pass takes the l (2 or 3) steps left over faster than single sweeps.
-// A pass takes about as long with fewer levels, FP64 and FP32 because memory
-// bounds it, FP16 because its planes' latency does; FP16 sweeps of whole 4-cell
+// A pass takes about as long with fewer levels, FP64 and FP32 because its planes
+// move the same bytes, FP16 because their latency stays; FP16 sweeps of whole 4-cell
 // lanes move so little that two of them cost less from the size of the last-level
 // cache on (us, sweeps / pass: two steps 128^3 37 / 31, 256^3 189 / 202, 320^3 334
 // / 415, 512^3 1270 / 2036; three steps 256^3 283 / 200, 512^3 1905 / 2102, 640^3

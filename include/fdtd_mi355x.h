@@ -338,7 +338,8 @@ int fdtd_zero_fields(fdtd_grid* grid);
  * fdtd_update_fields call also stores the next call's first B half step,
  * (B_n + d) + d, in two extra B buffer sets allocated on first use, so
  * consecutive calls -- the reference drivers' one-step loops -- run no B/2
- * prologue.  Results are bit-identical either way; host writes to E or B
+ * prologue; FP64 and FP32 runs of staged strip passes only do so where they
+ * found one.  Results are bit-identical either way; host writes to E or B
  * drop the carried step.  enable = 0 frees the buffers. */
 int fdtd_set_step_carry(fdtd_grid* grid, int enable);
 
@@ -359,7 +360,7 @@ int fdtd_autotune(fdtd_grid* grid, int reps, int out[3], float* best_ms);
  * sweep); L = 0 returns to the full-row fused sweep.  0 picks a default for
  * V, lanes, TYg, kchunk.  Results are bit-identical to unblocked steps
  * (FP16 with in-run rescaling: to FP16 rounding, as it rescales between passes).
- * get: {L, V, lanes, TYg, kchunk}.  fdtd_autotune_blocking times the
+ * get: {L, V, lanes, TYg, kchunk} (of strip passes, lanes of a tile row).  fdtd_autotune_blocking times the
  * full-row sweep and tiled/blocked candidates on scratch copies of the
  * state and keeps the fastest per step (best_ms: ms per step). */
 int fdtd_set_time_blocking(fdtd_grid* grid, int L, int V, int lanes, int TYg, int kchunk);
